@@ -146,7 +146,8 @@ enum {
 
 /* Kernel stages reported by ne_get_stage_times. */
 enum {
-  NE_STAGE_MEGAKERNEL = 0, /* one thread per (pixel, sample chunk), whole paths */
+  NE_STAGE_MEGAKERNEL = 0, /* whole paths in one launch: one thread per (pixel, sample chunk), or (mode AUTO,
+                              FP32, volume-only scenes) the persistent volume path kernel */
   NE_STAGE_PLAN = 1,       /* wavefront: hand out new path ids per chunk (until every path is issued) */
   NE_STAGE_REGEN = 2,      /* wavefront: camera rays into free slots (volume-only scenes: inside MEDIUM) */
   NE_STAGE_TRACE = 3,      /* wavefront: BVH closest hit */
@@ -176,8 +177,10 @@ typedef struct ne_render_params {
   int32_t samples_per_thread; /* 0 = library default */
   int32_t block_size;         /* 0 = library default */
   int32_t occupancy;          /* megakernel FP32 variant built for >= this many waves per SIMD: 0, 4, 6 */
-  int32_t mode;               /* NE_MODE_*: 0 = auto (wavefront for FP32, megakernel for FP64) */
-  int32_t pool_size;          /* wavefront path slots (rounded up to 256); 0 = library default
+  int32_t mode;               /* NE_MODE_*: 0 = auto (FP32: the persistent volume path kernel on scenes
+                                 without surfaces, where no flag or pool_size asks for the staged
+                                 wavefront, else the staged wavefront; FP64: megakernel) */
+  int32_t pool_size;          /* staged wavefront path slots (rounded up to 256); 0 = library default
                                  (2^23 for surface-only scenes and for renders of 2^28 paths
                                  or more, else 2^22) */
 } ne_render_params;

@@ -48,6 +48,8 @@ struct ne_ctx {
   uint32_t wfg_P = 0;
   void* sbuf = nullptr;         // wavefront per-sample radiance (grown on demand)
   size_t sbuf_bytes = 0;
+  int cus = 0;                  // compute units of the device
+  void* paths_scratch = nullptr;  // the persistent path kernel's (made on its first use)
   double* scratch = nullptr;    // this device's copy of the static scratch array (ne_render_noalloc)
 };
 
@@ -452,6 +454,7 @@ ne_status ne_ctx_create(int32_t device, ne_ctx** out) {
   c->device = device;
   if (hipSetDevice(device) != hipSuccess || hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
       hipMalloc(&c->d_counters, sizeof(DevCounters)) != hipSuccess ||
+      hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess ||
       hipHostMalloc((void**)&c->h_status, 64 * sizeof(uint32_t), hipHostMallocDefault) != hipSuccess ||
       hipEventCreate(&c->ev0) != hipSuccess ||
       hipEventCreate(&c->ev1) != hipSuccess) {
@@ -471,6 +474,7 @@ static void ctx_free(ne_ctx* c) {
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   if (c->d_partial) (void)hipFree(c->d_partial);
   if (c->d_counters) (void)hipFree(c->d_counters);
+  if (c->paths_scratch) (void)hipFree(c->paths_scratch);
   if (c->wf_buf) (void)hipFree(c->wf_buf);
   if (c->h_status) (void)hipHostFree(c->h_status);
   for (hipEvent_t e : c->ev_pool) (void)hipEventDestroy(e);
@@ -639,6 +643,7 @@ ne_status ne_scene_upload(ne_ctx* c, const ne_scene_desc* d, ne_scene** out) {
     ds.sigma_bar = (st3[0] * d->vol_mult + st3[1] * d->vol_mult + st3[2] * d->vol_mult) / 3.0f;
     ds.g = d->vol_g;
     ds.mres = homog ? 1 : d->maj_res;
+    ds.inv_mres = 1.0f / float(ds.mres);
     {
       // row-major upload into a scratch buffer, bricked copy kept (zero padded,
       // plus one brick of slack after the last)
@@ -687,6 +692,12 @@ ne_status ne_scene_upload(ne_ctx* c, const ne_scene_desc* d, ne_scene** out) {
                 ds.occ_hi[a] = std::max(ds.occ_hi[a], cxyz[a]);
               }
             }
+    }
+    // its faces, in the DDA's arithmetic (each operation rounded on its own)
+    for (int a = 0; a < 3; ++a) {
+      const float lo = float(ds.occ_lo[a]) * ds.inv_mres, hi = float(ds.occ_hi[a] + 1) * ds.inv_mres;
+      ds.occ_face[a] = lo - 0.5f;
+      ds.occ_face[3 + a] = hi - 0.5f;
     }
     if (!d->maj_no_skip && std::any_of(mh.begin(), mh.end(), [](float v) { return !(v > 0.0f); })) {
       encode_empty_distance(mh, ds.mres);
@@ -841,6 +852,23 @@ static uint64_t default_pool(const DevScene& ds, uint64_t total) {
   return total >= (uint64_t(1) << 28) ? (uint64_t(1) << 23) : (uint64_t(1) << 22);
 }
 
+// Scenes that the persistent path kernel takes (paths.hip): a volume, and
+// lights without geometry; a guide only frozen and tabulated.
+static bool persistent_scene(const DevScene& ds, bool guided, bool tabulated) {
+  return ds.has_volume && ds.n_nodes == 0 && (!guided || tabulated);
+}
+// Renders that take it: mode AUTO on such a scene.  Counting runs, the orders
+// of the staged kernels (sort, spatial), an explicit pool, the plan's test
+// hook, training and per-vertex network evaluation need the staged pipeline,
+// as does an explicit NE_MODE_WAVEFRONT; both trace the same paths with the
+// same arithmetic, and the persistent kernel was faster at every size measured
+// (from 4,000 to 530 million paths).
+static bool persistent_paths(const DevScene& ds, const ne_render_params* p, const WfGuideHook* gh) {
+  const int staged = NE_FLAG_COUNT | NE_FLAG_SORT | NE_FLAG_SPATIAL | NE_FLAG_TEST_PLAN_STALL;
+  return p->mode == NE_MODE_AUTO && p->pool_size == 0 && !(p->flags & staged) && !(gh && gh->g.train) &&
+         persistent_scene(ds, gh != nullptr, gh && gh->g.cache.mix);
+}
+
 static ne_status render_wavefront(ne_ctx* c, const ne_scene* s, const DevCamera& dc, const ne_render_params* p,
                                   ne_film* f, bool count, bool timed, StageTimer* tm, WfGuideHook* gh = nullptr) {
   const uint64_t total = uint64_t(p->x1 - p->x0) * uint64_t(p->y1 - p->y0) * uint64_t(p->spp);
@@ -848,7 +876,8 @@ static ne_status render_wavefront(ne_ctx* c, const ne_scene* s, const DevCamera&
   uint64_t P = p->pool_size > 0 ? uint64_t(p->pool_size) : default_pool(s->dev, total);
   P = std::min<uint64_t>(P, total);
   P = (P + kChunk - 1) / kChunk * kChunk;
-  if (P > c->wf_P) {
+  const bool persistent = persistent_paths(s->dev, p, gh);
+  if (!persistent && P > c->wf_P) {
     if (c->wf_buf) {
       NE_HIP(c, hipStreamSynchronize(c->stream));
       void* old = c->wf_buf;  // cleared first: a failing free never leaves it to be freed twice
@@ -866,8 +895,6 @@ static ne_status render_wavefront(ne_ctx* c, const ne_scene* s, const DevCamera&
     NE_HIP(c, hipMalloc(&f->d_fixed, bytes));
     NE_HIP(c, hipMemsetAsync(f->d_fixed, 0, bytes, c->stream));
   }
-  WfState w{};
-  wf_carve(c->wf_buf, uint32_t(P), w);
   WfArgs a{};
   a.W = p->width; a.H = p->height; a.x0 = p->x0; a.y0 = p->y0; a.x1 = p->x1; a.y1 = p->y1;
   a.max_bounces = p->max_bounces; a.sample_offset = p->sample_offset; a.job = p->job; a.nchunks = uint32_t(P / kChunk);
@@ -911,6 +938,24 @@ static ne_status render_wavefront(ne_ctx* c, const ne_scene* s, const DevCamera&
     a.sbuf = sbytes <= c->sbuf_bytes ? static_cast<float*>(c->sbuf) : nullptr;
   }
   a.gstate[0] = a.gstate[1] = nullptr;
+  if (persistent) {
+    GuideUse gu{};
+    if (gh) {
+      gu.cache = gh->g.cache;
+      gu.max_depth = gh->g.max_depth;
+      gu.prob = gh->g.prob;
+    }
+    if (!c->paths_scratch) NE_HIP(c, hipMalloc(&c->paths_scratch, paths_scratch_bytes(c->cus)));
+    if (timed) NE_HIP(c, hipEventRecord(c->ev0, c->stream));
+    NE_HIP(c, launch_paths(s->dev, dc, a, gu, c->paths_scratch, c->cus, c->stream, tm));
+    if (timed) {
+      NE_HIP(c, hipEventRecord(c->ev1, c->stream));
+      c->timed = true;
+    }
+    return NE_OK;
+  }
+  WfState w{};
+  wf_carve(c->wf_buf, uint32_t(P), w);
   if (gh) {
     if (P > c->wfg_P) {
       if (c->wfg_buf) {
@@ -1341,6 +1386,7 @@ ne_status ne_test_rng(ne_ctx* c, uint64_t seed, uint32_t pixel, uint32_t sample,
 // A stream of the wavefront executor, with its own path pool and status word.
 struct BatchLane {
   hipStream_t stream = nullptr;
+  void* paths_scratch = nullptr;  // the persistent path kernel's
   void* pool = nullptr;
   uint32_t pool_P = 0;
   void* sbuf = nullptr;  // per-sample radiance slots (12 B per sample of the lane's largest job)
@@ -1386,6 +1432,7 @@ void batch_free(ne_batch* b) {
   for (BatchLane& L : b->lanes) {
     if (L.stream) (void)hipStreamDestroy(L.stream);
     if (L.pool) (void)hipFree(L.pool);
+    if (L.paths_scratch) (void)hipFree(L.paths_scratch);
     if (L.sbuf) (void)hipFree(L.sbuf);
     if (L.status) (void)hipHostFree(L.status);
   }
@@ -1509,6 +1556,11 @@ static uint64_t lane_job_pool(const ne_job& J, int div, uint64_t* samples) {
   return (P + kChunk - 1) / kChunk * kChunk;
 }
 
+// Whether the persistent path kernel renders job J (no path pool then).
+static bool lane_job_persistent(const ne_job& J) {
+  return persistent_scene(J.scene->dev, J.guide != nullptr, J.guide && J.guide->cache.mix);
+}
+
 // One job through the wavefront pipeline on a lane (called from the lane's
 // own host thread): the FP32 ne_render path at ceil(spp / div) samples into
 // the job's fixed-point batch film, a guided job with its frozen tabulated
@@ -1521,10 +1573,9 @@ hipError_t lane_render(ne_batch* b, BatchLane& L, size_t j, int div, uint32_t re
   const DevScene& ds = J.scene->dev;
   uint64_t total = 0;
   const uint64_t P = lane_job_pool(J, div, &total);
-  if (P > L.pool_P) return hipErrorInvalidValue;
+  const bool persistent = lane_job_persistent(J);
+  if (!persistent && P > L.pool_P) return hipErrorInvalidValue;
   hipError_t e;
-  WfState w{};
-  wf_carve(L.pool, uint32_t(P), w);
   WfArgs a{};
   a.W = J.width; a.H = J.height; a.x0 = 0; a.y0 = 0; a.x1 = J.width; a.y1 = J.height;
   a.max_bounces = J.max_bounces; a.sample_offset = 0; a.job = J.job; a.nchunks = uint32_t(P / kChunk);
@@ -1543,6 +1594,15 @@ hipError_t lane_render(ne_batch* b, BatchLane& L, size_t j, int div, uint32_t re
     a.sbuf = static_cast<float*>(L.sbuf);
   }
   a.gstate[0] = a.gstate[1] = nullptr;
+  if (persistent) {
+    if (!L.paths_scratch) return hipErrorInvalidValue;
+    if ((e = launch_paths(ds, make_camera(&J.camera), a, J.guide ? guide_use(J.guide) : GuideUse{}, L.paths_scratch,
+                          b->ctx->cus, L.stream, nullptr)) != hipSuccess)
+      return e;
+    return hipStreamSynchronize(L.stream);
+  }
+  WfState w{};
+  wf_carve(L.pool, uint32_t(P), w);
   WfGuideHook hook{};
   WfGuideHook* gh = nullptr;
   if (J.guide) {  // frozen: no training records, no steps
@@ -1587,14 +1647,18 @@ ne_status batch_run_lanes(ne_batch* b, int div, float* ms) {
   // before the timed run (slots for the jobs that use them, lane_render)
   uint64_t Pmax = 0;
   size_t sbytes = 0;
+  bool paths = false;
   for (const ne_job& J : b->jobs) {
     uint64_t t = 0;
-    Pmax = std::max(Pmax, lane_job_pool(J, div, &t));
+    const uint64_t P = lane_job_pool(J, div, &t);
+    if (lane_job_persistent(J)) paths = true;
+    else Pmax = std::max(Pmax, P);
     const size_t jb = size_t(t) * 3 * sizeof(float);
     if (jb <= kMaxSampleBuffer) sbytes = std::max(sbytes, jb);
   }
   for (int i = 0; i < nl; ++i) {
     BatchLane& L = b->lanes[i];
+    if (paths && !L.paths_scratch) NE_HIP(c, hipMalloc(&L.paths_scratch, paths_scratch_bytes(c->cus)));
     if (Pmax > L.pool_P) {
       void* old = L.pool;
       L.pool = nullptr;

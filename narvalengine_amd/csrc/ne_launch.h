@@ -157,6 +157,18 @@ struct WfGuideHook;  // guided mode: proposal, training records, online training
 // it).  h_status: pinned host words.
 hipError_t launch_wavefront(const DevScene& s, const DevCamera& cam, WfState& w, WfArgs a, bool count,
                             hipStream_t st, uint32_t* h_status, StageTimer* tm, WfGuideHook* gh);
+// Sums the per-sample slots and the fixed-point film into a.film (or, without
+// a.film, the slots into the fixed-point film) after a render's last stage.
+hipError_t wf_flush(const WfArgs& a, hipStream_t st);
+// ---- persistent volume path kernel -----------------------------------------
+// A volume lit by the sun, the environment and point lights (no BVH): whole
+// paths in one launch (paths.hip), with the staged pipeline's draws and
+// arithmetic.  scratch: paths_scratch_bytes of device memory of this stream's
+// own.  gu.cache.mix != nullptr: medium vertices sample the guide's tabulated
+// proposal.
+size_t paths_scratch_bytes(int cus);
+hipError_t launch_paths(const DevScene& s, const DevCamera& cam, const WfArgs& a, const GuideUse& gu, void* scratch,
+                        int cus, hipStream_t st, StageTimer* tm);
 // ---- persistent batched renderer -------------------------------------------
 constexpr int kMaxBatchJobs = 1024;
 struct BatchJob {

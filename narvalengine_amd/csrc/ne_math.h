@@ -104,6 +104,14 @@ template <typename R> NE_HD R power_heuristic(R a, R b) { return (a * a) / (a * 
 
 // ---- Philox-4x32-10 (Salmon et al., SC'11) ---------------------------------
 
+// a ^ b ^ c: one v_bitop3_b32 on gfx950 (the compiler keeps two v_xor_b32)
+NE_HD uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) {
+#ifdef __HIP_DEVICE_COMPILE__
+  return __builtin_amdgcn_bitop3_b32(a, b, c, 0x96);
+#else
+  return a ^ b ^ c;
+#endif
+}
 NE_HD void philox10(uint32_t c[4], uint32_t k0, uint32_t k1) {
 #pragma unroll
   for (int r = 0; r < 10; ++r) {
@@ -113,7 +121,7 @@ NE_HD void philox10(uint32_t c[4], uint32_t k0, uint32_t k1) {
     const uint64_t p0 = uint64_t(0xD2511F53u) * c[0], p1 = uint64_t(0xCD9E8D57u) * c[2];
     const uint32_t hi0 = uint32_t(p0 >> 32), lo0 = uint32_t(p0);
     const uint32_t hi1 = uint32_t(p1 >> 32), lo1 = uint32_t(p1);
-    uint32_t n0 = hi1 ^ c[1] ^ k0, n2 = hi0 ^ c[3] ^ k1;
+    uint32_t n0 = xor3(hi1, c[1], k0), n2 = xor3(hi0, c[3], k1);
     c[0] = n0; c[1] = lo1; c[2] = n2; c[3] = lo0;
   }
 }
@@ -192,6 +200,31 @@ struct PathRng {
       shift();
     }
     return float(r >> 8) * (1.0f / 16777216.0f);
+  }
+  // Resume after n draws with the current block's undrawn words at hand.
+  NE_HD void restore(uint32_t n, uint32_t w0, uint32_t w1, uint32_t w2, uint32_t block0 = 0) {
+    block = block0 + ((n + 3u) >> 2);
+    idx = (n & 3u) ? int(n & 3u) : 4;
+    b0 = w0; b1 = w1; b2 = w2; b3 = 0;
+  }
+  // The five uniforms of the stream after n draws; the stream then stands
+  // after them.  They lie in two blocks whatever n is, so both are generated
+  // at once: next() five times has a refill site per draw, each of which a
+  // wave runs whenever one of its lanes stands at a block's end.
+  NE_HD void five(uint32_t n, float u[5]) {
+    uint32_t a[4] = {pixel, sample, n >> 2, job}, c[4] = {pixel, sample, (n >> 2) + 1u, job};
+    philox10(a, k0, k1);
+    philox10(c, k0, k1);
+    const bool h = (n & 2u) != 0u, o = (n & 1u) != 0u;  // words n & 3 .. (n & 3) + 4 of the eight
+    const uint32_t w0 = h ? a[2] : a[0], w1 = h ? a[3] : a[1], w2 = h ? c[0] : a[2], w3 = h ? c[1] : a[3],
+                   w4 = h ? c[2] : c[0], w5 = h ? c[3] : c[1];
+    u[0] = float((o ? w1 : w0) >> 8) * (1.0f / 16777216.0f);
+    u[1] = float((o ? w2 : w1) >> 8) * (1.0f / 16777216.0f);
+    u[2] = float((o ? w3 : w2) >> 8) * (1.0f / 16777216.0f);
+    u[3] = float((o ? w4 : w3) >> 8) * (1.0f / 16777216.0f);
+    u[4] = float((o ? w5 : w4) >> 8) * (1.0f / 16777216.0f);
+    // the second block's words from (n + 5) & 3 on (none if that is 0)
+    restore(n + 5u, h ? c[3] : (o ? c[2] : c[1]), o ? c[3] : c[2], c[3]);
   }
   // The next buffered word; only directly after next_keep1().
   NE_HD float next_buffered() {

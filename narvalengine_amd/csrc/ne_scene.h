@@ -78,8 +78,10 @@ struct DevScene {
   int32_t homog;          // homogeneous medium: density 1 everywhere in the cube
   int32_t res[3];
   int32_t mres;
+  float inv_mres;         // 1 / mres (IEEE division, as on the device)
   int32_t occ_lo[3], occ_hi[3];  // majorant cells with a positive majorant lie in [occ_lo, occ_hi]
                                  // (occ_lo > occ_hi: none)
+  float occ_face[6];  // that box's faces in the volume's cube: lo x, y, z, hi x, y, z
   float inv[12];          // WCS -> OCS, rows of a 3x4 matrix
   const float* grid;      // bricked (grid_offset), zero-padded to at least res + 2 voxels per axis
   uint32_t grid_step_y;   // floats from one brick row (4 voxels in y) to the next

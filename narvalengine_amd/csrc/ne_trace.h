@@ -711,6 +711,126 @@ NE_DEV R ratio_track(const DevScene& s, Vec3<R> o, Vec3<R> d, R ta, R tb, PathRn
   return Tr;
 }
 
+// The majorant walk of majorant_dda as a resumable object, for kernels that
+// regroup rays between steps: leave() steps out of the current cell, look()
+// enters it.  The same cells, boundaries and tracking intervals: cell
+// boundaries depend on the cell index alone, so a walk restored from its cell
+// (resume) continues with the same bits.
+struct Walk {
+  Vec3<float> oo, dd, inv, tn;  // OCS ray, reciprocal direction (0 where the direction is 0), cell exits
+  int cx, cy, cz;
+  float t, tb;     // position (while in a cell: of the last tentative collision), end of the walk
+  float c1, imu;   // the current cell's exit and reciprocal majorant, while in it
+  int skip;        // empty cells ahead whose majorants need no read
+
+  NE_DEV static float exit_t(float d, int c, float o, float inv, float invM) {
+    const float bnd = float(d > 0.0f ? c + 1 : c) * invM;
+    return d != 0.0f ? ((bnd - 0.5f) - o) * inv : xinf<float>();
+  }
+  NE_DEV void exits(const DevScene& s) {
+    tn = v3(exit_t(dd.x, cx, oo.x, inv.x, s.inv_mres), exit_t(dd.y, cy, oo.y, inv.y, s.inv_mres),
+            exit_t(dd.z, cz, oo.z, inv.z, s.inv_mres));
+  }
+  NE_DEV void ray(const DevScene& s, Vec3<float> o, Vec3<float> d) {
+    oo = xf_point<float>(s.inv, o);
+    dd = xf_vec<float>(s.inv, d);
+    inv = v3(dd.x != 0.0f ? 1.0f / dd.x : 0.0f, dd.y != 0.0f ? 1.0f / dd.y : 0.0f, dd.z != 0.0f ? 1.0f / dd.z : 0.0f);
+  }
+  // box_interval of the ray with the reciprocals above (an infinite one, of
+  // either sign, bounds an axis the same way)
+  NE_DEV bool box(float& ta, float& te) const {
+    float t0 = -xinf<float>(), t1 = xinf<float>();
+    auto axis = [&](float o, float d, float i) {
+      const float id = d != 0.0f ? i : xinf<float>();
+      float tn_ = (-0.5f - o) * id, tf = (0.5f - o) * id;
+      if (tn_ > tf) { const float x = tn_; tn_ = tf; tf = x; }
+      t0 = tn_ > t0 ? tn_ : t0;
+      t1 = tf < t1 ? tf : t1;
+    };
+    axis(oo.x, dd.x, inv.x);
+    axis(oo.y, dd.y, inv.y);
+    axis(oo.z, dd.z, inv.z);
+    ta = t0;
+    te = t1;
+    return t0 <= t1;
+  }
+  // Walk of [ta, te), clipped to the box of the cells with a positive
+  // majorant; false if nothing is left of it.  Stands before its first cell.
+  NE_DEV bool start(const DevScene& s, float ta, float te) {
+    const float Mr = float(s.mres);
+    auto clip = [&](float da, float oa, float ia, float blo, float bhi) {
+      const float t0 = (blo - oa) * ia, t1 = (bhi - oa) * ia;
+      const bool par = da == 0.0f, out = !(oa >= blo && oa <= bhi);
+      ta = par ? ta : xmax(ta, xmin(t0, t1));
+      te = par ? (out ? ta : te) : xmin(te, xmax(t0, t1));
+    };
+    clip(dd.x, oo.x, inv.x, s.occ_face[0], s.occ_face[3]);
+    clip(dd.y, oo.y, inv.y, s.occ_face[1], s.occ_face[4]);
+    clip(dd.z, oo.z, inv.z, s.occ_face[2], s.occ_face[5]);
+    if (s.occ_lo[0] > s.occ_hi[0]) te = ta;  // no cell has a positive majorant
+    tb = te;
+    const Vec3<float> pe = oo + ta * dd;
+    auto cell = [&](float p) {
+      const int c = int(floorf((p + 0.5f) * Mr));
+      return c < 0 ? 0 : (c > s.mres - 1 ? s.mres - 1 : c);
+    };
+    cx = cell(pe.x); cy = cell(pe.y); cz = cell(pe.z);
+    exits(s);
+    t = ta;
+    skip = 0;
+    return ta < te;
+  }
+  NE_DEV uint32_t packed() const {  // 24 bits: maj_res <= 256
+    return uint32_t(cx) | (uint32_t(cy) << 8) | (uint32_t(cz) << 16);
+  }
+  NE_DEV void resume(const DevScene& s, float t_, float tb_, uint32_t cell) {
+    cx = int(cell & 255u); cy = int((cell >> 8) & 255u); cz = int((cell >> 16) & 255u);
+    exits(s);
+    t = t_;
+    tb = tb_;
+    skip = 0;  // a run of empty cells is read again: the majorant there says how many are left
+  }
+  // Out of the current cell; true at the end of the walk.
+  NE_DEV bool leave(const DevScene& s) {
+    // (selects over values: over members they would become an indexed access)
+    const Vec3<float> o = oo, d = dd, i = inv, n = tn;
+    const int x = cx, y = cy, z = cz;
+    // exit axis: ties keep the lower axis
+    const bool s1 = n.y < n.x;
+    const float t01 = s1 ? n.y : n.x;
+    const bool s2 = n.z < t01;
+    const float tna = s2 ? n.z : t01;
+    const float da = s2 ? d.z : (s1 ? d.y : d.x);
+    const int c = (s2 ? z : (s1 ? y : x)) + (da > 0.0f ? 1 : -1);
+    const bool over = tna >= tb || uint32_t(c) >= uint32_t(s.mres);
+    t = tna;
+    const float bnd = float(da > 0.0f ? c + 1 : c) * s.inv_mres;
+    const float oa = s2 ? o.z : (s1 ? o.y : o.x);
+    const float nt = ((bnd - 0.5f) - oa) * (s2 ? i.z : (s1 ? i.y : i.x));
+    const bool a1 = s1 && !s2, a0 = !s1 && !s2;
+    cx = a0 ? c : x;
+    cy = a1 ? c : y;
+    cz = s2 ? c : z;
+    tn = v3(a0 ? nt : n.x, a1 ? nt : n.y, s2 ? nt : n.z);
+    return over;
+  }
+  // Into the cell; true if it has a majorant (c1, imu) and an interval.
+  NE_DEV bool look(const DevScene& s) {
+    if (skip > 0) {
+      --skip;
+      return false;
+    }
+    const uint32_t M = uint32_t(s.mres);
+    const uint32_t ci = uint32_t(cx) + __umul24(uint32_t(cy), M) + __umul24(uint32_t(cz), M * M);
+    const float2 mp = *reinterpret_cast<const float2*>(reinterpret_cast<const char*>(s.maj_pair) + size_t(ci * 8u));
+    const float tc = xmin(xmin(tn.x, xmin(tn.y, tn.z)), tb);
+    skip = mp.x < 0.0f ? int(-mp.x) - 1 : 0;
+    c1 = tc;
+    imu = mp.y;
+    return mp.y > 0.0f && tc > t;  // the reciprocal is 0 unless the majorant is positive and finite
+  }
+};
+
 // ---------------------------------------------------------------------------
 // Phase function and surface BSDF
 // ---------------------------------------------------------------------------
@@ -970,19 +1090,23 @@ NE_DEV R sphere_cone_width(R dc2, R r2) {  // 1 - cos theta_max, cancellation-fr
   return sin2 / (R(1) + xsqrt(xmax(R(0), R(1) - sin2)));
 }
 template <typename R>
+NE_DEV void sample_point(const DevScene& s, uint32_t slot, Vec3<R> x, Vec3<R>& wi, R& dist, R& pl, Vec3<R>& Le) {
+  const float4 pt = s.points[slot];
+  const Vec3<R> dv = v3f4<R>(pt) - x;
+  const R d2 = dot(dv, dv);
+  dist = xsqrt(d2);
+  wi = dv / dist;
+  pl = d2 > R(0) ? R(1) : R(0);
+  Le = v3f<R>(s.mats + 12 * size_t(__float_as_int(pt.w)) + 6) / d2;
+}
+template <typename R>
 NE_DEV bool sample_emitter(const DevScene& s, uint32_t code, Vec3<R> x, R ua, R ub, Vec3<R>& wi, R& dist, R& pl,
                            Vec3<R>& Le) {
   const int type = int(code >> 30);
   const uint32_t slot = code & 0x3FFFFFFFu;
   int mat;
   if (type == kLightPoint) {
-    const float4 pt = s.points[slot];
-    const Vec3<R> dv = v3f4<R>(pt) - x;
-    const R d2 = dot(dv, dv);
-    dist = xsqrt(d2);
-    wi = dv / dist;
-    pl = d2 > R(0) ? R(1) : R(0);
-    Le = v3f<R>(s.mats + 12 * size_t(__float_as_int(pt.w)) + 6) / d2;
+    sample_point<R>(s, slot, x, wi, dist, pl, Le);
     return true;
   }
   if (type == PRIM_RECT) {
