@@ -664,7 +664,24 @@ ne_status ne_scene_upload(ne_ctx* c, const ne_scene_desc* d, ne_scene** out) {
       ds.grid = static_cast<const float*>(pg);
       ds.grid_step_y = (px / 4u) * kBrickFloats;
       ds.grid_step_z = (px / 4u) * (py / 4u) * kBrickFloats;
-      ds.grid_small = nb < (size_t(1) << 32) && ds.grid_step_z < (1u << 24) ? 1 : 0;
+      ds.grid_form = nb < (size_t(1) << 32) && ds.grid_step_z < (1u << 24) ? kGridBrick : kGridWide;
+      // the quads: four times the memory; without room for them the bricks serve
+      const uint32_t qx = quad_pad(ds.res[0]), qy = quad_pad(ds.res[1]), qz = quad_pad_z(ds.res[2]);
+      const uint64_t qstep = uint64_t(qx / 2u) * (qy / 2u) * 8u, qbytes = qstep * (qz / 2u) * sizeof(float4);
+      void* pq = nullptr;
+      if (ds.grid_form == kGridBrick && qbytes < (uint64_t(1) << 32) && qstep < (1u << 24)) {
+        if (hipMalloc(&pq, qbytes) == hipSuccess) {
+          s->allocs.push_back(pq);
+          s->bytes += qbytes;
+          NE_HIP_BAIL(launch_quad_grid(ds, static_cast<float4*>(pq), c->stream));
+          ds.quad = static_cast<const float4*>(pq);
+          ds.quad_step_y = (qx / 2u) * 8u;
+          ds.quad_step_z = uint32_t(qstep);
+          ds.grid_form = kGridQuad;
+        } else {
+          (void)hipGetLastError();
+        }
+      }
     }
     size_t ncell = size_t(ds.mres) * ds.mres * ds.mres;
     void* pm = nullptr;

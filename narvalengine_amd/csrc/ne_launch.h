@@ -328,6 +328,8 @@ hipError_t launch_li(const DevScene& s, int n, const float* rays, int max_bounce
                      float* out, hipStream_t st);
 // row-major density -> bricked layout (grid_offset), zero padding
 hipError_t launch_brick_grid(const float* lin, float* out, const int res[3], hipStream_t st);
+// the bricked grid s.grid -> quad layout (quad_pad sizes)
+hipError_t launch_quad_grid(const DevScene& s, float4* out, hipStream_t st);
 hipError_t launch_majorants(const DevScene& s, float* maj, hipStream_t st);
 
 }  // namespace ne

@@ -477,34 +477,49 @@ NE_DEV float grid_at(const DevScene& s, int x, int y, int z) {
 // corners at index >= res read as 0 (the grid's zero padding).
 // A homogeneous medium (HomogeneousMedia, src/materials/HomogeneousMedia.cpp)
 // reads density 1 everywhere; the multiplier carries its density.
-// SMALL (grid_small scenes): corner addresses are 32-bit byte offsets from
-// the grid base (uniform), so each load takes a scalar base and a 32-bit lane
-// offset and no lane does 64-bit address arithmetic; same corners, same value.
-template <bool SMALL = false>
+// GRID: the scene's grid_form or a wider one.  kGridBrick and kGridQuad
+// address the corners by 32-bit byte offsets from a uniform base, so each load
+// takes a scalar base and a 32-bit lane offset and no lane does 64-bit address
+// arithmetic; kGridQuad reads them by two 16-byte loads.  Same corners, same
+// value.
+template <int GRID = kGridWide>
 NE_DEV float density_gcs(const DevScene& s, Vec3<float> gp) {
   if (s.homog) return 1.0f;
   // clamp to [0, res] (std::max with 0, then std::min with res): for finite
   // values the median of (x, 0, res) is that clamp, one v_med3_f32
   gp = v3(__builtin_amdgcn_fmed3f(gp.x, 0.0f, float(s.res[0])), __builtin_amdgcn_fmed3f(gp.y, 0.0f, float(s.res[1])),
           __builtin_amdgcn_fmed3f(gp.z, 0.0f, float(s.res[2])));
-  if constexpr (SMALL) {
+  if constexpr (GRID != kGridWide) {
     // x >= 0 here: the truncating conversion is floor(x), and v_fract_f32
     // returns x - floor(x), which is exact (the low bits of x): the same
     // index and fraction as int(floorf(x)) and x - float(ix) below
     const uint32_t ix = uint32_t(gp.x), iy = uint32_t(gp.y), iz = uint32_t(gp.z);
     const float dx = __builtin_amdgcn_fractf(gp.x), dy = __builtin_amdgcn_fractf(gp.y),
                 dz = __builtin_amdgcn_fractf(gp.z);
-    // both steps are under 2^24 and every offset under 2^32: 24-bit multiplies are exact
-    const uint32_t b = (__umul24(iz >> 1, uint32_t(s.grid_step_z)) + __umul24(iy >> 2, uint32_t(s.grid_step_y)) +
-                        (ix >> 2) * kBrickFloats +
-                        (((iz & 1u) << 4) | ((iy & 3u) << 2) | (ix & 3u))) * 4u;
-    const uint32_t bx = (ix & 3u) != 3u ? 4u : (kBrickFloats - 3u) * 4u;  // x + 1: same brick or the next
-    const uint32_t by = (iy & 3u) != 3u ? 16u : (s.grid_step_y - 12u) * 4u;
-    const uint32_t bz = (iz & 1u) == 0u ? 64u : (s.grid_step_z - 16u) * 4u;
-    const char* g = reinterpret_cast<const char*>(s.grid);
-    auto at = [&](uint32_t o) { return *reinterpret_cast<const float*>(g + size_t(o)); };
-    const float c000 = at(b), c100 = at(b + bx), c010 = at(b + by), c110 = at(b + by + bx);
-    const float c001 = at(b + bz), c101 = at(b + bz + bx), c011 = at(b + by + bz), c111 = at(b + by + bz + bx);
+    float c000, c100, c010, c110, c001, c101, c011, c111;
+    if constexpr (GRID == kGridQuad) {
+      // steps under 2^24 and offsets under 2^32: 24-bit multiplies are exact
+      const uint32_t b = (__umul24(iz >> 1, s.quad_step_z) + __umul24(iy >> 1, s.quad_step_y) + (ix >> 1) * 8u +
+                          (((iz & 1u) << 2) | ((iy & 1u) << 1) | (ix & 1u))) * 16u;
+      const uint32_t bz = (iz & 1u) == 0u ? 64u : (s.quad_step_z - 4u) * 16u;
+      const char* g = reinterpret_cast<const char*>(s.quad);
+      const float4 q0 = *reinterpret_cast<const float4*>(g + size_t(b));
+      const float4 q1 = *reinterpret_cast<const float4*>(g + size_t(b + bz));
+      c000 = q0.x; c100 = q0.y; c010 = q0.z; c110 = q0.w;
+      c001 = q1.x; c101 = q1.y; c011 = q1.z; c111 = q1.w;
+    } else {
+      // both steps are under 2^24 and every offset under 2^32: 24-bit multiplies are exact
+      const uint32_t b = (__umul24(iz >> 1, uint32_t(s.grid_step_z)) + __umul24(iy >> 2, uint32_t(s.grid_step_y)) +
+                          (ix >> 2) * kBrickFloats +
+                          (((iz & 1u) << 4) | ((iy & 3u) << 2) | (ix & 3u))) * 4u;
+      const uint32_t bx = (ix & 3u) != 3u ? 4u : (kBrickFloats - 3u) * 4u;  // x + 1: same brick or the next
+      const uint32_t by = (iy & 3u) != 3u ? 16u : (s.grid_step_y - 12u) * 4u;
+      const uint32_t bz = (iz & 1u) == 0u ? 64u : (s.grid_step_z - 16u) * 4u;
+      const char* g = reinterpret_cast<const char*>(s.grid);
+      auto at = [&](uint32_t o) { return *reinterpret_cast<const float*>(g + size_t(o)); };
+      c000 = at(b); c100 = at(b + bx); c010 = at(b + by); c110 = at(b + by + bx);
+      c001 = at(b + bz); c101 = at(b + bz + bx); c011 = at(b + by + bz); c111 = at(b + by + bz + bx);
+    }
     const float d00 = mixf(c000, c100, dx), d10 = mixf(c010, c110, dx);
     const float d01 = mixf(c001, c101, dx), d11 = mixf(c011, c111, dx);
     const float d0 = mixf(d00, d10, dy), d1 = mixf(d01, d11, dy);
@@ -540,9 +555,9 @@ NE_DEV float density_gcs(const DevScene& s, Vec3<float> gp) {
   float d0 = mixf(d00, d10, dy), d1 = mixf(d01, d11, dy);
   return mixf(d0, d1, dz);
 }
-template <bool SMALL = false>
+template <int GRID = kGridWide>
 NE_DEV float density_ocs(const DevScene& s, Vec3<float> p) {
-  return density_gcs<SMALL>(s, (p + v3s(0.5f)) * v3(float(s.res[0]), float(s.res[1]), float(s.res[2])));
+  return density_gcs<GRID>(s, (p + v3s(0.5f)) * v3(float(s.res[0]), float(s.res[1]), float(s.res[2])));
 }
 
 // 1 / mu for the tracking step: in FP32 the cell's stored reciprocal (the
@@ -653,17 +668,17 @@ NE_DEV void majorant_dda(const DevScene& s, Vec3<R> oo, Vec3<R> dd, R ta, R tb, 
   }
 }
 
-template <typename R, bool C, bool SMALL = false>
+template <typename R, bool C, int GRID = kGridWide>
 NE_DEV R sigma_at(const DevScene& s, Vec3<R> oo, Vec3<R> dd, R t, Count<C>& cnt) {
   Vec3<R> p = oo + t * dd;
   cnt.lookup();
-  return R(density_ocs<SMALL>(s, v3(float(p.x), float(p.y), float(p.z)))) * R(s.sigma_bar);
+  return R(density_ocs<GRID>(s, v3(float(p.x), float(p.y), float(p.z)))) * R(s.sigma_bar);
 }
 
 // Delta tracking (GridMedia::sample, src/materials/GridMedia.cpp:71-98) with
 // per-cell majorants: step t -= log(1 - xi) * (1 / mu), accept if
 // sigma * (1 / mu) > xi', the reference's multiply-by-inverse form.
-template <typename R, bool C, bool SMALL = false>
+template <typename R, bool C, int GRID = kGridWide>
 NE_DEV bool delta_track(const DevScene& s, Vec3<R> o, Vec3<R> d, R ta, R tb, PathRng& rng, Count<C>& cnt, R& th) {
   Vec3<R> oo = xf_point<R>(s.inv, o), dd = xf_vec<R>(s.inv, d);
   bool hit = false;
@@ -675,7 +690,7 @@ NE_DEV bool delta_track(const DevScene& s, Vec3<R> o, Vec3<R> d, R ta, R tb, Pat
       R r = R(rng.next_keep1());
       t -= log1m_draw(r) * imu;
       if (!(t < c1)) return true;
-      R sig = sigma_at<R, C, SMALL>(s, oo, dd, t, cnt);
+      R sig = sigma_at<R, C, GRID>(s, oo, dd, t, cnt);
       R ra = R(rng.next_buffered());
       if (sig * imu > ra) { hit = true; th = t; return false; }
     }
@@ -684,7 +699,7 @@ NE_DEV bool delta_track(const DevScene& s, Vec3<R> o, Vec3<R> d, R ta, R tb, Pat
 }
 
 // Ratio tracking with the reference's Russian roulette (GridMedia.cpp:54-66).
-template <typename R, bool C, bool SMALL = false>
+template <typename R, bool C, int GRID = kGridWide>
 // A homogeneous medium takes the expectation in closed form,
 // HomogeneousMedia::Tr (HomogeneousMedia.cpp:15-18) with the grey extinction
 // of the tracking step law, and draws nothing.
@@ -699,7 +714,7 @@ NE_DEV R ratio_track(const DevScene& s, Vec3<R> o, Vec3<R> d, R ta, R tb, PathRn
     while (true) {
       t -= log1m_draw(R(rng.next_keep1())) * imu;
       if (!(t < c1)) return true;
-      R sig = sigma_at<R, C, SMALL>(s, oo, dd, t, cnt);
+      R sig = sigma_at<R, C, GRID>(s, oo, dd, t, cnt);
       Tr *= R(1) - xmax(R(0), sig * imu);
       if (Tr < R(0.1)) {
         R q = xmax(R(0.05), R(1) - Tr);

@@ -151,7 +151,7 @@ __device__ __forceinline__ void list_add(PathLists& l, uint32_t buf, int which, 
 // Six waves per SIMD: 80 VGPRs without spills, and six blocks' 26.7 KB of LDS
 // in a CU's 160 KB (seven waves, with half of the walks' state in memory:
 // cloud 123 ms; five waves: 122 ms against 121 ms on an earlier form).
-template <bool GUIDED, bool SMALL>
+template <bool GUIDED, int GRID>
 __global__ __launch_bounds__(kPathBlock, 6) void k_paths(PathArgs args) {
   __shared__ PathSlots P;
   __shared__ PathLists S;
@@ -363,7 +363,7 @@ __global__ __launch_bounds__(kPathBlock, 6) void k_paths(PathArgs args) {
             w.t -= log1m_draw(rng.next_keep1()) * w.imu;
             in = w.t < w.c1;
             if (in) {
-              const float sig = sigma_at<float, false, SMALL>(s, w.oo, w.dd, w.t, cnt);
+              const float sig = sigma_at<float, false, GRID>(s, w.oo, w.dd, w.t, cnt);
               const float ra = rng.next_buffered();
               if (sig * w.imu > ra) {
                 hit = true;
@@ -444,7 +444,7 @@ __global__ __launch_bounds__(kPathBlock, 6) void k_paths(PathArgs args) {
             w.t -= log1m_draw(rng.next_keep1()) * w.imu;
             in = w.t < w.c1;
             if (in) {
-              const float sig = sigma_at<float, false, SMALL>(s, w.oo, w.dd, w.t, cnt);
+              const float sig = sigma_at<float, false, GRID>(s, w.oo, w.dd, w.t, cnt);
               tr *= 1.0f - xmax(0.0f, sig * w.imu);
               if (tr < 0.1f) {  // Russian roulette
                 const float qq = xmax(0.05f, 1.0f - tr);
@@ -506,9 +506,12 @@ size_t paths_scratch_bytes(int cus) {
 hipError_t launch_paths(const DevScene& s, const DevCamera& cam, const WfArgs& a, const GuideUse& gu, void* scratch,
                         int cus, hipStream_t st, StageTimer* tm) {
   hipError_t e = hipSuccess;
-  const bool guided = gu.cache.mix != nullptr, small = s.grid_small != 0 && !a.wide_offsets;
-  void (*fn)(PathArgs) = guided ? (small ? &k_paths<true, true> : &k_paths<true, false>)
-                                : (small ? &k_paths<false, true> : &k_paths<false, false>);
+  const bool guided = gu.cache.mix != nullptr;
+  const int form = a.wide_offsets ? int(kGridWide) : s.grid_form;
+  void (*fn)(PathArgs) =
+      form == kGridQuad    ? (guided ? &k_paths<true, kGridQuad> : &k_paths<false, kGridQuad>)
+      : form == kGridBrick ? (guided ? &k_paths<true, kGridBrick> : &k_paths<false, kGridBrick>)
+                           : (guided ? &k_paths<true, kGridWide> : &k_paths<false, kGridWide>);
   int per_cu = 0;
   if ((e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(fn), kPathBlock, 0)) !=
       hipSuccess)

@@ -249,6 +249,30 @@ hipError_t launch_brick_grid(const float* lin, float* out, const int res[3], hip
   return hipGetLastError();
 }
 
+// Bricked density -> quads: one thread per quad, in storage order.  A quad's
+// four corners come from one or two brick lines, which neighbouring threads
+// share; the kernel is bound by its 16-byte stores.
+__global__ void k_quad_grid(DevScene s, float4* out, uint32_t nbx, uint32_t nby, uint64_t total) {
+  const uint64_t i = uint64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (i >= total) return;
+  const uint32_t inner = uint32_t(i & 7u);
+  const uint64_t b = i >> 3;
+  const uint32_t x = uint32_t(b % nbx) * 2u + (inner & 1u), y = uint32_t((b / nbx) % nby) * 2u + ((inner >> 1) & 1u);
+  const uint32_t z = uint32_t(b / (uint64_t(nbx) * nby)) * 2u + (inner >> 2);
+  const bool in = z < uint32_t(s.res[2]);
+  auto at = [&](uint32_t X, uint32_t Y) {
+    return in && X < uint32_t(s.res[0]) && Y < uint32_t(s.res[1]) ? grid_at(s, int(X), int(Y), int(z)) : 0.0f;
+  };
+  out[i] = make_float4(at(x, y), at(x + 1u, y), at(x, y + 1u), at(x + 1u, y + 1u));
+}
+
+hipError_t launch_quad_grid(const DevScene& s, float4* out, hipStream_t st) {
+  const uint32_t nbx = quad_pad(s.res[0]) / 2u, nby = quad_pad(s.res[1]) / 2u, nbz = quad_pad_z(s.res[2]) / 2u;
+  const uint64_t total = uint64_t(nbx) * nby * nbz * 8u;
+  hipLaunchKernelGGL(k_quad_grid, dim3(uint32_t((total + 255) / 256)), dim3(256), 0, st, s, out, nbx, nby, total);
+  return hipGetLastError();
+}
+
 hipError_t launch_majorants(const DevScene& s, float* maj, hipStream_t st) {
   const uint32_t cells = uint32_t(s.mres) * uint32_t(s.mres) * uint32_t(s.mres);
   const int split = int(cells >= 2048u ? 1u : 2048u / cells);  // at least ~2048 blocks
@@ -333,13 +357,16 @@ __global__ void k_test_delta(DevScene s, int n, const float* rays, uint64_t seed
   }
 }
 
-// Even points take the 32-bit-offset lookup when the grid allows it, odd
-// points the general one, so one call checks both against the caller's values.
+// Odd points take the general lookup, even ones the 32-bit-offset lookups of
+// the bricks and of the quads in turn where the grid allows them, so one call
+// checks all three against the caller's values.
 __global__ void k_test_density(DevScene s, int n, const float* gcs, float* out) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const Vec3<float> p = v3f<float>(gcs + 3 * i);
-  out[i] = (s.grid_small && (i & 1) == 0) ? density_gcs<true>(s, p) : density_gcs<false>(s, p);
+  if ((i & 1) == 0 && (i & 2) == 0 && s.grid_form == kGridQuad) out[i] = density_gcs<kGridQuad>(s, p);
+  else if ((i & 1) == 0 && s.grid_form != kGridWide) out[i] = density_gcs<kGridBrick>(s, p);
+  else out[i] = density_gcs<kGridWide>(s, p);
 }
 
 __global__ void k_test_bsdf(int kind, int n, const float* in0, const float* in1, const float* in2, const float* in3,

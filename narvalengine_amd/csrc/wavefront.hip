@@ -399,8 +399,8 @@ __global__ __launch_bounds__(kChunk) void k_wf_trace(WfState w, WfArgs a, DevSce
 // same trajectories).
 // REGEN (volume-only scenes): the block first makes its chunk's new paths, as
 // k_wf_regen would, which saves that stage's launch every iteration.
-// SMALL: the scene's grid is under 4 GiB (density lookups by 32-bit offsets).
-template <bool C, bool HAS_SURF, bool SPATIAL, bool REGEN, bool SMALL>
+// GRID: how density lookups read the grid (kGrid*).
+template <bool C, bool HAS_SURF, bool SPATIAL, bool REGEN, int GRID>
 __global__ __launch_bounds__(kChunk) void k_wf_medium(WfState w, WfArgs a, DevScene s, DevCamera cam) {
   __shared__ uint32_t red[kChunk / 64];
   __shared__ uint32_t skey[SPATIAL ? kChunk : 1];
@@ -459,7 +459,7 @@ __global__ __launch_bounds__(kChunk) void k_wf_medium(WfState w, WfArgs a, DevSc
         PathRng rng;
         rng.init(a.seed, ppix, psmp, a.job);
         rng.seek(prngn);
-        medium = delta_track<float, C, SMALL>(s, o, d, ta, tb, rng, cnt, th);
+        medium = delta_track<float, C, GRID>(s, o, d, ta, tb, rng, cnt, th);
         A.rngn[i] = rng.consumed();
       }
     }
@@ -558,8 +558,8 @@ __global__ __launch_bounds__(kChunk) void k_wf_guide(WfState w, WfArgs a, DevSce
 // path; frozen guided renders carry none, and are held to the plain stage's
 // 7 waves per SIMD (71 VGPRs, no spills).
 // FUSE (volume-only scenes, plain renders): the stage tracks each vertex's
-// shadow ray itself (ratio tracking, as k_wf_shadow does, 2: by 32-bit grid
-// offsets, 1: 64-bit) and adds the light sample to the path's radiance or
+// shadow ray itself (ratio tracking, as k_wf_shadow does, lookups by the grid
+// form FUSE - 1) and adds the light sample to the path's radiance or
 // the film; no shadow queue, no shadow stage.
 template <bool GUIDED, bool SORT, bool TRAIN, int FUSE = 0>
 __global__ __launch_bounds__(kChunk, (GUIDED && !TRAIN) ? 7 : 1) void k_wf_shade(WfState w, WfArgs a, DevScene s, WfGuide gd) {
@@ -840,7 +840,7 @@ __global__ __launch_bounds__(kChunk, (GUIDED && !TRAIN) ? 7 : 1) void k_wf_shade
       if (box_interval<float>(s, oo, dd, ta, tb)) {
         ta = xmax(ta, 0.0f);
         tb = xmin(tb, tmax);
-        if (ta < tb) tr = ratio_track<float, false, (FUSE == 2)>(s, x, wi, ta, tb, srng, nc);
+        if (ta < tb) tr = ratio_track<float, false, FUSE - 1>(s, x, wi, ta, tb, srng, nc);
       }
       if (tr > 0.0f) {
         const float q = tr * wt * float(s.n_lights) / pl;
@@ -978,8 +978,8 @@ __global__ __launch_bounds__(kChunk) void k_wf_shadow_surf(WfState w, WfArgs a, 
 // the megakernel's transmittance() split by scene content.
 // SPATIAL: the chunk's shadow rays are taken in Morton order of their origins
 // (each keeps its own stream: same transmittances).
-// SMALL: the scene's grid is under 4 GiB (density lookups by 32-bit offsets).
-template <bool C, bool HAS_SURF, bool HAS_VOL, bool SPATIAL, bool SMALL>
+// GRID: how density lookups read the grid (kGrid*).
+template <bool C, bool HAS_SURF, bool HAS_VOL, bool SPATIAL, int GRID>
 __global__ __launch_bounds__(kChunk) void k_wf_shadow(WfState w, WfArgs a, DevScene s) {
   __shared__ uint32_t lds_stack[HAS_SURF ? kShortStack * kChunk : 1];
   __shared__ uint32_t red[kChunk / 64];
@@ -1031,7 +1031,7 @@ __global__ __launch_bounds__(kChunk) void k_wf_shadow(WfState w, WfArgs a, DevSc
       if (box_interval<float>(s, oo, dd, ta, tb)) {
         ta = xmax(ta, 0.0f);
         tb = xmin(tb, tmax);
-        if (ta < tb) tr = ratio_track<float, C, SMALL>(s, x, wi, ta, tb, srng, cnt);
+        if (ta < tb) tr = ratio_track<float, C, GRID>(s, x, wi, ta, tb, srng, cnt);
       }
     }
     if (tr > 0.0f) shadow_deliver(S, B, a, s, k, tr, own);
@@ -1204,7 +1204,7 @@ hipError_t launch_wavefront(const DevScene& s, const DevCamera& cam, WfState& w,
   const bool hs = s.n_nodes > 0, hv = s.has_volume != 0;
   const bool sort = (a.sort & 1) != 0;
   const bool spatial = (a.sort & 2) != 0;  // tracking stages in Morton order of the ray origins
-  const bool small = s.grid_small != 0 && !a.wide_offsets;  // density lookups by 32-bit offsets
+  const int form = a.wide_offsets ? int(kGridWide) : s.grid_form;  // how density lookups read the grid
   // the volume shadow stage reads a continuing path's origin and RNG key
   // from its next record; the surface-only shadow stage reads whole records
   a.shadow_full = hv ? 0 : 1;
@@ -1275,8 +1275,10 @@ hipError_t launch_wavefront(const DevScene& s, const DevCamera& cam, WfState& w,
       NE_MARK(kStageMedium);
 #define NE_MEDIUM(CNT, S_, SP, RG)                                                                       \
   do {                                                                                                   \
-    if (small) hipLaunchKernelGGL((k_wf_medium<CNT, S_, SP, RG, true>), grid, blk, 0, st, w, a, s, cam); \
-    else hipLaunchKernelGGL((k_wf_medium<CNT, S_, SP, RG, false>), grid, blk, 0, st, w, a, s, cam);     \
+    if (form == kGridQuad) hipLaunchKernelGGL((k_wf_medium<CNT, S_, SP, RG, kGridQuad>), grid, blk, 0, st, w, a, s, cam); \
+    else if (form == kGridBrick)                                                                          \
+      hipLaunchKernelGGL((k_wf_medium<CNT, S_, SP, RG, kGridBrick>), grid, blk, 0, st, w, a, s, cam);    \
+    else hipLaunchKernelGGL((k_wf_medium<CNT, S_, SP, RG, kGridWide>), grid, blk, 0, st, w, a, s, cam); \
   } while (0)
       if (spatial) {
         if (count) { if (hs) NE_MEDIUM(true, true, true, false); else NE_MEDIUM(true, false, true, false); }
@@ -1306,11 +1308,13 @@ hipError_t launch_wavefront(const DevScene& s, const DevCamera& cam, WfState& w,
     // volume-only renders (plain, or with a frozen guide and a grid under
     // 4 GiB: the other guided variant would spill): shade tracks the shadow
     // rays itself
-    const bool fuse = hv && !hs && !count && !spatial && !training && (!gh || small);
+    const bool fuse = hv && !hs && !count && !spatial && !training && (!gh || form != kGridWide);
 #define NE_SHADE_FUSED(G, SO, GD)                                                                           \
   do {                                                                                                      \
-    if (small) hipLaunchKernelGGL((k_wf_shade<G, SO, false, 2>), grid, blk, 0, st, w, a, s, GD);           \
-    else hipLaunchKernelGGL((k_wf_shade<G, SO, false, 1>), grid, blk, 0, st, w, a, s, GD);                 \
+    if (form == kGridQuad) hipLaunchKernelGGL((k_wf_shade<G, SO, false, 1 + kGridQuad>), grid, blk, 0, st, w, a, s, GD); \
+    else if (form == kGridBrick)                                                                             \
+      hipLaunchKernelGGL((k_wf_shade<G, SO, false, 1 + kGridBrick>), grid, blk, 0, st, w, a, s, GD);        \
+    else hipLaunchKernelGGL((k_wf_shade<G, SO, false, 1 + kGridWide>), grid, blk, 0, st, w, a, s, GD);     \
   } while (0)
     if (fuse && gh && sort) NE_SHADE_FUSED(true, true, gh->g);
     else if (fuse && gh) NE_SHADE_FUSED(true, false, gh->g);
@@ -1331,8 +1335,9 @@ hipError_t launch_wavefront(const DevScene& s, const DevCamera& cam, WfState& w,
   } while (0)
 #define NE_SHADOW(CNT, S_, V_)                       \
   do {                                               \
-    if (V_ && small) NE_SHADOW_SP(CNT, S_, V_, true); \
-    else NE_SHADOW_SP(CNT, S_, V_, false);           \
+    if (V_ && form == kGridQuad) NE_SHADOW_SP(CNT, S_, V_, kGridQuad);        \
+    else if (V_ && form == kGridBrick) NE_SHADOW_SP(CNT, S_, V_, kGridBrick); \
+    else NE_SHADOW_SP(CNT, S_, V_, kGridWide);       \
   } while (0)
     if (fuse) {
       // done in the shading stage
