@@ -1949,7 +1949,7 @@ ne_status ne_guide_create(ne_ctx* c, const ne_guide_config* cfg_in, ne_guide** o
   g->table_n = size_t(kGuideLevels) * (size_t(1) << n.log2T) * kGuideFeat;
   const size_t cap = size_t(cfg.batch);
   GuideTrain& t = g->train;
-  t.waves = 512;
+  t.parts = 512;
   auto bail = [&](ne_status st) { guide_free(g); delete g; return st; };
   bool ok = guide_alloc(g, n.table, g->table_n) && guide_alloc(g, n.table_bf, g->table_n / kGuideFeat) &&
             guide_alloc(g, n.table_grad, g->table_n) &&
@@ -1960,8 +1960,9 @@ ne_status ne_guide_create(ne_ctx* c, const ne_guide_config* cfg_in, ne_guide** o
             guide_alloc(g, g->batch.s, 10 * cap) && guide_alloc(g, g->batch.count, 1) &&
             guide_alloc(g, t.act, size_t(kGuideLayers) * cap * kGuideWidth) &&
             guide_alloc(g, t.dy, cap * kGuideWidth) && guide_alloc(g, t.dy2, cap * kGuideWidth) &&
-            guide_alloc(g, t.denc, cap * kGuideEnc) && guide_alloc(g, t.partial, size_t(t.waves) * kGuideParams) &&
-            guide_alloc(g, t.loss, 2);
+            guide_alloc(g, t.denc, cap * kGuideEnc) && guide_alloc(g, t.partial, size_t(t.parts) * kGuideParams) &&
+            guide_alloc(g, t.loss, 2) && guide_alloc(g, t.loss_part, 2 * size_t(kGuideFwdBlocks)) && guide_alloc(g, t.aos, 10 * cap);
+  if (ok && guide_table_chunks(n) > 1) ok = guide_alloc(g, t.table_part, size_t(guide_table_chunks(n)) * g->table_n);
   if (ok && cfg.cache_res > 0) {
     const size_t entries = size_t(cfg.cache_res) * cfg.cache_res * cfg.cache_res * size_t(cfg.cache_dirs) * cfg.cache_dirs;
     ok = guide_alloc(g, g->cache_mix, entries * 40);
@@ -2042,16 +2043,10 @@ ne_status ne_guide_train_step(ne_guide* g, int32_t n, const float* smp, int32_t 
       return fail(c, NE_ERR_INVALID_ARG, "sample weights must be finite and >= 0");
   std::lock_guard<std::mutex> lk(c->mu);
   NE_HIP(c, hipSetDevice(c->device));
-  // samples: AoS from the caller -> SoA batch buffer
-  const size_t cap = g->batch.cap;
-  std::vector<float> soa(10 * cap, 0.0f);
-  for (int32_t i = 0; i < n; ++i)
-    for (int k = 0; k < 10; ++k) soa[size_t(k) * cap + size_t(i)] = smp[10 * i + k];
   const uint32_t cnt = uint32_t(n);
-  NE_HIP(c, hipMemcpyAsync(g->batch.s, soa.data(), soa.size() * sizeof(float), hipMemcpyHostToDevice, c->stream));
-  NE_HIP(c, hipMemcpyAsync(g->batch.count, &cnt, sizeof(cnt), hipMemcpyHostToDevice, c->stream));
-  NE_HIP(c, hipMemsetAsync(g->net.table_grad, 0, g->table_n * sizeof(float), c->stream));
-  NE_HIP(c, launch_guide_grad(g->net, g->batch, g->train, c->stream));
+  NE_HIP(c, hipMemcpyAsync(g->train.aos, smp, size_t(n) * 10 * sizeof(float), hipMemcpyHostToDevice, c->stream));
+  NE_HIP(c, launch_guide_set_batch(g->train.aos, g->batch, cnt, c->stream));
+  NE_HIP(c, launch_guide_grad(g->net, g->batch, g->train, cnt, c->stream));
   float lw[2] = {0, 0};
   NE_HIP(c, hipMemcpyAsync(lw, g->train.loss, sizeof(lw), hipMemcpyDeviceToHost, c->stream));
   NE_HIP(c, hipStreamSynchronize(c->stream));

@@ -18,8 +18,10 @@
 // batch of (position, direction, sampled direction w_i, weight r_i).  Backward
 // runs layer by layer over the whole batch; weight gradients are reduced from
 // per-wave partial sums in a fixed order (deterministic), hash-feature
-// gradients are scattered with atomics.  Adam updates FP32 masters; BF16
+// gradients are summed in LDS, range by range.  Adam updates FP32 masters; BF16
 // operand copies (MLP weights and hash features) are re-packed after each step.
+#include <algorithm>
+
 #include "ne_guide.h"
 
 namespace ne {
@@ -81,6 +83,9 @@ __global__ __launch_bounds__(kGuideBlock) void k_guide_bake(GuideNet g, GuideCac
 // ---- training: forward + loss gradient --------------------------------------------
 // Per tile: layer inputs stored for backward (act[l][row][64] BF16), loss
 // gradient w.r.t. the 40 raw outputs into dy (BF16, columns 40..47 zero).
+// A tile is a chain of gathers, layers and the 16 rows' losses: latency, not
+// bandwidth, so every wave takes one tile (65,536 samples in 4096 waves: 75
+// us against 218 us with 8 tiles each in 512 waves and a row's 8 lobes on one lane).
 __global__ __launch_bounds__(kGuideBlock) void k_guide_train_fwd(GuideNet g, GuideBatch b, GuideTrain t) {
   __shared__ uint16_t xa[kWavesPerBlock][16 * kLdA];
   __shared__ uint16_t xb[kWavesPerBlock][16 * kLdA];
@@ -125,73 +130,130 @@ __global__ __launch_bounds__(kGuideBlock) void k_guide_train_fwd(GuideNet g, Gui
     guide_layer<4>(g, xa[wv], xb[wv], out[wv]);
     wave_sync();
 #undef NE_STORE_ACT
-    if (lane < 16) {
-      const uint32_t q = tt * 16 + uint32_t(lane);
-      const float* y = &out[wv][lane * kLdO];
-      float dy[kGuideOutputs];
-      for (int c = 0; c < kGuideOutputs; ++c) dy[c] = 0.0f;
+    {
+      // row r's lobes 2 grp and 2 grp + 1 on lane r + 16 grp; the sums over the
+      // lobes run in lobe order on every lane (values by shuffle), so they
+      // round as one lane's loop would
+      const int row = lane & 15, grp = lane >> 4;
+      const uint32_t q = tt * 16 + uint32_t(row);
+      const float* y = &out[wv][row * kLdO];
+      const float* o = y + 10 * grp;
+      auto lobe_sum = [&](float a, float b) {
+        float acc = 0.0f;
+        for (int k = 0; k < 4; ++k) {
+          acc += __shfl(a, row + 16 * k);
+          acc += __shfl(b, row + 16 * k);
+        }
+        return acc;
+      };
+      const uint32_t qq = q < n ? q : 0u;
+      const Vec3<float> w = v3(S[6 * cap + qq], S[7 * cap + qq], S[8 * cap + qq]);
+      const float r = S[9 * cap + qq];
+      float mx = y[0];
+      for (int k = 1; k < kGuideLobes; ++k) mx = xmax(mx, y[5 * k]);
+      const float e0 = expf(o[0] - mx), e1 = expf(o[5] - mx);
+      const float z = lobe_sum(e0, e1);
+      float pi[2] = {e0 / z, e1 / z}, v[2], kap[2], nm[2], cs[2], mu[2][3];
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const float* p = o + 5 * k;
+        nm[k] = xmax(sqrtf(p[1] * p[1] + p[2] * p[2] + p[3] * p[3]), 1e-12f);
+        kap[k] = guide_kappa(p[4]);
+        v[k] = vmf_pdf(kap[k], (p[1] * w.x + p[2] * w.y + p[3] * w.z) / nm[k]);
+#pragma unroll
+        for (int a = 0; a < 3; ++a) mu[k][a] = p[1 + a] / nm[k];
+        cs[k] = mu[k][0] * w.x + mu[k][1] * w.y + mu[k][2] * w.z;
+      }
+      const float qsum = xmax(lobe_sum(pi[0] * v[0], pi[1] * v[1]), 1e-30f);
       if (q < n) {
-        const Vec3<float> w = v3(S[6 * cap + q], S[7 * cap + q], S[8 * cap + q]);
-        const float r = S[9 * cap + q];
-        float mx = y[0];
-        for (int k = 1; k < kGuideLobes; ++k) mx = xmax(mx, y[5 * k]);
-        float z = 0.0f;
-        for (int k = 0; k < kGuideLobes; ++k) z += expf(y[5 * k] - mx);
-        float pi[kGuideLobes], v[kGuideLobes], qsum = 0.0f;
-        for (int k = 0; k < kGuideLobes; ++k) {
-          const float* o = y + 5 * k;
-          pi[k] = expf(o[0] - mx) / z;
-          const float nm = xmax(sqrtf(o[1] * o[1] + o[2] * o[2] + o[3] * o[3]), 1e-12f);
-          const float c = (o[1] * w.x + o[2] * w.y + o[3] * w.z) / nm;
-          const float kap = guide_kappa(o[4]);
-          v[k] = vmf_pdf(kap, c);
-          qsum += pi[k] * v[k];
+        if (grp == 0) {
+          loss += -r * logf(qsum);
+          wsum += r;
         }
-        qsum = xmax(qsum, 1e-30f);
-        loss += -r * logf(qsum);
-        wsum += r;
-        const float s = -r / qsum;  // d(-r log q) / dq
-        for (int k = 0; k < kGuideLobes; ++k) {
-          const float* o = y + 5 * k;
-          dy[5 * k] = s * pi[k] * (v[k] - qsum);
-          const float nm = xmax(sqrtf(o[1] * o[1] + o[2] * o[2] + o[3] * o[3]), 1e-12f);
-          const float mu[3] = {o[1] / nm, o[2] / nm, o[3] / nm};
-          const float c = mu[0] * w.x + mu[1] * w.y + mu[2] * w.z;
-          const float kap = guide_kappa(o[4]);
-          const float pv = s * pi[k] * v[k];
-          const float wk[3] = {w.x, w.y, w.z};
-          for (int a = 0; a < 3; ++a) dy[5 * k + 1 + a] = pv * kap * (wk[a] - c * mu[a]) / nm;
-          dy[5 * k + 4] = (o[4] < 8.0f && o[4] > -10.0f) ? pv * kap * vmf_dlog_dkappa(kap, c) : 0.0f;
+        const float sc = -r / qsum;  // d(-r log q) / dq
+        uint16_t* d = t.dy + size_t(q) * kGuideWidth;
+        const float wk[3] = {w.x, w.y, w.z};
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          const float* p = o + 5 * k;
+          uint16_t* dk = d + 10 * grp + 5 * k;
+          dk[0] = f2bf(sc * pi[k] * (v[k] - qsum));
+          const float pv = sc * pi[k] * v[k];
+#pragma unroll
+          for (int a = 0; a < 3; ++a) dk[1 + a] = f2bf(pv * kap[k] * (wk[a] - cs[k] * mu[k][a]) / nm[k]);
+          dk[4] = f2bf((p[4] < 8.0f && p[4] > -10.0f) ? pv * kap[k] * vmf_dlog_dkappa(kap[k], cs[k]) : 0.0f);
         }
-        for (int c = 0; c < 48; ++c) t.dy[size_t(q) * kGuideWidth + c] = f2bf(c < kGuideOutputs ? dy[c] : 0.0f);
-        for (int c = 48; c < 64; ++c) t.dy[size_t(q) * kGuideWidth + c] = 0;
+        for (int c = 40 + 6 * grp; c < 46 + 6 * grp; ++c) d[c] = 0;
       }
     }
   }
-  // loss statistics: one atomic pair per wave
+  // loss statistics of the block, summed over the blocks by k_guide_loss
   for (int o = 32; o > 0; o >>= 1) {
     loss += __shfl_down(loss, o);
     wsum += __shfl_down(wsum, o);
   }
+  __shared__ float red[2][kWavesPerBlock];
   if (lane == 0) {
-    atomicAdd(&t.loss[0], loss);
-    atomicAdd(&t.loss[1], wsum);
+    red[0][wv] = loss;
+    red[1][wv] = wsum;
   }
+  __syncthreads();
+  if (threadIdx.x < 2) {
+    float v = 0.0f;
+    for (int k = 0; k < kWavesPerBlock; ++k) v += red[threadIdx.x][k];
+    t.loss_part[2 * blockIdx.x + threadIdx.x] = v;
+  }
+}
+
+// loss[0..1]: the blocks' sums, in a fixed order.
+__global__ __launch_bounds__(256) void k_guide_loss(GuideTrain t, int blocks) {
+  __shared__ float red[2][256];
+  float a = 0.0f, b = 0.0f;
+  for (int k = int(threadIdx.x); k < blocks; k += 256) {
+    a += t.loss_part[2 * k];
+    b += t.loss_part[2 * k + 1];
+  }
+  red[0][threadIdx.x] = a;
+  red[1][threadIdx.x] = b;
+  __syncthreads();
+  for (int w = 128; w > 0; w >>= 1) {
+    if (int(threadIdx.x) < w) {
+      red[0][threadIdx.x] += red[0][threadIdx.x + w];
+      red[1][threadIdx.x] += red[1][threadIdx.x + w];
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x < 2) t.loss[threadIdx.x] = red[threadIdx.x][0];
 }
 
 // ---- training: backward of layer L ------------------------------------------------
 // dy: gradient w.r.t. this layer's (pre-ReLU for hidden, raw for the last) output,
 // BF16 [n][64].  Writes dx = dy W^T masked by the ReLU of this layer's input
 // (which is the previous layer's output) into dx (BF16) or, for L = 0, the
-// encoding gradient into denc (FP32); accumulates this wave's dW / db partial.
+// encoding gradient into denc (FP32, [column][sample], read by level below);
+// accumulates dW / db over the wave's tiles, then over the block's waves in
+// LDS (in wave order), into the block's partial.  Bound by the latency of a
+// tile's loads: 8 waves a block and as many blocks as tiles ask for (65,536
+// samples: 4096 waves of one tile staged in LDS, 29 us per 64 x 64 layer; 41 us
+// with two-byte reads of its columns from memory, 82 us with 512 waves of 8
+// tiles besides).
+constexpr int kBwdBlock = 512, kBwdWaves = kBwdBlock / 64;
 template <int L>
-__global__ __launch_bounds__(kGuideBlock) void k_guide_train_bwd(GuideNet g, GuideBatch b, GuideTrain t,
+__global__ __launch_bounds__(kBwdBlock) void k_guide_train_bwd(GuideNet g, GuideBatch b, GuideTrain t,
                                                                  const uint16_t* dy, uint16_t* dx) {
   constexpr int KIN = guide_in(L), NOUT = guide_out(L);
-  const float scale = t.loss[1] > 0.0f ? 1.0f / t.loss[1] : 0.0f;  // loss normalised by sum r
-  const int lane = __lane_id();
+  // the wave's tile of layer inputs and output gradients (rows of 72: 16-byte
+  // aligned, columns on different banks); the block's sums use the same space
+  // after the tiles
+  constexpr int kLdB = 72;
+  constexpr int kTiles = kBwdWaves * 2 * 16 * kLdB * 2, kSums = (KIN * NOUT + NOUT) * 4;
+  __shared__ __align__(16) unsigned char buf[kTiles > kSums ? kTiles : kSums];
+  const int lane = __lane_id(), wv = int(threadIdx.x >> 6);
+  uint16_t* sx = reinterpret_cast<uint16_t*>(buf) + wv * (2 * 16 * kLdB);
+  uint16_t* sd = sx + 16 * kLdB;
+  float* sw = reinterpret_cast<float*>(buf);
   const int r = lane & 15, kq = 4 * (lane >> 4);
-  const int wid = blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6);
+  const int wid = int(blockIdx.x) * kBwdWaves + wv;
   const uint32_t n = min(*b.count, b.cap);
   const uint32_t tiles = (n + 15) / 16;
   const uint32_t cap = b.cap;
@@ -205,17 +267,29 @@ __global__ __launch_bounds__(kGuideBlock) void k_guide_train_bwd(GuideNet g, Gui
   float db[NOUT / 16];
 #pragma unroll
   for (int nt = 0; nt < NOUT / 16; ++nt) db[nt] = 0.0f;
-  for (uint32_t tt = uint32_t(wid); tt < tiles; tt += uint32_t(t.waves)) {
+  for (uint32_t tt = uint32_t(wid); tt < tiles; tt += gridDim.x * uint32_t(kBwdWaves)) {
     const uint32_t row0 = tt * 16;
+    // 16 rows of 128 bytes each: lane l holds 16 bytes of rows l / 8 and 8 + l / 8
+    wave_sync();
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int row = 8 * h + (lane >> 3), c = 8 * (lane & 7);
+      uint4 vx = make_uint4(0, 0, 0, 0), vd = vx;
+      if (row0 + uint32_t(row) < n) {
+        vx = *reinterpret_cast<const uint4*>(X + size_t(row0 + row) * kGuideWidth + c);
+        vd = *reinterpret_cast<const uint4*>(dy + size_t(row0 + row) * kGuideWidth + c);
+      }
+      *reinterpret_cast<uint4*>(sx + row * kLdB + c) = vx;
+      *reinterpret_cast<uint4*>(sd + row * kLdB + c) = vd;
+    }
+    wave_sync();
     // dx = dy W^T: A = dy rows (k = output index), B = W^T (k = output, n = input)
     f32x4 ax[KIN / 16];
 #pragma unroll
     for (int mt = 0; mt < KIN / 16; ++mt) ax[mt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    const uint32_t ra = row0 + uint32_t(r);
 #pragma unroll
     for (int ks = 0; ks < NOUT / 16; ++ks) {
-      bf16x4 a = bf16x4{0, 0, 0, 0};
-      if (ra < n) a = *reinterpret_cast<const bf16x4*>(dy + size_t(ra) * kGuideWidth + 16 * ks + kq);
+      const bf16x4 a = *reinterpret_cast<const bf16x4*>(sd + r * kLdB + 16 * ks + kq);
 #pragma unroll
       for (int nt = 0; nt < KIN / 16; ++nt) {
         const bf16x4 bb = *reinterpret_cast<const bf16x4*>(wb + (16 * nt + r) * NOUT + 16 * ks + kq);
@@ -230,124 +304,175 @@ __global__ __launch_bounds__(kGuideBlock) void k_guide_train_bwd(GuideNet g, Gui
         const uint32_t row = row0 + uint32_t(kq + j);
         if (row >= n) continue;
         if (L == 0) {
-          if (col < kGuideEnc) t.denc[size_t(row) * kGuideEnc + col] = ax[nt][j];
+          if (col < kGuideEnc) t.denc[size_t(col) * cap + row] = ax[nt][j];
         } else {
-          const float xin = bf2f(X[size_t(row) * kGuideWidth + col]);  // ReLU output of layer L-1
+          const float xin = bf2f(sx[(kq + j) * kLdB + col]);  // ReLU output of layer L-1
           dx[size_t(row) * kGuideWidth + col] = f2bf(xin > 0.0f ? ax[nt][j] : 0.0f);
         }
       }
     }
-    // dW += X^T dy: A = X^T (m = input, k = row), B = dy (k = row, n = output)
+    // dW += X^T dy: A = X^T (m = input, k = row), B = dy (k = row, n = output); rows past n are zero
+    bf16x4 bb[NOUT / 16];
+#pragma unroll
+    for (int nt = 0; nt < NOUT / 16; ++nt)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const uint16_t v = sd[(kq + j) * kLdB + 16 * nt + r];
+        bb[nt][j] = short(v);
+        db[nt] += bf2f(v);
+      }
 #pragma unroll
     for (int mt = 0; mt < KIN / 16; ++mt) {
       bf16x4 a;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const uint32_t row = row0 + uint32_t(kq + j);
-        a[j] = row < n ? short(X[size_t(row) * kGuideWidth + 16 * mt + r]) : short(0);
-      }
+      for (int j = 0; j < 4; ++j) a[j] = short(sx[(kq + j) * kLdB + 16 * mt + r]);
 #pragma unroll
-      for (int nt = 0; nt < NOUT / 16; ++nt) {
-        bf16x4 bb;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const uint32_t row = row0 + uint32_t(kq + j);
-          bb[j] = row < n ? short(dy[size_t(row) * kGuideWidth + 16 * nt + r]) : short(0);
-        }
-        dw[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, bb, dw[mt][nt], 0, 0, 0);
-      }
+      for (int nt = 0; nt < NOUT / 16; ++nt) dw[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, bb[nt], dw[mt][nt], 0, 0, 0);
     }
-#pragma unroll
-    for (int nt = 0; nt < NOUT / 16; ++nt)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const uint32_t row = row0 + uint32_t(kq + j);
-        if (row < n) db[nt] += bf2f(dy[size_t(row) * kGuideWidth + 16 * nt + r]);
-      }
   }
-  // this wave's partial: dW[in][out] (lane: rows kq..kq+3 of each m-tile, column r of each n-tile)
-  float* part = t.partial + size_t(wid) * kGuideParams;
-#pragma unroll
-  for (int mt = 0; mt < KIN / 16; ++mt)
-#pragma unroll
-    for (int nt = 0; nt < NOUT / 16; ++nt)
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        part[guide_w_off(L) + (16 * mt + kq + j) * NOUT + 16 * nt + r] = dw[mt][nt][j] * scale;
+  __syncthreads();  // the tiles' space becomes the block's sums
+  // the block's partial: dW[in][out] (lane: rows kq..kq+3 of each m-tile, column r of each n-tile), db
 #pragma unroll
   for (int nt = 0; nt < NOUT / 16; ++nt) {
-    float s = db[nt];
-    s += __shfl_xor(s, 16);
-    s += __shfl_xor(s, 32);
-    if (lane < 16) part[guide_b_off(L) + 16 * nt + r] = s * scale;
+    db[nt] += __shfl_xor(db[nt], 16);
+    db[nt] += __shfl_xor(db[nt], 32);
   }
+  for (int k = 0; k < kBwdWaves; ++k) {
+    if (wv == k) {
+#pragma unroll
+      for (int mt = 0; mt < KIN / 16; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < NOUT / 16; ++nt)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            float& d = sw[(16 * mt + kq + q) * NOUT + 16 * nt + r];
+            d = k == 0 ? dw[mt][nt][q] : d + dw[mt][nt][q];
+          }
+#pragma unroll
+      for (int nt = 0; nt < NOUT / 16; ++nt)
+        if (lane < 16) {
+          float& d = sw[KIN * NOUT + 16 * nt + r];
+          d = k == 0 ? db[nt] : d + db[nt];
+        }
+    }
+    __syncthreads();
+  }
+  float* part = t.partial + size_t(blockIdx.x) * kGuideParams;
+  for (int e = int(threadIdx.x); e < KIN * NOUT; e += kBwdBlock) part[guide_w_off(L) + e] = sw[e];
+  if (threadIdx.x < NOUT) part[guide_b_off(L) + threadIdx.x] = sw[KIN * NOUT + threadIdx.x];
 }
 
-// mlp_grad[p] = sum over waves of the partials, in a fixed order
-// (deterministic): a block takes 64 parameters, its 4 thread groups sum the
-// waves w = j mod 4 each, and the 4 group sums are added in order.
-__global__ __launch_bounds__(256) void k_guide_reduce(GuideNet g, GuideTrain t) {
-  __shared__ float part[4][64];
+// mlp_grad[p] = sum over the backward blocks of the partials, in a fixed order
+// (deterministic), over sum r: a block takes 64 parameters, its 16 thread groups
+// sum the partials w = j mod 16 each, and the group sums are added in order.
+__global__ __launch_bounds__(1024) void k_guide_reduce(GuideNet g, GuideTrain t, int parts) {
+  const float scale = t.loss[1] > 0.0f ? 1.0f / t.loss[1] : 0.0f;  // loss normalised by sum r
+  __shared__ float part[16][64];
   const int j = int(threadIdx.x >> 6), col = int(threadIdx.x & 63);
   const int p = int(blockIdx.x) * 64 + col;
   float s = 0.0f;
   if (p < kGuideParams)
-    for (int w = j; w < t.waves; w += 4) s += t.partial[size_t(w) * kGuideParams + p];
+#pragma unroll 4
+    for (int w = j; w < parts; w += 16) s += t.partial[size_t(w) * kGuideParams + p];
   part[j][col] = s;
   __syncthreads();
-  if (j == 0 && p < kGuideParams) g.mlp_grad[p] = ((part[0][col] + part[1][col]) + part[2][col]) + part[3][col];
+  if (j == 0 && p < kGuideParams) {
+    float v = part[0][col];
+    for (int k = 1; k < 16; ++k) v += part[k][col];
+    g.mlp_grad[p] = v * scale;
+  }
 }
 
-// hash-feature gradients: scatter denc * corner weight (scaled) into
-// table_grad.  One thread per sample, levels in turn.  On the coarse levels
-// (resolution <= 64) the samples of a wave mostly share corners, so the wave
-// first merges equal entries: the lowest pending lane's entry is taken, the
-// lanes holding it are summed across the wave and one lane adds the sum (up
-// to 4 entries per corner); whatever is left, and every finer level, adds
-// directly.
-__global__ __launch_bounds__(256) void k_guide_table_grad(GuideNet g, GuideBatch b, GuideTrain t) {
+// Hash-feature gradients: every sample adds (corner weight x encoding
+// gradient) to 8 entries per level.  As global atomics that is 16.8 M adds per
+// 65,536 samples, at about 11 G/s across the XCDs (0.9 ms uniform positions,
+// 1.5 ms in a cloud).  Instead a block owns kTableRange entries of one level in
+// LDS, reads a share of the samples, adds what falls into its range by LDS
+// atomics, and writes the range once: no global atomics.  The sums are FP64
+// because the LDS adds doubles nine times as fast as floats (64 random adds of
+// a wave: ds_add_f64 21 cycles, ds_add_f32 194).  A sample is read by every
+// block of its level, but only the blocks that own one of its corners work on
+// it: tables of more ranges than the chip has CUs take all samples in every
+// block; smaller ones split the samples into `chunks` and sum the chunks'
+// copies after (k_guide_table_sum).  The whole training pass with its copies,
+// 65,536 samples, this kernel against atomics at every level, us:
+// log2_table 15: 488 / 1306, 17: 648 / 1292, 19: 658 / 1301, 21: 971 / 1360;
+// 8192 samples: 15: 316 / 454, 21: 279 / 333.  Atomics for the large levels
+// only lost at every size too (19: 1038).
+constexpr uint32_t kTableRange = 8192;   // 128 KiB of LDS: one block per CU
+constexpr int kTableBlock = 1024;
+// entries that level l addresses (dense levels fewer than the table holds)
+__host__ __device__ inline uint32_t guide_level_entries(const GuideNet& g, int l) {
+  const uint32_t T = 1u << g.log2T, r1 = uint32_t(g.res[l]) + 1u;
+  const uint64_t dense = uint64_t(r1) * r1 * r1;
+  return dense <= T ? uint32_t(dense) : T;
+}
+__global__ __launch_bounds__(kTableBlock) void k_guide_table_grad(GuideNet g, GuideBatch b, GuideTrain t, int chunks,
+                                                                  float* out, size_t stride) {
+  __shared__ double acc[2 * kTableRange];
+  // blockIdx -> level, range of the level, chunk of the samples
+  uint32_t unit = blockIdx.x / uint32_t(chunks), chunk = blockIdx.x % uint32_t(chunks);
+  int l = 0;
+  uint32_t ent = guide_level_entries(g, 0), nr = (ent + kTableRange - 1) / kTableRange;
+  while (unit >= nr) {
+    unit -= nr;
+    ++l;
+    ent = guide_level_entries(g, l);
+    nr = (ent + kTableRange - 1) / kTableRange;
+  }
+  const uint32_t base = unit * kTableRange, len = ent - base < kTableRange ? ent - base : kTableRange;
+  for (uint32_t k = threadIdx.x; k < 2 * len; k += kTableBlock) acc[k] = 0.0;
+  __syncthreads();
   const float scale = t.loss[1] > 0.0f ? 1.0f / t.loss[1] : 0.0f;
-  const uint32_t n = min(*b.count, b.cap);
-  const uint32_t q = blockIdx.x * blockDim.x + threadIdx.x;
-  const bool valid = q < n;  // no early exit: every lane takes part in the wave merges
-  const int lane = __lane_id();
-  const uint32_t qq = valid ? q : 0u;
-  const Vec3<float> p = v3(b.s[qq], b.s[b.cap + qq], b.s[2 * b.cap + qq]);
-  for (int l = 0; l < kGuideLevels; ++l) {
-    const float d0 = valid ? t.denc[size_t(qq) * kGuideEnc + 2 * l] * scale : 0.0f;
-    const float d1 = valid ? t.denc[size_t(qq) * kGuideEnc + 2 * l + 1] * scale : 0.0f;
-    const bool coarse = g.res[l] <= 64;  // the same for every lane
+  const uint32_t n = min(*b.count, b.cap), T = 1u << g.log2T, r1 = uint32_t(g.res[l]) + 1u;
+  const uint32_t per = (n + uint32_t(chunks) - 1) / uint32_t(chunks), q1 = min(n, (chunk + 1) * per);
+  const bool dense = uint64_t(r1) * r1 * r1 <= T;
+  const float rf = float(g.res[l]);
+  const float* D0 = t.denc + size_t(2 * l) * b.cap;
+  for (uint32_t q = chunk * per + threadIdx.x; q < q1; q += kTableBlock) {
+    // the corners of guide_corner, their shared parts computed once
+    const float sx = xmin(xmax(b.s[q], 0.0f), 1.0f) * rf, sy = xmin(xmax(b.s[b.cap + q], 0.0f), 1.0f) * rf,
+                sz = xmin(xmax(b.s[2 * size_t(b.cap) + q], 0.0f), 1.0f) * rf;
+    const float fx = xmin(floorf(sx), rf - 1.0f), fy = xmin(floorf(sy), rf - 1.0f), fz = xmin(floorf(sz), rf - 1.0f);
+    const float tx = sx - fx, ty = sy - fy, tz = sz - fz;
+    const uint32_t x = uint32_t(fx), y = uint32_t(fy), z = uint32_t(fz);
+    const uint32_t my = dense ? r1 : 2654435761u, mz = dense ? r1 * r1 : 805459861u;
+    const uint32_t hy0 = y * my, hy1 = hy0 + my, hz0 = z * mz, hz1 = hz0 + mz;
+    uint32_t e[8];
+    bool any = false;
+#pragma unroll
     for (int k = 0; k < 8; ++k) {
-      uint32_t ent;
-      float w;
-      guide_corner(g, l, p, k, ent, w);
-      const float v0 = w * d0, v1 = w * d1;
-      bool pend = valid && (v0 != 0.0f || v1 != 0.0f);
-      if (coarse) {
-        for (int it = 0; it < 4; ++it) {
-          const uint64_t m = __ballot(pend);
-          if (m == 0) break;
-          const int leader = __ffsll((long long)m) - 1;
-          const uint32_t key = uint32_t(__shfl(int(ent), leader));
-          const bool mine = pend && ent == key;
-          float s0 = mine ? v0 : 0.0f, s1 = mine ? v1 : 0.0f;
-          for (int o = 32; o > 0; o >>= 1) {
-            s0 += __shfl_xor(s0, o);
-            s1 += __shfl_xor(s1, o);
-          }
-          if (lane == leader) {
-            atomicAdd(&g.table_grad[2 * size_t(key)], s0);
-            atomicAdd(&g.table_grad[2 * size_t(key) + 1], s1);
-          }
-          pend = pend && !mine;
-        }
-      }
-      if (pend) {
-        atomicAdd(&g.table_grad[2 * size_t(ent)], v0);
-        atomicAdd(&g.table_grad[2 * size_t(ent) + 1], v1);
+      const uint32_t xx = x + (k & 1), yy = (k & 2) ? hy1 : hy0, zz = (k & 4) ? hz1 : hz0;
+      e[k] = (dense ? xx + yy + zz : (xx ^ yy ^ zz) & (T - 1u)) - base;
+      any = any || e[k] < len;
+    }
+    if (!any) continue;
+    const float d0 = D0[q] * scale, d1 = D0[b.cap + q] * scale;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const float w = ((k & 1) ? tx : 1.0f - tx) * ((k & 2) ? ty : 1.0f - ty) * ((k & 4) ? tz : 1.0f - tz);
+      if (e[k] < len) {
+        atomicAdd(&acc[2 * e[k]], double(w * d0));
+        atomicAdd(&acc[2 * e[k] + 1], double(w * d1));
       }
     }
   }
+  __syncthreads();
+  float2* o = reinterpret_cast<float2*>(out + size_t(chunk) * stride) + size_t(l) * T + base;
+  for (uint32_t k = threadIdx.x; k < len; k += kTableBlock) o[k] = make_float2(float(acc[2 * k]), float(acc[2 * k + 1]));
+}
+// table_grad = the chunks' copies summed in order, over the entries the levels address
+__global__ __launch_bounds__(256) void k_guide_table_sum(GuideNet g, const float* part, size_t stride, int chunks) {
+  const uint32_t T = 1u << g.log2T;
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x, l = i >> g.log2T, k = i & (T - 1u);
+  if (l >= uint32_t(kGuideLevels) || k >= guide_level_entries(g, int(l))) return;
+  float2 s = reinterpret_cast<const float2*>(part)[i];
+  for (int c = 1; c < chunks; ++c) {
+    const float2 v = reinterpret_cast<const float2*>(part + size_t(c) * stride)[i];
+    s.x += v.x;
+    s.y += v.y;
+  }
+  reinterpret_cast<float2*>(g.table_grad)[i] = s;
 }
 
 // BF16 copy of the hash features that the encoder reads (after every change
@@ -451,24 +576,55 @@ hipError_t launch_guide_bake(const GuideNet& g, const GuideCache& c, float* mix,
   return hipGetLastError();
 }
 
-__global__ void k_guide_zero_loss(GuideTrain t) {
-  if (threadIdx.x < 2) t.loss[threadIdx.x] = 0.0f;
+// Training samples as the caller gives them (10 floats each) -> the batch's
+// arrays, by a block of 256 samples through LDS; *count = n.
+__global__ __launch_bounds__(256) void k_guide_set_batch(const float* aos, GuideBatch b, uint32_t n) {
+  __shared__ float v[256 * 11];  // a row of 11: conflict-free columns
+  const uint32_t q0 = blockIdx.x * 256u, m = n - q0 < 256u ? n - q0 : 256u;
+  for (uint32_t e = threadIdx.x; e < 10u * m; e += 256u) v[e / 10u * 11u + e % 10u] = aos[size_t(q0) * 10u + e];
+  __syncthreads();
+  if (threadIdx.x < m)
+    for (uint32_t k = 0; k < 10u; ++k) b.s[size_t(k) * b.cap + q0 + threadIdx.x] = v[threadIdx.x * 11u + k];
+  if (blockIdx.x == 0 && threadIdx.x == 0) *b.count = n;
+}
+hipError_t launch_guide_set_batch(const float* aos, const GuideBatch& b, uint32_t n, hipStream_t st) {
+  hipLaunchKernelGGL(k_guide_set_batch, dim3((n + 255) / 256), dim3(256), 0, st, aos, b, n);
+  return hipGetLastError();
 }
 
-// Gradients of the weight-normalised loss -sum r log q / sum r (the scale
-// 1 / sum r is read on the device after the forward pass).
-hipError_t launch_guide_grad(const GuideNet& g, const GuideBatch& b, const GuideTrain& t, hipStream_t st) {
-  const dim3 blk(kGuideBlock);
-  const uint32_t blocks = uint32_t(t.waves / kWavesPerBlock);
-  hipLaunchKernelGGL(k_guide_zero_loss, dim3(1), dim3(64), 0, st, t);
-  hipLaunchKernelGGL(k_guide_train_fwd, dim3(blocks), blk, 0, st, g, b, t);
+static int table_units(const GuideNet& g) {
+  int units = 0;
+  for (int l = 0; l < kGuideLevels; ++l) units += int((guide_level_entries(g, l) + kTableRange - 1) / kTableRange);
+  return units;
+}
+// Chunks of the samples in the table gradient: as many as fill the chip once
+// (256 CUs, one block each), at most kGuideTableChunks.
+int guide_table_chunks(const GuideNet& g) {
+  return std::min(kGuideTableChunks, std::max(1, 256 / table_units(g)));
+}
+
+// Gradients of the weight-normalised loss -sum r log q / sum r (1 / sum r is
+// read on the device after the forward pass).  n: at least the sample count.
+hipError_t launch_guide_grad(const GuideNet& g, const GuideBatch& b, const GuideTrain& t, uint32_t n, hipStream_t st) {
+  const uint32_t tiles = std::max<uint32_t>(1, (std::min(n, b.cap) + 15) / 16);
+  const uint32_t fblocks = std::min<uint32_t>(kGuideFwdBlocks, (tiles + kWavesPerBlock - 1) / kWavesPerBlock);
+  const uint32_t blocks = std::min<uint32_t>(uint32_t(t.parts), (tiles + kBwdWaves - 1) / kBwdWaves);
+  const dim3 blk(kBwdBlock);
+  hipLaunchKernelGGL(k_guide_train_fwd, dim3(fblocks), dim3(kGuideBlock), 0, st, g, b, t);
+  hipLaunchKernelGGL(k_guide_loss, dim3(1), dim3(256), 0, st, t, int(fblocks));
   hipLaunchKernelGGL((k_guide_train_bwd<4>), dim3(blocks), blk, 0, st, g, b, t, t.dy, t.dy2);
   hipLaunchKernelGGL((k_guide_train_bwd<3>), dim3(blocks), blk, 0, st, g, b, t, t.dy2, t.dy);
   hipLaunchKernelGGL((k_guide_train_bwd<2>), dim3(blocks), blk, 0, st, g, b, t, t.dy, t.dy2);
   hipLaunchKernelGGL((k_guide_train_bwd<1>), dim3(blocks), blk, 0, st, g, b, t, t.dy2, t.dy);
   hipLaunchKernelGGL((k_guide_train_bwd<0>), dim3(blocks), blk, 0, st, g, b, t, t.dy, t.dy2);
-  hipLaunchKernelGGL(k_guide_reduce, dim3((kGuideParams + 63) / 64), dim3(256), 0, st, g, t);
-  hipLaunchKernelGGL(k_guide_table_grad, dim3((b.cap + 255) / 256), dim3(256), 0, st, g, b, t);
+  hipLaunchKernelGGL(k_guide_reduce, dim3((kGuideParams + 63) / 64), dim3(1024), 0, st, g, t, int(blocks));
+  const int chunks = guide_table_chunks(g);
+  const size_t words = table_words(g);
+  float* out = chunks == 1 ? g.table_grad : t.table_part;
+  hipLaunchKernelGGL(k_guide_table_grad, dim3(uint32_t(table_units(g) * chunks)), dim3(kTableBlock), 0, st, g, b, t,
+                     chunks, out, words);
+  if (chunks > 1)
+    hipLaunchKernelGGL(k_guide_table_sum, dim3(uint32_t((words / 2 + 255) / 256)), dim3(256), 0, st, g, out, words, chunks);
   return hipGetLastError();
 }
 

@@ -249,11 +249,17 @@ struct GuideTrain {
   uint16_t* act;       // 5 layers x cap x 64 BF16 layer inputs
   uint16_t* dy;        // cap x 64 BF16 output gradient of the current layer
   uint16_t* dy2;       // cap x 64 BF16 (ping-pong)
-  float* denc;         // cap x 32 encoding gradient
-  float* partial;      // waves x kGuideParams weight/bias gradient partials
+  float* denc;         // 32 x cap encoding gradient
+  float* partial;      // parts x kGuideParams weight/bias gradient partials
   float* loss;         // [0] summed loss, [1] summed weight
-  int32_t waves;
+  float* loss_part;    // the same per forward block
+  float* aos;          // samples as the caller gave them (10 floats each)
+  float* table_part;   // table gradient per chunk of the samples (guide_table_chunks > 1)
+  int32_t parts;       // backward blocks at most
 };
+constexpr uint32_t kGuideFwdBlocks = 8192;
+constexpr int kGuideTableChunks = 16;
+int guide_table_chunks(const GuideNet& g);  // copies of the table gradient that a step keeps
 
 // Guided wavefront: per-path training record (one per slot and path buffer).
 // state 0: none; 1: a guided vertex was sampled, the radiance baseline is
@@ -299,8 +305,11 @@ hipError_t launch_guide_bake(const GuideNet& g, const GuideCache& c, float* mix,
 hipError_t launch_guide_eval(const GuideNet& g, int n, const float* in6, float* out40, hipStream_t st);
 // raw network outputs (n x 40) before the head, for parity tests
 hipError_t launch_guide_raw(const GuideNet& g, int n, const float* in6, float* out40, hipStream_t st);
-// one step on the batch: forward, loss gradient, backward into mlp_grad / table_grad (no update)
-hipError_t launch_guide_grad(const GuideNet& g, const GuideBatch& b, const GuideTrain& t, hipStream_t st);
+// n samples of 10 floats (device memory) into the batch
+hipError_t launch_guide_set_batch(const float* aos, const GuideBatch& b, uint32_t n, hipStream_t st);
+// one step on the batch's samples (at most n of them): forward, loss gradient, backward into mlp_grad /
+// table_grad (both overwritten; no update)
+hipError_t launch_guide_grad(const GuideNet& g, const GuideBatch& b, const GuideTrain& t, uint32_t n, hipStream_t st);
 hipError_t launch_guide_adam(const GuideNet& g, float lr_table, float lr_mlp, float beta1, float beta2, float eps,
                              int step, hipStream_t st);
 

@@ -1249,7 +1249,7 @@ hipError_t launch_wavefront(const DevScene& s, const DevCamera& cam, WfState& w,
       }
       if (gh && gh->g.train && h_status[1] >= gh->min_batch) {
         NE_MARK(kStageTrain);
-        if ((e = launch_guide_grad(gh->g.net, gh->g.batch, gh->train, st)) != hipSuccess) return e;
+        if ((e = launch_guide_grad(gh->g.net, gh->g.batch, gh->train, h_status[1], st)) != hipSuccess) return e;
         gh->steps += 1;
         gh->samples += std::min(h_status[1], gh->g.batch.cap);
         if ((e = launch_guide_adam(gh->g.net, gh->lr_table, gh->lr_mlp, gh->beta1, gh->beta2, gh->eps,

@@ -90,6 +90,34 @@ def test_guide_gradients_match_reference(ctx):
     g.close()
 
 
+@pytest.mark.parametrize("n,log2_table", [(1, 10), (15, 12), (16, 14), (17, 19), (4095, 17), (8193, 16), (65553, 13)])
+def test_guide_gradients_at_the_edges_of_the_launch(ctx, n, log2_table):
+    """One tile and its remainders, a block's waves filled or not, more tiles
+    than waves; table ranges split over chunks of the samples (small tables)
+    or not (log2_table >= 17), dense and hashed levels.  The network's gradient
+    is held to the bound of the BF16 points above; the table's, of the device's
+    own FP32 arithmetic, to the same."""
+    print_case(f"guide gradients: {n} samples, log2_table {log2_table}")
+    g = Guide(ctx, log2_table=log2_table, batch=max(16, n), seed=1)
+    table, mlp = _random_params(g, 5)
+    g.set_params(table, mlp)
+    rng = np.random.default_rng(n)
+    w = rng.normal(size=(n, 3))
+    w /= np.linalg.norm(w, axis=1, keepdims=True)
+    s = np.concatenate([_queries(n, n + 1), w, rng.uniform(0.1, 2.0, (n, 1))], 1).astype(np.float32)
+    loss = g.train_step(s, update=False)
+    assert g.train_step(s, update=False) == loss  # gradients are written, not added to
+    gt, gm = g.grads()
+    rl, rt, rm = G.loss_and_grad(s, table, mlp, g.level_res, log2_table, quantize=True)
+    assert abs(loss - rl) < 1e-3 * abs(rl) + 1e-4, (loss, rl)
+    for got, ref in ((gm, rm), (gt, rt)):
+        cos = got @ ref / (np.linalg.norm(got) * np.linalg.norm(ref))
+        rel = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+        assert cos > 0.995 and rel < 0.08, (cos, rel)
+    assert not gt[rt == 0.0].any()  # entries that no sample's corner names
+    g.close()
+
+
 def test_guide_learns_a_position_dependent_lobe(ctx):
     """Samples drawn from one vMF lobe whose mean depends on position: training
     must raise the proposal density of the true mean direction."""
