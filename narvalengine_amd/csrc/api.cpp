@@ -572,17 +572,33 @@ ne_status ne_scene_upload(ne_ctx* c, const ne_scene_desc* d, ne_scene** out) {
       storage[i] = rslot++;
     }
   }
-  // leaf children: refs position -> storage slot of the leaf's type
-  for (size_t k = 0; k < bvh.nodes.size() / kNodeFloats; ++k) {
-    float* f = &bvh.nodes[k * kNodeFloats];
-    uint32_t meta;
+  // device nodes: planes decoded (a byte times a power of two is exact: each
+  // plane rounds once), leaf children as work items on their type's storage
+  const size_t n_nodes = bvh.nodes.size() / kNodeFloats;
+  std::vector<float> nodes(n_nodes * 4 * kNodeQuads, 0.0f);
+  for (size_t k = 0; k < n_nodes; ++k) {
+    const float* f = &bvh.nodes[k * kNodeFloats];
+    float* o = &nodes[k * 4 * kNodeQuads];
+    uint32_t exps, q[6], meta;
+    std::memcpy(&exps, &f[3], 4);
+    std::memcpy(q, &f[4], 24);
     std::memcpy(&meta, &f[10], 4);
+    for (int a = 0; a < 3; ++a) {
+      const float sc = std::ldexp(1.0f, int((exps >> (8 * a)) & 0xFFu) - 127);
+      for (int ch = 0; ch < 4; ++ch) {
+        o[8 * a + ch] = float((q[a] >> (8 * ch)) & 0xFFu) * sc + f[a];
+        o[8 * a + 4 + ch] = float((q[3 + a] >> (8 * ch)) & 0xFFu) * sc + f[a];
+      }
+    }
     for (int ch = 0; ch < 4; ++ch) {
-      int32_t first;
-      std::memcpy(&first, &f[12 + ch], 4);
-      if (first < 0 || ((meta >> (8 * ch)) & kMetaLeaf) == 0) continue;
-      int32_t slot = int32_t(storage[size_t(first)]);
-      std::memcpy(&f[12 + ch], &slot, 4);
+      int32_t ref;
+      std::memcpy(&ref, &f[12 + ch], 4);
+      const uint32_t m = (meta >> (8 * ch)) & 0xFFu;
+      uint32_t item = uint32_t(ref);
+      if (ref < 0) item = kItemNone;
+      else if (m & kMetaLeaf)
+        item = kItemLeaf | (((m >> 4) & 3u) << 29) | (((m & 15u) - 1u) << kItemCountShift) | storage[size_t(ref)];
+      std::memcpy(&o[24 + ch], &item, 4);
     }
   }
   // emissive primitives in the light-selection order: rectangles, spheres,
@@ -604,10 +620,10 @@ ne_status ne_scene_upload(ne_ctx* c, const ne_scene_desc* d, ne_scene** out) {
     emitters.push_back(uint32_t(kLightPoint) << 30 | q);
   }
   const float4* f4 = nullptr;
-  if ((st = dev_upload(c, s, reinterpret_cast<const float4*>(bvh.nodes.data()), bvh.nodes.size() / 4, &f4)) != NE_OK)
+  if ((st = dev_upload(c, s, reinterpret_cast<const float4*>(nodes.data()), nodes.size() / 4, &f4)) != NE_OK)
     return bail(st);
   ds.nodes = f4;
-  ds.n_nodes = uint32_t(bvh.nodes.size() / kNodeFloats);
+  ds.n_nodes = uint32_t(n_nodes);
   if ((st = dev_upload(c, s, reinterpret_cast<const float4*>(tris.data()), tris.size() / 4, &ds.tris)) != NE_OK)
     return bail(st);
   if ((st = dev_upload(c, s, reinterpret_cast<const float4*>(sph.data()), sph.size() / 4, &ds.sph)) != NE_OK)

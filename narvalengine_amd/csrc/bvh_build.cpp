@@ -1,5 +1,5 @@
-// bvh_build.cpp -- host binned-SAH BVH builder producing the device layout
-// described in ne_scene.h: a binary SAH tree collapsed to 4-wide nodes that
+// bvh_build.cpp -- host binned-SAH BVH builder producing the nodes
+// described in bvh_build.h: a binary SAH tree collapsed to 4-wide nodes that
 // store their children's boxes quantized to 8 bits per plane against the
 // node's own box (conservatively: the FP32 decode the traversal performs
 // always contains the true box), leaves referenced from the parent, wide

@@ -2,18 +2,14 @@
 // code and kernels).
 //
 // HBM layout (all arrays 16-byte aligned):
-//   nodes   4-wide BVH, 64 B per node = 4 x float4, child boxes quantized
-//           to 8 bits per plane against the node's box:
-//             f0 = (origin.xyz, exponents: byte a = e_a + 127)
-//             f1 = (qlo.x, qlo.y, qlo.z, qhi.x)  f2 = (qhi.y, qhi.z, meta, 0)
-//             f3 = int child[4]
-//           each q word holds one byte per child; child c's box on axis a is
-//           [origin_a + qlo_a[c] * 2^e_a, origin_a + qhi_a[c] * 2^e_a] in FP32
-//           (the builder makes that decode contain the true box).  meta byte
-//           c is 0 for an inner child (child[c] = node index) or
-//           0x80 | type << 4 | count for a leaf of count primitives of type
-//           (0 triangle, 1 sphere, 2 rectangle) at slots [child[c],
-//           child[c] + count) of that type's array.  child < 0: empty slot.
+//   nodes   4-wide BVH, 128 B per node (one cache line) = 8 x float4:
+//             lo.x hi.x lo.y hi.y lo.z hi.z of the four children's boxes,
+//             their four work items (kItem*; kItemNone: no child), 16 B unused.
+//           The builder's nodes hold the planes quantized to 8 bits
+//           (bvh_build.h); upload decodes them once, so that a visit does not:
+//           a byte, scale and origin per plane were 48 of a visit's 290 VALU
+//           instructions, unpacking the children's items 32 more.  A ray reads
+//           an axis' near planes from offset 0 or 16 by its direction's sign.
 //   tris    48 B per triangle in leaf order: (v0, material), (v1-v0, original
 //           index), (v2-v0, 0).  Original index = position in the input.
 //   sph     (centre, radius) in leaf order + material and original-index
@@ -47,6 +43,7 @@ constexpr uint32_t kItemLeaf = 0x80000000u;
 constexpr uint32_t kItemFirstMask = (1u << 26) - 1;  // slots per primitive type < 2^26
 constexpr uint32_t kItemCountShift = 26;
 constexpr uint32_t kItemNone = 0xFFFFFFFFu;  // no item (leaf type 3 does not exist)
+constexpr uint32_t kNodeQuads = 8;    // float4 per node
 constexpr uint32_t kItemMaxLeaf = 8;  // count - 1 in 3 bits
 
 // Density grid layout: bricks of 4 x 4 x 2 voxels (32 floats: one 128-byte

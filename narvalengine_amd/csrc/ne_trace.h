@@ -149,25 +149,26 @@ NE_DEV bool isect_rect(const float4* rc, Vec3<R> o, Vec3<R> d, R tmin, R tmax, R
   return true;
 }
 
-// Conservative slab test against a float box (Ize 2013: far distances scaled
-// by 1 + 2 gamma(3)).  invd is finite (trav_init keeps |d| >= 2^-100 per
-// axis), so no (plane - o) * invd is 0 * inf and min/max see no NaN.  The far
-// scale is applied once to the smallest far distance: multiplying by a
-// positive constant is monotone, so this equals scaling each one.
 NE_DEV float fmin_(float a, float b) { return __builtin_fminf(a, b); }
 NE_DEV double fmin_(double a, double b) { return __builtin_fmin(a, b); }
 NE_DEV float fmax_(float a, float b) { return __builtin_fmaxf(a, b); }
 NE_DEV double fmax_(double a, double b) { return __builtin_fmax(a, b); }
+// Conservative slab test against a float box (Ize 2013: far distances scaled
+// by 1 + 2 gamma(3)) from the planes that the direction's signs make near and
+// far.  invd is finite (trav_init keeps |d| >= 2^-100 per axis), so no
+// (plane - o) * invd is 0 * inf, and the product is monotone in the plane: the
+// near plane's is the smaller one.  The far scale is applied once to the
+// smallest far distance: multiplying by a positive constant is monotone, so
+// this equals scaling each one.
 template <typename R>
-NE_DEV bool slab(float mnx, float mny, float mnz, float mxx, float mxy, float mxz, Vec3<R> o, Vec3<R> invd, R tmax,
-                 R& tent) {
-  const R nx = (R(mnx) - o.x) * invd.x, fx = (R(mxx) - o.x) * invd.x;
-  const R ny = (R(mny) - o.y) * invd.y, fy = (R(mxy) - o.y) * invd.y;
-  const R nz = (R(mnz) - o.z) * invd.z, fz = (R(mxz) - o.z) * invd.z;
-  const R t0 = fmax_(fmax_(R(0), fmin_(nx, fx)), fmax_(fmin_(ny, fy), fmin_(nz, fz)));
-  const R far = fmin_(fmax_(nx, fx), fmin_(fmax_(ny, fy), fmax_(nz, fz))) * R(1.0000003576);
+NE_DEV bool slab(float px, float py, float pz, float qx, float qy, float qz, Vec3<R> o, Vec3<R> invd, R tmax, R& tent) {
+  const R nx = (R(px) - o.x) * invd.x, fx = (R(qx) - o.x) * invd.x;
+  const R ny = (R(py) - o.y) * invd.y, fy = (R(qy) - o.y) * invd.y;
+  const R nz = (R(pz) - o.z) * invd.z, fz = (R(qz) - o.z) * invd.z;
+  const R t0 = fmax_(R(0), fmax_(nx, fmax_(ny, nz)));
+  const R far = fmin_(fx, fmin_(fy, fz)) * R(1.0000003576);
   tent = t0;
-  return t0 <= fmin_(tmax, far);
+  return t0 <= far && t0 <= tmax;
 }
 
 template <typename R>
@@ -195,6 +196,7 @@ template <typename R>
 struct TravState {
   Vec3<R> o, d, invd;
   R tmin, tmax, best;
+  uint32_t nx, ny, nz;  // byte offset of the near planes within an axis' pair (0 or 16)
   uint32_t cur, leaf, bkey, bslot;  // leaf: parked leaf item (trav_step_wave), or kItemNone
   int sp, btype;
   bool found;
@@ -209,6 +211,9 @@ NE_DEV void trav_init(TravState<R>& st, Vec3<R> o, Vec3<R> d, R tmin, R tmax) {
   const R tiny = R(7.888609052210118e-31);  // 2^-100
   auto nz = [tiny](R v) { return xfabs(v) < tiny ? (__builtin_signbit(v) ? -tiny : tiny) : v; };
   st.invd = v3(R(1) / nz(d.x), R(1) / nz(d.y), R(1) / nz(d.z));
+  st.nx = __builtin_signbit(st.invd.x) ? 16u : 0u;
+  st.ny = __builtin_signbit(st.invd.y) ? 16u : 0u;
+  st.nz = __builtin_signbit(st.invd.z) ? 16u : 0u;
   st.tmin = tmin;
   st.tmax = tmax;
   st.best = tmax;
@@ -219,16 +224,6 @@ NE_DEV void trav_init(TravState<R>& st, Vec3<R> o, Vec3<R> d, R tmin, R tmax) {
   st.btype = 0;
   st.bkey = 0;
   st.bslot = 0;
-}
-
-// Byte c of a packed word of quantized planes, as a float.
-NE_DEV float qbyte(uint32_t w, int c) { return float((w >> (8 * c)) & 0xFFu); }
-// Child c of a wide node -> work item: an inner node index, or for a leaf
-// (meta byte 0x80 | type << 4 | count) the packed leaf item.
-NE_DEV uint32_t child_item(uint32_t ref, uint32_t meta, int c) {
-  const uint32_t m = (meta >> (8 * c)) & 0xFFu;
-  if (!(m & 0x80u)) return ref;
-  return kItemLeaf | (((m >> 4) & 3u) << 29) | (((m & 15u) - 1u) << kItemCountShift) | ref;
 }
 
 template <typename R>
@@ -243,7 +238,9 @@ template <typename R>
 NE_DEV bool trav_pop(TravState<R>& st, const uint32_t* lds, int lane_stride, const uint32_t* spill) {
   if (st.sp == 0) return true;
   --st.sp;
-  st.cur = st.sp < kShortStack ? lds[st.sp * lane_stride] : spill[st.sp - kShortStack];
+  // two loads, not one through a pointer to either: that would be a flat load
+  st.cur = lds[(st.sp < kShortStack ? st.sp : kShortStack - 1) * lane_stride];
+  if (st.sp >= kShortStack) st.cur = spill[st.sp - kShortStack];
   return false;
 }
 
@@ -287,45 +284,39 @@ NE_DEV bool trav_prim(const DevScene& s, TravState<R>& st, uint32_t it, uint32_t
 // (no child hit and the stack is empty).  Closest-hit queries go nearest child
 // first; any-hit queries only move the nearest hit child to the front (one
 // pass of three exchanges): any occluder ends the query.
+// VALU issue bounds a visit (92% of the time with nodes of bytes, 290
+// instructions); decoded planes read by the ray's octant, ready work items,
+// selects instead of branches and one predicate for the three pushes leave 150
+// (surface1m at 64 spp: 101.3 -> 87.6 ms).  The seven loads go out together,
+// which takes 68 VGPRs in k_wf_trace: held to 64 for an eighth wave the
+// compiler splits them and the frame takes 97 ms.
 template <typename R, bool ANY, bool C>
 NE_DEV bool trav_node(const DevScene& s, TravState<R>& st, uint32_t* lds, int lane_stride, uint32_t* spill,
                       Count<C>& cnt) {
-  const uint32_t it = st.cur;
-  // 4-wide inner node (64 B): decode the four quantized child boxes, test
-  // them, continue with the nearest hit child and push the others farthest
-  // first (entry distances sorted by a five-exchange network; misses sort
-  // last at +inf)
-  const float4* nd = s.nodes + 4 * size_t(it);
-  const float4 f0 = nd[0];
-  const uint4 f1 = reinterpret_cast<const uint4*>(nd)[1], f2 = reinterpret_cast<const uint4*>(nd)[2];
-  const int4 ch = reinterpret_cast<const int4*>(nd)[3];
+  // 4-wide inner node (128 B): test the four child boxes, continue with the
+  // nearest hit child and push the others farthest first (entry distances
+  // sorted by a five-exchange network; misses sort last at +inf)
+  const char* nd = reinterpret_cast<const char*>(s.nodes) + (size_t(st.cur) << 7);
+  auto planes = [nd](uint32_t off) { return *reinterpret_cast<const float4*>(nd + off); };
+  const float4 ax = planes(st.nx), bx = planes(st.nx ^ 16u);
+  const float4 ay = planes(32u + st.ny), by = planes(32u + (st.ny ^ 16u));
+  const float4 az = planes(64u + st.nz), bz = planes(64u + (st.nz ^ 16u));
+  const uint4 ch = *reinterpret_cast<const uint4*>(nd + 96);
   cnt.node();
-  const uint32_t ex = __float_as_uint(f0.w);
-  const float sx = __uint_as_float((ex & 0xFFu) << 23), sy = __uint_as_float(((ex >> 8) & 0xFFu) << 23),
-              sz = __uint_as_float(((ex >> 16) & 0xFFu) << 23);
   const R inf = xinf<R>();
-  R t0 = inf, t1 = inf, t2 = inf, t3 = inf, te;
-#define NE_CHILD_SLAB(c, ref, tout)                                                                           \
-  if ((ref) >= 0 &&                                                                                         \
-      slab<R>(__builtin_fmaf(qbyte(f1.x, c), sx, f0.x), __builtin_fmaf(qbyte(f1.y, c), sy, f0.y),             \
-              __builtin_fmaf(qbyte(f1.z, c), sz, f0.z), __builtin_fmaf(qbyte(f1.w, c), sx, f0.x),             \
-              __builtin_fmaf(qbyte(f2.x, c), sy, f0.y), __builtin_fmaf(qbyte(f2.y, c), sz, f0.z), st.o,       \
-              st.invd, st.best, te))                                                                        \
-    tout = te;
-  NE_CHILD_SLAB(0, ch.x, t0)
-  NE_CHILD_SLAB(1, ch.y, t1)
-  NE_CHILD_SLAB(2, ch.z, t2)
-  NE_CHILD_SLAB(3, ch.w, t3)
-#undef NE_CHILD_SLAB
-  uint32_t i0 = child_item(uint32_t(ch.x), f2.z, 0);
-  uint32_t i1 = child_item(uint32_t(ch.y), f2.z, 1);
-  uint32_t i2 = child_item(uint32_t(ch.z), f2.z, 2);
-  uint32_t i3 = child_item(uint32_t(ch.w), f2.z, 3);
+  auto entry = [&](uint32_t item, float px, float py, float pz, float qx, float qy, float qz) {
+    R te;
+    const bool hit = slab<R>(px, py, pz, qx, qy, qz, st.o, st.invd, st.best, te);
+    return (hit & (item != kItemNone)) ? te : inf;
+  };
+  R t0 = entry(ch.x, ax.x, ay.x, az.x, bx.x, by.x, bz.x), t1 = entry(ch.y, ax.y, ay.y, az.y, bx.y, by.y, bz.y);
+  R t2 = entry(ch.z, ax.z, ay.z, az.z, bx.z, by.z, bz.z), t3 = entry(ch.w, ax.w, ay.w, az.w, bx.w, by.w, bz.w);
+  uint32_t i0 = ch.x, i1 = ch.y, i2 = ch.z, i3 = ch.w;
   auto order = [](R& ta, uint32_t& ia, R& tb, uint32_t& ib) {
-    if (tb < ta) {
-      const R t = ta; ta = tb; tb = t;
-      const uint32_t i = ia; ia = ib; ib = i;
-    }
+    const bool swap = tb < ta;
+    const R lo = swap ? tb : ta, hi = swap ? ta : tb;
+    const uint32_t il = swap ? ib : ia, ih = swap ? ia : ib;
+    ta = lo; tb = hi; ia = il; ib = ih;
   };
   if constexpr (ANY) {
     order(t2, i2, t3, i3);
@@ -339,9 +330,22 @@ NE_DEV bool trav_node(const DevScene& s, TravState<R>& st, uint32_t* lds, int la
     order(t1, i1, t2, i2);
   }
   if (!(t0 < inf)) return trav_pop(st, lds, lane_stride, spill);
-  if (t3 < inf) trav_push(st, i3, lds, lane_stride, spill);
-  if (t2 < inf) trav_push(st, i2, lds, lane_stride, spill);
-  if (t1 < inf) trav_push(st, i1, lds, lane_stride, spill);
+  const bool h1 = t1 < inf, h2 = t2 < inf, h3 = t3 < inf;
+  if (st.sp + 3 <= kShortStack) {
+    // every slot is written, and one that holds a miss is written over by the
+    // next push: no branch per child
+    uint32_t* top = lds + st.sp * lane_stride;
+    top[0] = i3;
+    top += h3 ? lane_stride : 0;
+    top[0] = i2;
+    top += h2 ? lane_stride : 0;
+    top[0] = i1;
+    st.sp += int(h1) + int(h2) + int(h3);
+  } else {
+    if (h3) trav_push(st, i3, lds, lane_stride, spill);
+    if (h2) trav_push(st, i2, lds, lane_stride, spill);
+    if (h1) trav_push(st, i1, lds, lane_stride, spill);
+  }
   st.cur = i0;
   return false;
 }
