@@ -874,14 +874,16 @@ ne_status ne_film_tonemap(ne_film* f, int32_t spp, float* pixels) {
 constexpr size_t kMaxSampleBuffer = size_t(16) << 30;
 
 // Default wavefront pool (slots) for a render of `total` paths, measured on
-// MI355X: 2^23 for surface-only scenes, where fewer, larger BVH launches
-// amortise each launch's tail; with a volume 2^22, where a larger pool adds
+// MI355X.  Surface-only scenes: fewer, larger BVH launches amortise each
+// launch's tail, 2^24 slots for renders of 2^25 paths and more, else 2^23
+// (surface1m, ms at 2^23 / 2^24 slots: 16 spp 25.0 / 25.8, 32 spp 45.3 / 44.3,
+// 64 spp 84.5 / 81.0).  With a volume 2^22, where a larger pool adds
 // cache pressure, except for long renders (2^28 paths and more, e.g. the
 // 1920x1080 cloud at 256 spp), whose iterations' fixed costs (launches, the
 // plan scan) halve with 2^23 slots: 236.4 -> 231.5 ms per cloud frame, while
 // a 512^2 x 64-spp volume frame took 12.0 ms at 2^22 and 13.4 ms at 2^23.
 static uint64_t default_pool(const DevScene& ds, uint64_t total) {
-  if (ds.n_nodes > 0 && !ds.has_volume) return uint64_t(1) << 23;
+  if (ds.n_nodes > 0 && !ds.has_volume) return uint64_t(1) << (total >= (uint64_t(1) << 25) ? 24 : 23);
   return total >= (uint64_t(1) << 28) ? (uint64_t(1) << 23) : (uint64_t(1) << 22);
 }
 
@@ -942,8 +944,7 @@ static ne_status render_wavefront(ne_ctx* c, const ne_scene* s, const DevCamera&
     NE_HIP(c, wf_refill_blocks_per_cu(&per_cu));
     c->refill_blocks = uint32_t(std::max(1, cus * std::max(1, per_cu)));
   }
-  // chunks per refill block: one round of resident blocks covers the pool
-  a.refill = std::min<uint32_t>(kMaxRefill, std::max<uint32_t>(1, (a.nchunks + c->refill_blocks - 1) / c->refill_blocks));
+  a.refill_blocks = c->refill_blocks;
   a.total_paths = total;
   a.counters = c->d_counters;
   a.film_fixed = f->d_fixed;
@@ -1615,7 +1616,7 @@ hipError_t lane_render(ne_batch* b, BatchLane& L, size_t j, int div, uint32_t re
   a.seed = J.seed;
   a.sort = 0;
   a.refill_min = kRefillMinIdle;
-  a.refill = std::min<uint32_t>(kMaxRefill, std::max<uint32_t>(1, (a.nchunks + refill_blocks - 1) / refill_blocks));
+  a.refill_blocks = refill_blocks;
   a.total_paths = total;
   a.counters = nullptr;
   a.film_fixed = b->d_films + b->film_off[j];

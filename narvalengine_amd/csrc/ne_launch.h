@@ -58,10 +58,8 @@ hipError_t launch_render(const DevScene& s, const DevCamera& cam, const RenderAr
 // The path pool is split into chunks of kChunk slots; stage kernels run one
 // block of kChunk threads per chunk and keep each chunk's live paths packed.
 constexpr uint32_t kChunk = 256;
-constexpr uint32_t kMaxRefill = 64;  // chunks per block in the lane-refill kernels
 // Idle lanes a wave waits for before it refills.  Measured on MI355X with
-// surface1m (ms per frame): 1: 444, 8: 427, 16: 421, 24: 416, 32: 417,
-// 48: 459, 64: 771.
+// surface1m at 64 spp (ms per frame): 16: 84.9, 24: 84.5, 32: 85.1.
 constexpr int kRefillMinIdle = 24;
 // stage ids (the public NE_STAGE_* values)
 enum { kStageMegakernel = 0, kStagePlan, kStageRegen, kStageTrace, kStageMedium, kStageShade, kStageShadow,
@@ -130,7 +128,7 @@ struct WfArgs {
   int32_t W, H, x0, y0, x1, y1;
   int32_t max_bounces;
   uint32_t sample_offset, job, nchunks;
-  uint32_t refill;  // chunks per block of the lane-refill kernels, 1..kMaxRefill
+  uint32_t refill_blocks;  // resident blocks of the lane-refill kernels
   uint64_t seed;
   unsigned long long total_paths;
   int32_t cur;

@@ -287,90 +287,98 @@ __global__ __launch_bounds__(kChunk) void k_wf_regen(WfState w, WfArgs a, DevCam
 // ---- lane refill -------------------------------------------------------------
 // Traversal lengths are heavy-tailed (rays grazing dense geometry visit many
 // nodes), so a wave that holds one ray per lane waits for its slowest lane.
-// The BVH kernels below give each 256-thread block a pool of a.refill chunks
-// (sized on the host so the grid is one round of resident blocks) and run one
-// flattened loop: every iteration, lanes without a ray take the next one from
-// the pool (one LDS atomic per wave) and every lane with a ray does one node
-// visit.  A lane leaves the loop only when the pool is empty.
-
-// Per-block pool over the chunks blockIdx.x + j * gridDim.x (j < n): chunks
-// map to image regions, so interleaving spreads expensive regions over all
-// blocks.  Items are numbered chunk by chunk, pre[j] = first item of chunk j,
-// pre[n] = total.
-struct RefillPool {
-  uint32_t pre[kMaxRefill + 1];
-  uint32_t n, next;
+// The BVH kernels below run one round of resident waves in one flattened loop:
+// lanes without a ray take the next ones of the wave's unit, every lane with a
+// ray does one node visit.
+//
+// A unit is 64 slots of a chunk; its chunk's four units go to the four waves of
+// a block, the chunks blockIdx.x + round * gridDim.x to one block (chunks map to
+// image regions, so interleaving spreads expensive regions over all blocks).
+// The block's waves take its units in turn from an LDS counter, so a wave holds
+// one unit at a time, in registers, and a refill is a rank in a ballot: against
+// a block-wide queue of single rays, and finished rays stored one by one as they
+// ended, surface1m at 64 spp takes 84.5 instead of 88.0 ms and a 640 x 360
+// preview 2.47 instead of 2.63.  Units shared by all blocks through global
+// counters gained nothing more: a device-wide atomic is slower than what an
+// even split of so many units loses (86.3 ms with a quarter of them shared).
+struct UnitQueue {
+  uint32_t* next;     // the block's next unit (LDS)
+  uint32_t nchunks;
+  uint32_t cur, end;  // slots left of the current unit
 };
-
-__device__ __forceinline__ uint32_t pool_chunk(uint32_t j) { return blockIdx.x + j * gridDim.x; }
-
-__device__ __forceinline__ void pool_init(RefillPool& p, const uint32_t* cnt, uint32_t nchunks) {
-  if (threadIdx.x == 0) {
-    uint32_t n = 0, acc = 0;
-    while (n < kMaxRefill && pool_chunk(n) < nchunks) {
-      p.pre[n] = acc;
-      acc += cnt[pool_chunk(n)];
-      ++n;
-    }
-    p.pre[n] = acc;
-    p.n = n;
-    p.next = 0;
-  }
+constexpr uint32_t kUnits = kChunk / 64;  // per chunk
+__device__ __forceinline__ uint32_t uniform(uint32_t v) { return uint32_t(__builtin_amdgcn_readfirstlane(int(v))); }
+__device__ __forceinline__ void units_init(UnitQueue& q, uint32_t* next, uint32_t nchunks) {
+  if (threadIdx.x == 0) *next = 0u;
+  q.next = next;
+  q.nchunks = nchunks;
+  q.cur = q.end = 0;
   __syncthreads();
 }
-
-// Lanes with need == true take consecutive items (wave-aggregated LDS atomic).
-// Returns the slot (chunk * kChunk + position) or kNoHit when the pool is empty.
-// Every lane still in the caller's loop must call it.
-__device__ __forceinline__ uint32_t pool_fetch(RefillPool& p, bool need) {
-  const unsigned long long m = __ballot(need);
-  if (m == 0) return kNoHit;
-  const int lane = __lane_id();
-  const int leader = __ffsll((long long)m) - 1;
-  uint32_t base = 0;
-  if (lane == leader) base = atomicAdd(&p.next, uint32_t(__popcll(m)));
-  base = __shfl(base, leader);
-  if (!need) return kNoHit;
-  const uint32_t k = base + uint32_t(__popcll(m & ((1ull << lane) - 1ull)));
-  const uint32_t n = p.n;
-  if (k >= p.pre[n]) return kNoHit;
-  // largest j < n with pre[j] <= k (pre is non-decreasing, pre[0] = 0)
-  uint32_t lo = 0, hi = n - 1;
-  while (lo < hi) {
-    const uint32_t mid = (lo + hi + 1) >> 1;
-    if (p.pre[mid] <= k) lo = mid; else hi = mid - 1;
+// Next unit that holds rays (cnt: rays per chunk) into q.cur, q.end; false when
+// the block has none left.  The whole wave calls it.
+__device__ __forceinline__ bool units_next(UnitQueue& q, const uint32_t* cnt) {
+  while (true) {
+    uint32_t u = 0;
+    if (__lane_id() == 0) u = atomicAdd(q.next, 1u);
+    u = uniform(u);
+    const uint32_t c = blockIdx.x + u / kUnits * gridDim.x, lo = u % kUnits * 64;
+    if (c >= q.nchunks) return false;
+    const uint32_t n = uniform(cnt[c]);
+    if (n > lo) {
+      q.cur = c * kChunk + lo;
+      q.end = c * kChunk + (n < lo + 64 ? n : lo + 64);
+      return true;
+    }
   }
-  return pool_chunk(lo) * kChunk + (k - p.pre[lo]);
+}
+// Slots for the lanes with need == true from the current unit (or the next);
+// kNoHit for the lanes that it does not reach.  none: nothing is left.
+__device__ __forceinline__ uint32_t units_fetch(UnitQueue& q, const uint32_t* cnt, bool need, bool& none) {
+  if (q.cur == q.end && !units_next(q, cnt)) {
+    none = true;
+    return kNoHit;
+  }
+  const unsigned long long m = __ballot(need);
+  const uint32_t k = q.cur + uint32_t(__popcll(m & ((1ull << __lane_id()) - 1ull)));
+  const uint32_t got = need && k < q.end ? k : kNoHit;
+  const uint32_t take = uint32_t(__popcll(m)), left = q.end - q.cur;
+  q.cur += take < left ? take : left;
+  return got;
 }
 
-// Refill vote of the lanes still in a refill loop: true (on every such lane)
-// once at least `min_idle` of them, or all of them, have no ray.  Idle lanes
-// wait in between, so the refill path runs on fewer steps.
-__device__ __forceinline__ bool refill_due(bool have, int min_idle) {
-  const unsigned long long idle = __ballot(!have), looping = __ballot(true);
-  return idle != 0ull && (__popcll(idle) >= min_idle || idle == looping);
-}
+// Refill vote: true once at least `min_idle` of the wave's lanes, or all of
+// them, have no ray.  Idle lanes wait in between, so the refill path runs on
+// fewer steps, and so do the finished rays' stores, which are made there.
+__device__ __forceinline__ bool refill_due(bool have, int min_idle) { return __popcll(__ballot(!have)) >= min_idle; }
 
 // Closest surface hit of every live ray: pure BVH traversal (no random
-// numbers), lane refill over the block's pool.
+// numbers), lane refill.
 template <bool C>
 __global__ __launch_bounds__(kChunk) void k_wf_trace(WfState w, WfArgs a, DevScene s) {
   __shared__ uint32_t lds_stack[kShortStack * kChunk];
   __shared__ uint32_t red[kChunk / 64];
-  __shared__ RefillPool pool;
   const WfPaths A = w.paths[a.cur];
-  pool_init(pool, w.cnt_paths[a.cur], a.nchunks);
+  __shared__ uint32_t next;
+  UnitQueue q;
+  units_init(q, &next, a.nchunks);
   uint32_t* stk = lds_stack + threadIdx.x;
   uint32_t spill[kSpillStack];
   Count<C> cnt;
   TravState<float> st;
   uint32_t slot = kNoHit;
-  bool have = false;
+  bool have = false, none = false;
   while (true) {
-    if (refill_due(have, a.refill_min)) {
-      const uint32_t got = pool_fetch(pool, !have);  // every lane still looping calls it
-      if (!have) {
-        if (got == kNoHit) break;
+    if (refill_due(have, none ? 64 : a.refill_min)) {
+      if (!have && slot != kNoHit) {
+        A.hit_t[slot] = st.found ? st.best : xinf<float>();
+        A.hit_ref[slot] = st.found ? ((uint32_t(st.btype) << 30) | st.bslot) : kNoHit;
+        A.kind[slot] = st.found ? uint32_t(WF_KIND_SURFACE) : uint32_t(WF_KIND_MISS);
+        slot = kNoHit;
+      }
+      if (none) break;
+      const uint32_t got = units_fetch(q, w.cnt_paths[a.cur], !have, none);
+      if (got != kNoHit) {
         slot = got;
         have = true;
         cnt.ext();
@@ -378,12 +386,7 @@ __global__ __launch_bounds__(kChunk) void k_wf_trace(WfState w, WfArgs a, DevSce
                   xinf<float>());
       }
     }
-    if (have && trav_step_wave<float, false, C>(s, st, stk, kChunk, spill, cnt)) {
-      A.hit_t[slot] = st.found ? st.best : xinf<float>();
-      A.hit_ref[slot] = st.found ? ((uint32_t(st.btype) << 30) | st.bslot) : kNoHit;
-      A.kind[slot] = st.found ? uint32_t(WF_KIND_SURFACE) : uint32_t(WF_KIND_MISS);
-      have = false;
-    }
+    if (have && trav_step_wave<float, false, C>(s, st, stk, kChunk, spill, cnt)) have = false;
   }
   if constexpr (C) {
     block_count<C>(&a.counters->ext_rays, cnt.n_ext, red);
@@ -923,49 +926,53 @@ __device__ __forceinline__ void shadow_deliver(const WfShadow& S, const WfPaths&
   }
 }
 
-// Shadow rays of scenes without a volume: any-hit BVH occlusion with lane
-// refill over the block's pool of shadow-queue chunks, then delivery of the
-// unoccluded rays' contributions.
-template <bool C>
-__global__ __launch_bounds__(kChunk) void k_wf_shadow_surf(WfState w, WfArgs a, DevScene s) {
+// Shadow rays against the surfaces: any-hit BVH occlusion with lane refill.
+// Occluded rays are marked (tmax = -1) for the stage that delivers the others:
+// out of the refill loop, where a finishing lane would hold its whole wave.
+// FULL: the queue's layout (WfArgs::shadow_full).
+template <bool C, bool FULL>
+__global__ __launch_bounds__(kChunk) void k_wf_occlude(WfState w, WfArgs a, DevScene s) {
   __shared__ uint32_t lds_stack[kShortStack * kChunk];
   __shared__ uint32_t red[kChunk / 64];
-  __shared__ RefillPool pool;
   const WfShadow S = w.shadow;
   const WfPaths B = w.paths[a.cur ^ 1];
-  pool_init(pool, w.cnt_shadow, a.nchunks);
+  __shared__ uint32_t next;
+  UnitQueue q;
+  units_init(q, &next, a.nchunks);
   uint32_t* stk = lds_stack + threadIdx.x;
   uint32_t spill[kSpillStack];
   Count<C> cnt;
   TravState<float> st;
   uint32_t k = kNoHit;
-  bool have = false;
+  bool have = false, none = false;
   while (true) {
-    if (refill_due(have, a.refill_min)) {
-      const uint32_t got = pool_fetch(pool, !have);  // every lane still looping calls it
-      if (!have) {
-        if (got == kNoHit) break;
-        k = got;
-        have = true;
-        cnt.shadow();
-        trav_init(st, v3(S.ox[k], S.oy[k], S.oz[k]), v3(S.dx[k], S.dy[k], S.dz[k]), 1e-4f, S.tmax[k]);
+    if (refill_due(have, none ? 64 : a.refill_min)) {
+      if (!have && k != kNoHit) {
+        if (st.found) S.tmax[k] = -1.0f;
+        k = kNoHit;
+      }
+      if (none) break;
+      const uint32_t got = units_fetch(q, w.cnt_shadow, !have, none);
+      if (got != kNoHit) {
+        Vec3<float> x;
+        bool hole = false;
+        if constexpr (FULL) {
+          x = v3(S.ox[got], S.oy[got], S.oz[got]);
+        } else {
+          const bool own = got % kChunk < w.cnt_paths[a.cur ^ 1][got / kChunk];
+          uint32_t pix, smp, vert;
+          shadow_source(S, B, got, own, x, pix, smp, vert);
+          hole = own && !(S.pl[got] > 0.0f);
+        }
+        if (!hole) {
+          k = got;
+          have = true;
+          cnt.shadow();
+          trav_init(st, x, v3(S.dx[k], S.dy[k], S.dz[k]), 1e-4f, S.tmax[k]);
+        }
       }
     }
-    if (have && trav_step_wave<float, true, C>(s, st, stk, kChunk, spill, cnt)) {
-      if (st.found) S.tmax[k] = -1.0f;  // occluded: marked for the delivery pass
-      have = false;
-    }
-  }
-  // Delivery pass over the block's chunks, one queue entry per thread in
-  // order: coalesced, and out of the refill loop, where a finishing lane
-  // would hold its whole wave through the delivery.
-  __syncthreads();
-  for (uint32_t j = 0; j < pool.n; ++j) {
-    const uint32_t ch = pool_chunk(j), n = pool.pre[j + 1] - pool.pre[j];
-    for (uint32_t t = threadIdx.x; t < n; t += kChunk) {
-      const uint32_t q = ch * kChunk + t;
-      if (S.tmax[q] >= 0.0f) shadow_deliver(S, B, a, s, q, 1.0f);
-    }
+    if (have && trav_step_wave<float, true, C>(s, st, stk, kChunk, spill, cnt)) have = false;
   }
   if constexpr (C) {
     block_count<C>(&a.counters->shadow_rays, cnt.n_shadow, red);
@@ -974,16 +981,30 @@ __global__ __launch_bounds__(kChunk) void k_wf_shadow_surf(WfState w, WfArgs a, 
   }
 }
 
-// Shadow rays: any-hit occlusion (HAS_SURF) then ratio tracking (HAS_VOL),
-// the megakernel's transmittance() split by scene content.
+// Scenes without a volume: the contributions of the rays that k_wf_occlude left
+// unoccluded, one queue entry per thread in order (coalesced).
+// C: count the rays (scenes without surfaces, where no other stage does).
+template <bool C>
+__global__ __launch_bounds__(kChunk) void k_wf_deliver(WfState w, WfArgs a, DevScene s) {
+  const uint32_t n = w.cnt_shadow[blockIdx.x], q = blockIdx.x * kChunk + threadIdx.x;
+  if (threadIdx.x < n && w.shadow.tmax[q] >= 0.0f) shadow_deliver(w.shadow, w.paths[a.cur ^ 1], a, s, q, 1.0f);
+  if (C && threadIdx.x == 0 && n) atomicAdd(&a.counters->shadow_rays, (unsigned long long)n);
+}
+
+// Shadow rays through the volume: ratio tracking, the megakernel's
+// transmittance() after its occlusion test.
+// HAS_SURF: k_wf_occlude has marked the occluded rays.  The rays that are left
+// and cross the volume are packed first, so that waves track whole: both in one
+// thread per ray ran 11% of the lanes (a room with a volume, 857 x 481 at 32
+// spp: 13.2 ms a frame; 8.0 ms in two stages, the frame 28.1 -> 23.0 ms).
 // SPATIAL: the chunk's shadow rays are taken in Morton order of their origins
 // (each keeps its own stream: same transmittances).
 // GRID: how density lookups read the grid (kGrid*).
-template <bool C, bool HAS_SURF, bool HAS_VOL, bool SPATIAL, int GRID>
+template <bool C, bool HAS_SURF, bool SPATIAL, int GRID>
 __global__ __launch_bounds__(kChunk) void k_wf_shadow(WfState w, WfArgs a, DevScene s) {
-  __shared__ uint32_t lds_stack[HAS_SURF ? kShortStack * kChunk : 1];
   __shared__ uint32_t red[kChunk / 64];
   __shared__ uint32_t skey[SPATIAL ? kChunk : 1];
+  __shared__ uint32_t list[HAS_SURF ? kChunk : 1];
   const WfShadow S = w.shadow;
   const WfPaths B = w.paths[a.cur ^ 1];
   const uint32_t c = blockIdx.x, t = threadIdx.x;
@@ -997,6 +1018,26 @@ __global__ __launch_bounds__(kChunk) void k_wf_shadow(WfState w, WfArgs a, DevSc
                                     : v3s(0.0f),
                               skey);
   }
+  uint32_t nt = n;  // threads that take a ray
+  if constexpr (HAS_SURF) {
+    const uint32_t k = c * kChunk + slot;
+    const bool own = slot < nc;
+    bool track = false;
+    if (t < n && (!own || S.pl[k] > 0.0f) && !(S.tmax[k] < 0.0f)) {  // holes and occluded rays skipped
+      Vec3<float> x;
+      uint32_t spix, ssmp, svert;
+      shadow_source(S, B, k, own, x, spix, ssmp, svert);
+      const Vec3<float> wi = v3(S.dx[k], S.dy[k], S.dz[k]);
+      float ta, tb;
+      track = box_interval<float>(s, xf_point<float>(s.inv, x), xf_vec<float>(s.inv, wi), ta, tb) &&
+              xmax(ta, 0.0f) < xmin(tb, S.tmax[k]);
+      if (!track) shadow_deliver(S, B, a, s, k, 1.0f, own);
+    }
+    const uint32_t at = block_compact(track, red, nt);
+    if (track) list[at] = slot;
+    __syncthreads();
+    if (t < nt) slot = list[t];
+  }
   const uint32_t k = c * kChunk + slot;
   const bool own = slot < nc;
   Count<C> cnt;
@@ -1007,7 +1048,7 @@ __global__ __launch_bounds__(kChunk) void k_wf_shadow(WfState w, WfArgs a, DevSc
   // record and path record exist, so the loads stay in bounds); the empty
   // asm takes the values here, so the loads are not sunk past the test into
   // one round trip each
-  if (t < n) {
+  if (t < nt) {
     shadow_source(S, B, k, own, x, spix, ssmp, svert);
     wi = v3(S.dx[k], S.dy[k], S.dz[k]);
     tmax = S.tmax[k];
@@ -1015,33 +1056,25 @@ __global__ __launch_bounds__(kChunk) void k_wf_shadow(WfState w, WfArgs a, DevSc
     asm volatile("" ::"v"(x.x), "v"(x.y), "v"(x.z), "v"(spix), "v"(ssmp), "v"(svert), "v"(wi.x), "v"(wi.y),
                  "v"(wi.z), "v"(tmax), "v"(pl));
   }
-  if (t < n && (!own || pl > 0.0f)) {  // holes skipped
+  if (t < nt && (!own || pl > 0.0f)) {  // holes skipped
     PathRng rng;
     rng.init(a.seed, spix, ssmp, a.job);
     PathRng srng = rng.shadow_stream(int(svert));
-    cnt.shadow();
+    if (!HAS_SURF) cnt.shadow();
     float tr = 1.0f;
-    if (HAS_SURF) {
-      SurfHit<float> h;
-      if (traverse<float, true, C>(s, x, wi, 1e-4f, tmax, lds_stack + t, kChunk, h, cnt)) tr = 0.0f;
-    }
-    if (HAS_VOL && tr > 0.0f) {
-      const Vec3<float> oo = xf_point<float>(s.inv, x), dd = xf_vec<float>(s.inv, wi);
-      float ta, tb;
-      if (box_interval<float>(s, oo, dd, ta, tb)) {
-        ta = xmax(ta, 0.0f);
-        tb = xmin(tb, tmax);
-        if (ta < tb) tr = ratio_track<float, C, GRID>(s, x, wi, ta, tb, srng, cnt);
-      }
+    const Vec3<float> oo = xf_point<float>(s.inv, x), dd = xf_vec<float>(s.inv, wi);
+    float ta, tb;
+    if (box_interval<float>(s, oo, dd, ta, tb)) {
+      ta = xmax(ta, 0.0f);
+      tb = xmin(tb, tmax);
+      if (ta < tb) tr = ratio_track<float, C, GRID>(s, x, wi, ta, tb, srng, cnt);
     }
     if (tr > 0.0f) shadow_deliver(S, B, a, s, k, tr, own);
   }
   if constexpr (C) {
-    block_count<C>(&a.counters->shadow_rays, cnt.n_shadow, red);
+    if (!HAS_SURF) block_count<C>(&a.counters->shadow_rays, cnt.n_shadow, red);
     block_count<C>(&a.counters->sh_lookups, cnt.n_lookup, red);
     block_count<C>(&a.counters->sh_cells, cnt.n_cell, red);
-    block_count<C>(&a.counters->sh_nodes, cnt.n_node, red);
-    block_count<C>(&a.counters->sh_prims, cnt.n_prim, red);
   }
 }
 
@@ -1198,7 +1231,7 @@ hipError_t launch_wavefront(const DevScene& s, const DevCamera& cam, WfState& w,
   NE_MARK(kStageOther);
   hipLaunchKernelGGL(k_wf_init, dim3((NC + 255) / 256), dim3(256), 0, st, w, NC);
   const dim3 grid = dim3(NC);
-  const dim3 pgrid = dim3((NC + a.refill - 1) / a.refill);  // lane-refill kernels
+  const dim3 pgrid = dim3(std::min(NC, a.refill_blocks));  // lane-refill kernels: one round of resident blocks
   const dim3 blk = dim3(unsigned(kChunk));
   if (!count) a.counters = nullptr;
   const bool hs = s.n_nodes > 0, hv = s.has_volume != 0;
@@ -1328,31 +1361,42 @@ hipError_t launch_wavefront(const DevScene& s, const DevCamera& cam, WfState& w,
     else if (sort) hipLaunchKernelGGL((k_wf_shade<false, true, false>), grid, blk, 0, st, w, a, s, WfGuide{});
     else hipLaunchKernelGGL((k_wf_shade<false, false, false>), grid, blk, 0, st, w, a, s, WfGuide{});
     if (!fuse) NE_MARK(kStageShadow);
-#define NE_SHADOW_SP(CNT, S_, V_, SM)                                                             \
-  do {                                                                                            \
-    if (spatial) hipLaunchKernelGGL((k_wf_shadow<CNT, S_, V_, true, SM>), grid, blk, 0, st, w, a, s); \
-    else hipLaunchKernelGGL((k_wf_shadow<CNT, S_, V_, false, SM>), grid, blk, 0, st, w, a, s);      \
+#define NE_SHADOW_SP(CNT, S_, SM)                                                                   \
+  do {                                                                                              \
+    if (spatial) hipLaunchKernelGGL((k_wf_shadow<CNT, S_, true, SM>), grid, blk, 0, st, w, a, s);     \
+    else hipLaunchKernelGGL((k_wf_shadow<CNT, S_, false, SM>), grid, blk, 0, st, w, a, s);          \
   } while (0)
-#define NE_SHADOW(CNT, S_, V_)                       \
-  do {                                               \
-    if (V_ && form == kGridQuad) NE_SHADOW_SP(CNT, S_, V_, kGridQuad);        \
-    else if (V_ && form == kGridBrick) NE_SHADOW_SP(CNT, S_, V_, kGridBrick); \
-    else NE_SHADOW_SP(CNT, S_, V_, kGridWide);       \
+#define NE_SHADOW(CNT, S_)                                      \
+  do {                                                          \
+    if (form == kGridQuad) NE_SHADOW_SP(CNT, S_, kGridQuad);        \
+    else if (form == kGridBrick) NE_SHADOW_SP(CNT, S_, kGridBrick); \
+    else NE_SHADOW_SP(CNT, S_, kGridWide);                      \
+  } while (0)
+#define NE_OCCLUDE(FULL)                                                                          \
+  do {                                                                                            \
+    if (count) hipLaunchKernelGGL((k_wf_occlude<true, FULL>), pgrid, blk, 0, st, w, a, s);         \
+    else hipLaunchKernelGGL((k_wf_occlude<false, FULL>), pgrid, blk, 0, st, w, a, s);              \
   } while (0)
     if (fuse) {
       // done in the shading stage
-    } else if (hs && !hv) {
-      if (count) hipLaunchKernelGGL(k_wf_shadow_surf<true>, pgrid, blk, 0, st, w, a, s);
-      else hipLaunchKernelGGL(k_wf_shadow_surf<false>, pgrid, blk, 0, st, w, a, s);
-    } else if (count) {
-      if (hs) NE_SHADOW(true, true, true);
-      else if (hv) NE_SHADOW(true, false, true); else NE_SHADOW(true, false, false);
+    } else if (hs && hv) {
+      NE_OCCLUDE(false);
+      if (count) NE_SHADOW(true, true);
+      else NE_SHADOW(false, true);
+    } else if (hs) {
+      NE_OCCLUDE(true);
+      hipLaunchKernelGGL(k_wf_deliver<false>, grid, blk, 0, st, w, a, s);
+    } else if (hv) {
+      if (count) NE_SHADOW(true, false);
+      else NE_SHADOW(false, false);
+    } else if (count) {  // neither: nothing is in the way
+      hipLaunchKernelGGL(k_wf_deliver<true>, grid, blk, 0, st, w, a, s);
     } else {
-      if (hs) NE_SHADOW(false, true, true);
-      else if (hv) NE_SHADOW(false, false, true); else NE_SHADOW(false, false, false);
+      hipLaunchKernelGGL(k_wf_deliver<false>, grid, blk, 0, st, w, a, s);
     }
 #undef NE_SHADOW
 #undef NE_SHADOW_SP
+#undef NE_OCCLUDE
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
   NE_MARK(kStageOther);
