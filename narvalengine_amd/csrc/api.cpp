@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cfloat>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -51,6 +52,12 @@ struct ne_ctx {
   int cus = 0;                  // compute units of the device
   void* paths_scratch = nullptr;  // the persistent path kernel's (made on its first use)
   double* scratch = nullptr;    // this device's copy of the static scratch array (ne_render_noalloc)
+  // pinned staging for copies between the device and the caller's memory
+  // (dev_read, tmp_in; used under mu): two chunks for reads, then the inputs'
+  char* stage = nullptr;
+  char* stage_dev = nullptr;    // its device address
+  hipEvent_t stage_ev[2] = {nullptr, nullptr};
+  size_t stage_in = 0;          // bytes of the inputs' part that copies in flight may read
 };
 
 struct ne_scene {
@@ -146,7 +153,63 @@ ne_status dev_upload(ne_ctx* c, ne_scene* s, const T* src, size_t count, const T
   return NE_OK;
 }
 
-// scoped device buffers for the parity entry points
+// The caller's memory is pageable, and a copy straight to it costs far more
+// than its bytes: HIP stages or pins it on each call.  Measured on MI355X, us,
+// through pinned memory of ours / straight: 72 rows of 384 B into a frame 8 /
+// 499, 256 KiB out 19 / 114, 4 MiB into fresh pages 82 / 247, 32 KiB in 9 / 20,
+// 256 KiB in 14 / 108.  Inputs of 1 MiB cost the same both ways (51 / 53) and
+// larger ones more (3 MiB: 120 / 105), so those go straight.
+constexpr size_t kStageChunk = size_t(2) << 20, kStageIn = size_t(1) << 20;
+constexpr size_t kLiDirect = size_t(512) << 10;
+
+// Device -> the caller's memory, after what c->stream holds; returns when it is
+// there.  Chunk k + 1 crosses the bus while chunk k is copied out.
+ne_status dev_read(ne_ctx* c, void* dst, const void* src, size_t bytes) {
+  if (!c->stage) {
+    NE_HIP(c, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream));
+    NE_HIP(c, hipStreamSynchronize(c->stream));
+    return NE_OK;
+  }
+  if (bytes <= kStageChunk) {
+    NE_HIP(c, hipMemcpyAsync(c->stage, src, bytes, hipMemcpyDeviceToHost, c->stream));
+    NE_HIP(c, hipStreamSynchronize(c->stream));
+    c->stage_in = 0;
+    std::memcpy(dst, c->stage, bytes);
+    return NE_OK;
+  }
+  auto issue = [&](size_t off) {
+    const size_t k = off / kStageChunk & 1;
+    const hipError_t e = hipMemcpyAsync(c->stage + k * kStageChunk, static_cast<const char*>(src) + off,
+                                        std::min(kStageChunk, bytes - off), hipMemcpyDeviceToHost, c->stream);
+    return e == hipSuccess ? hipEventRecord(c->stage_ev[k], c->stream) : e;
+  };
+  NE_HIP(c, issue(0));
+  for (size_t off = 0; off < bytes; off += kStageChunk) {
+    const size_t k = off / kStageChunk & 1;
+    if (off + kStageChunk < bytes) NE_HIP(c, issue(off + kStageChunk));
+    NE_HIP(c, hipEventSynchronize(c->stage_ev[k]));
+    std::memcpy(static_cast<char*>(dst) + off, c->stage + k * kStageChunk, std::min(kStageChunk, bytes - off));
+  }
+  NE_HIP(c, hipStreamSynchronize(c->stream));
+  c->stage_in = 0;
+  return NE_OK;
+}
+
+// Space for an input of at most kStageIn bytes, or null (no staging, or too
+// large); waits if copies in flight still read the part that it needs.
+char* stage_input(ne_ctx* c, size_t bytes) {
+  if (!c->stage || bytes > kStageIn) return nullptr;
+  bytes = (bytes + 255) & ~size_t(255);
+  if (c->stage_in + bytes > kStageIn) {
+    if (hipStreamSynchronize(c->stream) != hipSuccess) return nullptr;
+    c->stage_in = 0;
+  }
+  char* p = c->stage + 2 * kStageChunk + c->stage_in;
+  c->stage_in += bytes;
+  return p;
+}
+
+// scoped device buffers for the entry points that take host arrays
 struct DevBuf {
   void* p = nullptr;
   ~DevBuf() { if (p) (void)hipFree(p); }
@@ -156,7 +219,9 @@ template <class T>
 ne_status tmp_in(ne_ctx* c, DevBuf& b, const T* src, size_t count) {
   if (count == 0 || src == nullptr) return NE_OK;
   NE_HIP(c, hipMalloc(&b.p, count * sizeof(T)));
-  NE_HIP(c, hipMemcpyAsync(b.p, src, count * sizeof(T), hipMemcpyHostToDevice, c->stream));
+  const void* from = src;
+  if (char* p = stage_input(c, count * sizeof(T))) from = std::memcpy(p, src, count * sizeof(T));
+  NE_HIP(c, hipMemcpyAsync(b.p, from, count * sizeof(T), hipMemcpyHostToDevice, c->stream));
   return NE_OK;
 }
 template <class T>
@@ -166,8 +231,7 @@ ne_status tmp_out(ne_ctx* c, DevBuf& b, size_t count) {
 }
 template <class T>
 ne_status tmp_back(ne_ctx* c, T* dst, const DevBuf& b, size_t count) {
-  NE_HIP(c, hipMemcpyAsync(dst, b.p, count * sizeof(T), hipMemcpyDeviceToHost, c->stream));
-  return NE_OK;
+  return dev_read(c, dst, b.p, count * sizeof(T));
 }
 
 inline float len3(const float* v) { return std::sqrt(v[0] * v[0] + v[1] * v[1] + v[2] * v[2]); }
@@ -457,13 +521,22 @@ ne_status ne_ctx_create(int32_t device, ne_ctx** out) {
       hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess ||
       hipHostMalloc((void**)&c->h_status, 64 * sizeof(uint32_t), hipHostMallocDefault) != hipSuccess ||
       hipEventCreate(&c->ev0) != hipSuccess ||
-      hipEventCreate(&c->ev1) != hipSuccess) {
+      hipEventCreate(&c->ev1) != hipSuccess ||
+      hipEventCreateWithFlags(&c->stage_ev[0], hipEventDisableTiming) != hipSuccess ||
+      hipEventCreateWithFlags(&c->stage_ev[1], hipEventDisableTiming) != hipSuccess) {
     delete c;
     return fail(nullptr, NE_ERR_HIP, "context setup failed");
   }
   if (resolve_scratch(device, &c->scratch) != hipSuccess) {
     ctx_free(c);
     return fail(nullptr, NE_ERR_HIP, "static scratch address lookup failed");
+  }
+  // without it copies go straight to and from the caller's memory
+  if (hipHostMalloc((void**)&c->stage, 2 * kStageChunk + kStageIn, hipHostMallocDefault) != hipSuccess ||
+      hipHostGetDevicePointer((void**)&c->stage_dev, c->stage, 0) != hipSuccess) {
+    (void)hipGetLastError();
+    if (c->stage) (void)hipHostFree(c->stage);
+    c->stage = nullptr;
   }
   *out = c;
   return NE_OK;
@@ -477,6 +550,9 @@ static void ctx_free(ne_ctx* c) {
   if (c->paths_scratch) (void)hipFree(c->paths_scratch);
   if (c->wf_buf) (void)hipFree(c->wf_buf);
   if (c->h_status) (void)hipHostFree(c->h_status);
+  if (c->stage) (void)hipHostFree(c->stage);
+  for (hipEvent_t e : c->stage_ev)
+    if (e) (void)hipEventDestroy(e);
   for (hipEvent_t e : c->ev_pool) (void)hipEventDestroy(e);
   if (c->wfg_buf) (void)hipFree(c->wfg_buf);
   if (c->sbuf) (void)hipFree(c->sbuf);
@@ -850,9 +926,7 @@ ne_status ne_film_read(ne_film* f, double* sum) {
   ne_ctx* c = f->ctx;
   std::lock_guard<std::mutex> lk(c->mu);
   NE_HIP(c, hipSetDevice(c->device));
-  NE_HIP(c, hipMemcpyAsync(sum, f->d_sum, size_t(f->W) * f->H * 3 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  NE_HIP(c, hipStreamSynchronize(c->stream));
-  return NE_OK;
+  return dev_read(c, sum, f->d_sum, size_t(f->W) * f->H * 3 * sizeof(double));
 }
 
 ne_status ne_film_tonemap(ne_film* f, int32_t spp, float* pixels) {
@@ -865,10 +939,7 @@ ne_status ne_film_tonemap(ne_film* f, int32_t spp, float* pixels) {
   ne_status st = tmp_out<float>(c, b, size_t(npix) * 3);
   if (st != NE_OK) return st;
   NE_HIP(c, launch_tonemap(f->d_sum, npix, 1.0f / float(spp), static_cast<float*>(b.p), c->stream));
-  st = tmp_back(c, pixels, b, size_t(npix) * 3);
-  if (st != NE_OK) return st;
-  NE_HIP(c, hipStreamSynchronize(c->stream));
-  return NE_OK;
+  return tmp_back(c, pixels, b, size_t(npix) * 3);
 }
 
 constexpr size_t kMaxSampleBuffer = size_t(16) << 30;
@@ -1184,16 +1255,17 @@ ne_status ne_render_tile(ne_ctx* c, const ne_scene* s, const ne_camera_desc* cam
   NE_HIP(c, launch_clear_rect(f->d_sum, f->W, q.x0, q.y0, q.x1, q.y1, c->stream));
   st = render_locked(c, s, cam, &q, f);
   if (st != NE_OK) return st;
-  // post-process the tile only, then one strided copy into the caller's
-  // full-frame pixel array
+  // post-process the tile only, one contiguous read, then its rows into the
+  // caller's full-frame pixel array
   DevBuf b;
   if ((st = tmp_out<float>(c, b, size_t(tw) * th * 3)) != NE_OK) return st;
   NE_HIP(c, launch_tonemap_rect(f->d_sum, f->W, q.x0, q.y0, tw, th, 1.0f / float(p->spp), static_cast<float*>(b.p),
                                 c->stream));
-  const size_t row = size_t(tw) * 3 * sizeof(float);
-  NE_HIP(c, hipMemcpy2DAsync(pixels + (size_t(q.y0) * f->W + q.x0) * 3, size_t(f->W) * 3 * sizeof(float), b.p, row,
-                             row, size_t(th), hipMemcpyDeviceToHost, c->stream));
-  NE_HIP(c, hipStreamSynchronize(c->stream));
+  const size_t row = size_t(tw) * 3;
+  std::vector<float> tile(row * size_t(th));
+  if ((st = tmp_back(c, tile.data(), b, tile.size())) != NE_OK) return st;
+  for (int y = 0; y < th; ++y)
+    std::copy_n(&tile[row * size_t(y)], row, pixels + (size_t(q.y0 + y) * f->W + q.x0) * 3);
   return NE_OK;
 }
 
@@ -1259,15 +1331,28 @@ ne_status ne_li(ne_ctx* c, const ne_scene* s, int32_t n, const float* rays, int3
   if (n == 0) return NE_OK;
   std::lock_guard<std::mutex> lk(c->mu);
   NE_HIP(c, hipSetDevice(c->device));
+  // calls that fit in the staging: the kernel reads and writes it itself, with
+  // no copies to wait for (us, direct / through staging and copies / straight:
+  // 1 ray 35 / 40 / 47, 1000 rays 291 / 317 / 328, 12000 rays 356 / 377 / 377)
+  const size_t rb = size_t(n) * 6 * sizeof(float), ob = size_t(n) * 3 * sizeof(float);
+  char* p = rb + ob <= kLiDirect ? stage_input(c, rb + ob) : nullptr;
+  if (p) {
+    char* d = c->stage_dev + (p - c->stage);
+    std::memcpy(p, rays, rb);
+    NE_HIP(c, launch_li(s->dev, n, reinterpret_cast<const float*>(d), max_bounces, seed, sample_index,
+                        reinterpret_cast<float*>(d + rb), c->stream));
+    NE_HIP(c, hipStreamSynchronize(c->stream));
+    c->stage_in = 0;
+    std::memcpy(radiance, p + rb, ob);
+    return NE_OK;
+  }
   DevBuf br, bo;
   ne_status st;
   if ((st = tmp_in(c, br, rays, size_t(n) * 6)) != NE_OK) return st;
   if ((st = tmp_out<float>(c, bo, size_t(n) * 3)) != NE_OK) return st;
   NE_HIP(c, launch_li(s->dev, n, static_cast<const float*>(br.p), max_bounces, seed, sample_index,
                       static_cast<float*>(bo.p), c->stream));
-  if ((st = tmp_back(c, radiance, bo, size_t(n) * 3)) != NE_OK) return st;
-  NE_HIP(c, hipStreamSynchronize(c->stream));
-  return NE_OK;
+  return tmp_back(c, radiance, bo, size_t(n) * 3);
 }
 
 // ---- parity entry points ---------------------------------------------------
@@ -1287,7 +1372,6 @@ ne_status ne_test_primitive(ne_ctx* c, int32_t kind, int32_t n, const float* ray
   NE_HIP(c, launch_test_primitive(kind, n, (const float*)br.p, (const float*)bp.p, (int32_t*)bh.p, (float*)b0.p,
                                   (float*)b1.p, c->stream));
   if ((st = tmp_back(c, hit, bh, n)) || (st = tmp_back(c, t0, b0, n)) || (st = tmp_back(c, t1, b1, n))) return st;
-  NE_HIP(c, hipStreamSynchronize(c->stream));
   return NE_OK;
 }
 
@@ -1306,7 +1390,6 @@ ne_status ne_test_closest(ne_ctx* c, const ne_scene* s, int32_t n, const float* 
   NE_HIP(c, launch_test_closest(s->dev, n, (const float*)br.p, tmin, tmax, (float*)bt.p, (int32_t*)by.p,
                                 (int32_t*)bi.p, c->stream));
   if ((st = tmp_back(c, t, bt, n)) || (st = tmp_back(c, type, by, n)) || (st = tmp_back(c, index, bi, n))) return st;
-  NE_HIP(c, hipStreamSynchronize(c->stream));
   return NE_OK;
 }
 
@@ -1324,7 +1407,6 @@ ne_status ne_test_transmittance(ne_ctx* c, const ne_scene* s, int32_t n, const f
   NE_HIP(c, launch_test_transmittance(s->dev, n, (const float*)br.p, (const float*)bm.p, seed, precision,
                                       (double*)bo.p, c->stream));
   if ((st = tmp_back(c, tr, bo, n))) return st;
-  NE_HIP(c, hipStreamSynchronize(c->stream));
   return NE_OK;
 }
 
@@ -1343,7 +1425,6 @@ ne_status ne_test_delta_track(ne_ctx* c, const ne_scene* s, int32_t n, const flo
   NE_HIP(c, launch_test_delta(s->dev, n, (const float*)br.p, seed, precision, (int32_t*)bs.p, (double*)bt.p,
                               c->stream));
   if ((st = tmp_back(c, scattered, bs, n)) || (st = tmp_back(c, t, bt, n))) return st;
-  NE_HIP(c, hipStreamSynchronize(c->stream));
   return NE_OK;
 }
 
@@ -1359,7 +1440,6 @@ ne_status ne_test_density(ne_ctx* c, const ne_scene* s, int32_t n, const float* 
   if ((st = tmp_in(c, bg, gcs, size_t(n) * 3)) || (st = tmp_out<float>(c, bo, n))) return st;
   NE_HIP(c, launch_test_density(s->dev, n, (const float*)bg.p, (float*)bo.p, c->stream));
   if ((st = tmp_back(c, out, bo, n))) return st;
-  NE_HIP(c, hipStreamSynchronize(c->stream));
   return NE_OK;
 }
 
@@ -1370,9 +1450,7 @@ ne_status ne_test_majorants(ne_ctx* c, const ne_scene* s, float* out, int64_t ca
   if (capacity < n) return fail(c, NE_ERR_INVALID_ARG, "output holds fewer than maj_res^3 floats");
   std::lock_guard<std::mutex> lk(c->mu);
   NE_HIP(c, hipSetDevice(c->device));
-  NE_HIP(c, hipMemcpyAsync(out, s->dev.maj, size_t(n) * sizeof(float), hipMemcpyDeviceToHost, c->stream));
-  NE_HIP(c, hipStreamSynchronize(c->stream));
-  return NE_OK;
+  return dev_read(c, out, s->dev.maj, size_t(n) * sizeof(float));
 }
 
 ne_status ne_test_bsdf(ne_ctx* c, int32_t kind, int32_t n, const float* in0, const float* in1, const float* in2,
@@ -1396,7 +1474,6 @@ ne_status ne_test_bsdf(ne_ctx* c, int32_t kind, int32_t n, const float* in0, con
   NE_HIP(c, launch_test_bsdf(kind, n, (const float*)b[0].p, (const float*)b[1].p, (const float*)b[2].p,
                              (const float*)b[3].p, (float*)bo.p, c->stream));
   if ((st = tmp_back(c, out, bo, size_t(n) * w[kind][4]))) return st;
-  NE_HIP(c, hipStreamSynchronize(c->stream));
   return NE_OK;
 }
 
@@ -1410,7 +1487,6 @@ ne_status ne_test_rng(ne_ctx* c, uint64_t seed, uint32_t pixel, uint32_t sample,
   if ((st = tmp_out<float>(c, bo, n))) return st;
   NE_HIP(c, launch_test_rng(seed, pixel, sample, job, n, (float*)bo.p, c->stream));
   if ((st = tmp_back(c, out, bo, n))) return st;
-  NE_HIP(c, hipStreamSynchronize(c->stream));
   return NE_OK;
 }
 
@@ -1910,7 +1986,6 @@ ne_status ne_batch_read(ne_batch* b, int32_t job, double* sum) {
   if (st != NE_OK) return st;
   NE_HIP(c, launch_fixed_to_double(b->d_films + b->film_off[job], static_cast<double*>(t.p), n, c->stream));
   if ((st = tmp_back(c, sum, t, n)) != NE_OK) return st;
-  NE_HIP(c, hipStreamSynchronize(c->stream));
   return NE_OK;
 }
 
@@ -2047,7 +2122,6 @@ ne_status ne_guide_eval(ne_guide* g, int32_t n, const float* q, int32_t raw, flo
   if (raw) NE_HIP(c, launch_guide_raw(g->net, n, static_cast<float*>(bi.p), static_cast<float*>(bo.p), c->stream));
   else NE_HIP(c, launch_guide_eval(g->net, n, static_cast<float*>(bi.p), static_cast<float*>(bo.p), c->stream));
   if ((st = tmp_back(c, out, bo, size_t(n) * kGuideOutputs)) != NE_OK) return st;
-  NE_HIP(c, hipStreamSynchronize(c->stream));
   return NE_OK;
 }
 
@@ -2055,9 +2129,9 @@ ne_status ne_guide_train_step(ne_guide* g, int32_t n, const float* smp, int32_t 
   if (!g) return fail(nullptr, NE_ERR_INVALID_ARG, "guide is NULL");
   ne_ctx* c = g->ctx;
   if (n < 1 || uint32_t(n) > g->batch.cap || !smp) return fail(c, NE_ERR_INVALID_ARG, "sample count must be in [1, batch]");
-  for (int32_t i = 0; i < n; ++i)
-    if (!(smp[10 * i + 9] >= 0.0f) || !std::isfinite(smp[10 * i + 9]))
-      return fail(c, NE_ERR_INVALID_ARG, "sample weights must be finite and >= 0");
+  bool bad = false;
+  for (size_t i = 0; i < size_t(n); ++i) bad |= !(smp[10 * i + 9] >= 0.0f && smp[10 * i + 9] <= FLT_MAX);
+  if (bad) return fail(c, NE_ERR_INVALID_ARG, "sample weights must be finite and >= 0");
   std::lock_guard<std::mutex> lk(c->mu);
   NE_HIP(c, hipSetDevice(c->device));
   const uint32_t cnt = uint32_t(n);
@@ -2065,8 +2139,8 @@ ne_status ne_guide_train_step(ne_guide* g, int32_t n, const float* smp, int32_t 
   NE_HIP(c, launch_guide_set_batch(g->train.aos, g->batch, cnt, c->stream));
   NE_HIP(c, launch_guide_grad(g->net, g->batch, g->train, cnt, c->stream));
   float lw[2] = {0, 0};
-  NE_HIP(c, hipMemcpyAsync(lw, g->train.loss, sizeof(lw), hipMemcpyDeviceToHost, c->stream));
-  NE_HIP(c, hipStreamSynchronize(c->stream));
+  const ne_status st = dev_read(c, lw, g->train.loss, sizeof(lw));
+  if (st != NE_OK) return st;
   g->last_loss = lw[1] > 0 ? lw[0] / lw[1] : 0.0f;
   if (loss) *loss = g->last_loss;
   g->samples += uint64_t(n);
@@ -2094,9 +2168,10 @@ ne_status ne_guide_get_params(ne_guide* g, float* table, float* mlp) {
   ne_ctx* c = g->ctx;
   std::lock_guard<std::mutex> lk(c->mu);
   NE_HIP(c, hipSetDevice(c->device));
-  if (table) NE_HIP(c, hipMemcpy(table, g->net.table, g->table_n * sizeof(float), hipMemcpyDeviceToHost));
-  if (mlp) NE_HIP(c, hipMemcpy(mlp, g->net.mlp, kGuideParams * sizeof(float), hipMemcpyDeviceToHost));
-  return NE_OK;
+  ne_status st = NE_OK;
+  if (table) st = dev_read(c, table, g->net.table, g->table_n * sizeof(float));
+  if (st == NE_OK && mlp) st = dev_read(c, mlp, g->net.mlp, kGuideParams * sizeof(float));
+  return st;
 }
 
 ne_status ne_guide_set_params(ne_guide* g, const float* table, const float* mlp) {
@@ -2117,9 +2192,10 @@ ne_status ne_guide_get_grads(ne_guide* g, float* table_grad, float* mlp_grad) {
   ne_ctx* c = g->ctx;
   std::lock_guard<std::mutex> lk(c->mu);
   NE_HIP(c, hipSetDevice(c->device));
-  if (table_grad) NE_HIP(c, hipMemcpy(table_grad, g->net.table_grad, g->table_n * sizeof(float), hipMemcpyDeviceToHost));
-  if (mlp_grad) NE_HIP(c, hipMemcpy(mlp_grad, g->net.mlp_grad, kGuideParams * sizeof(float), hipMemcpyDeviceToHost));
-  return NE_OK;
+  ne_status st = NE_OK;
+  if (table_grad) st = dev_read(c, table_grad, g->net.table_grad, g->table_n * sizeof(float));
+  if (st == NE_OK && mlp_grad) st = dev_read(c, mlp_grad, g->net.mlp_grad, kGuideParams * sizeof(float));
+  return st;
 }
 
 // Re-tabulates the guide's proposal if its parameters changed since the last
@@ -2150,9 +2226,7 @@ ne_status ne_guide_get_cache(ne_guide* g, float* mix, uint64_t* entries) {
   NE_HIP(c, hipSetDevice(c->device));
   ne_status st = guide_refresh_cache(c, g);
   if (st != NE_OK) return st;
-  NE_HIP(c, hipMemcpyAsync(mix, g->cache_mix, size_t(n) * 40 * sizeof(float), hipMemcpyDeviceToHost, c->stream));
-  NE_HIP(c, hipStreamSynchronize(c->stream));
-  return NE_OK;
+  return dev_read(c, mix, g->cache_mix, size_t(n) * 40 * sizeof(float));
 }
 
 ne_status ne_render_guided(ne_ctx* c, const ne_scene* s, const ne_camera_desc* cam, const ne_render_params* p,
