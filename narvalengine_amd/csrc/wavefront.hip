@@ -993,23 +993,33 @@ __global__ __launch_bounds__(kChunk) void k_wf_deliver(WfState w, WfArgs a, DevS
 
 // Shadow rays through the volume: ratio tracking, the megakernel's
 // transmittance() after its occlusion test.
-// HAS_SURF: k_wf_occlude has marked the occluded rays.  The rays that are left
-// and cross the volume are packed first, so that waves track whole: both in one
+// SURF: with surfaces, the rays that are left unoccluded and cross the volume
+// are packed first, so that waves track whole: both tests in one go in one
 // thread per ray ran 11% of the lanes (a room with a volume, 857 x 481 at 32
-// spp: 13.2 ms a frame; 8.0 ms in two stages, the frame 28.1 -> 23.0 ms).
+// spp: 13.2 ms a frame; 8.0 ms with a stage for the occlusion and this one, the
+// frame 28.1 -> 23.0 ms).
+// kSurfInline keeps the occlusion test here, before the packing, and saves a
+// launch: for a BVH of a few nodes, whose traversals hardly differ in length,
+// and for small pools, which are launch bound.  Frames of 12 to 24 bounces, us,
+// inline / two stages: 1 node, 130k paths 1122 / 1172, 960k 2301 / 2396; 5936
+// nodes, 120k paths 2754 / 2858, 960k 8299 / 7596, 13M 29800 / 23060.
 // SPATIAL: the chunk's shadow rays are taken in Morton order of their origins
 // (each keeps its own stream: same transmittances).
 // GRID: how density lookups read the grid (kGrid*).
-template <bool C, bool HAS_SURF, bool SPATIAL, int GRID>
+constexpr uint32_t kInlineNodes = 8, kInlineChunks = 512;
+enum { kSurfNone, kSurfMarked, kSurfInline };  // no surfaces; k_wf_occlude has marked the occluded rays; tested here
+template <bool C, int SURF, bool SPATIAL, int GRID>
 __global__ __launch_bounds__(kChunk) void k_wf_shadow(WfState w, WfArgs a, DevScene s) {
+  __shared__ uint32_t lds_stack[SURF == kSurfInline ? kShortStack * kChunk : 1];
   __shared__ uint32_t red[kChunk / 64];
   __shared__ uint32_t skey[SPATIAL ? kChunk : 1];
-  __shared__ uint32_t list[HAS_SURF ? kChunk : 1];
+  __shared__ uint32_t list[SURF != kSurfNone ? kChunk : 1];
   const WfShadow S = w.shadow;
   const WfPaths B = w.paths[a.cur ^ 1];
   const uint32_t c = blockIdx.x, t = threadIdx.x;
   const uint32_t n = w.cnt_shadow[c];
   const uint32_t nc = a.shadow_full ? 0u : w.cnt_paths[a.cur ^ 1][c];  // slots of continuing paths' rays
+  Count<C> cnt;
   uint32_t slot = t;
   if constexpr (SPATIAL) {
     const uint32_t q = c * kChunk + t;
@@ -1019,19 +1029,28 @@ __global__ __launch_bounds__(kChunk) void k_wf_shadow(WfState w, WfArgs a, DevSc
                               skey);
   }
   uint32_t nt = n;  // threads that take a ray
-  if constexpr (HAS_SURF) {
+  if constexpr (SURF != kSurfNone) {
     const uint32_t k = c * kChunk + slot;
     const bool own = slot < nc;
     bool track = false;
-    if (t < n && (!own || S.pl[k] > 0.0f) && !(S.tmax[k] < 0.0f)) {  // holes and occluded rays skipped
+    if (t < n && (!own || S.pl[k] > 0.0f)) {  // holes skipped
+      const float tmax = S.tmax[k];
       Vec3<float> x;
       uint32_t spix, ssmp, svert;
       shadow_source(S, B, k, own, x, spix, ssmp, svert);
       const Vec3<float> wi = v3(S.dx[k], S.dy[k], S.dz[k]);
-      float ta, tb;
-      track = box_interval<float>(s, xf_point<float>(s.inv, x), xf_vec<float>(s.inv, wi), ta, tb) &&
-              xmax(ta, 0.0f) < xmin(tb, S.tmax[k]);
-      if (!track) shadow_deliver(S, B, a, s, k, 1.0f, own);
+      bool clear = !(tmax < 0.0f);
+      if constexpr (SURF == kSurfInline) {
+        cnt.shadow();
+        SurfHit<float> h;
+        clear = !traverse<float, true, C>(s, x, wi, 1e-4f, tmax, lds_stack + t, kChunk, h, cnt);
+      }
+      if (clear) {
+        float ta, tb;
+        track = box_interval<float>(s, xf_point<float>(s.inv, x), xf_vec<float>(s.inv, wi), ta, tb) &&
+                xmax(ta, 0.0f) < xmin(tb, tmax);
+        if (!track) shadow_deliver(S, B, a, s, k, 1.0f, own);
+      }
     }
     const uint32_t at = block_compact(track, red, nt);
     if (track) list[at] = slot;
@@ -1040,7 +1059,6 @@ __global__ __launch_bounds__(kChunk) void k_wf_shadow(WfState w, WfArgs a, DevSc
   }
   const uint32_t k = c * kChunk + slot;
   const bool own = slot < nc;
-  Count<C> cnt;
   Vec3<float> x = v3s(0.0f), wi = v3s(0.0f);
   uint32_t spix = 0, ssmp = 0, svert = 0;
   float tmax = 0.0f, pl = 0.0f;
@@ -1060,7 +1078,7 @@ __global__ __launch_bounds__(kChunk) void k_wf_shadow(WfState w, WfArgs a, DevSc
     PathRng rng;
     rng.init(a.seed, spix, ssmp, a.job);
     PathRng srng = rng.shadow_stream(int(svert));
-    if (!HAS_SURF) cnt.shadow();
+    if (SURF == kSurfNone) cnt.shadow();
     float tr = 1.0f;
     const Vec3<float> oo = xf_point<float>(s.inv, x), dd = xf_vec<float>(s.inv, wi);
     float ta, tb;
@@ -1072,7 +1090,11 @@ __global__ __launch_bounds__(kChunk) void k_wf_shadow(WfState w, WfArgs a, DevSc
     if (tr > 0.0f) shadow_deliver(S, B, a, s, k, tr, own);
   }
   if constexpr (C) {
-    if (!HAS_SURF) block_count<C>(&a.counters->shadow_rays, cnt.n_shadow, red);
+    if (SURF != kSurfMarked) block_count<C>(&a.counters->shadow_rays, cnt.n_shadow, red);
+    if (SURF == kSurfInline) {
+      block_count<C>(&a.counters->sh_nodes, cnt.n_node, red);
+      block_count<C>(&a.counters->sh_prims, cnt.n_prim, red);
+    }
     block_count<C>(&a.counters->sh_lookups, cnt.n_lookup, red);
     block_count<C>(&a.counters->sh_cells, cnt.n_cell, red);
   }
@@ -1379,16 +1401,19 @@ hipError_t launch_wavefront(const DevScene& s, const DevCamera& cam, WfState& w,
   } while (0)
     if (fuse) {
       // done in the shading stage
+    } else if (hs && hv && (s.n_nodes <= kInlineNodes || NC <= kInlineChunks)) {
+      if (count) NE_SHADOW(true, kSurfInline);
+      else NE_SHADOW(false, kSurfInline);
     } else if (hs && hv) {
       NE_OCCLUDE(false);
-      if (count) NE_SHADOW(true, true);
-      else NE_SHADOW(false, true);
+      if (count) NE_SHADOW(true, kSurfMarked);
+      else NE_SHADOW(false, kSurfMarked);
     } else if (hs) {
       NE_OCCLUDE(true);
       hipLaunchKernelGGL(k_wf_deliver<false>, grid, blk, 0, st, w, a, s);
     } else if (hv) {
-      if (count) NE_SHADOW(true, false);
-      else NE_SHADOW(false, false);
+      if (count) NE_SHADOW(true, kSurfNone);
+      else NE_SHADOW(false, kSurfNone);
     } else if (count) {  // neither: nothing is in the way
       hipLaunchKernelGGL(k_wf_deliver<true>, grid, blk, 0, st, w, a, s);
     } else {

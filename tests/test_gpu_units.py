@@ -20,6 +20,7 @@ def ctx():
 
 
 def _scene(which):
+    from narvalengine_amd import configs
     from narvalengine_amd.scene import Scene
     if which == "surface":
         return scenes.small_surface(subdiv=2), scenes.BOX_CAMERA
@@ -28,6 +29,10 @@ def _scene(which):
         s.add_rectangle(s.add_emitter((4.0, 4.0, 4.0)), position=(0, 0.9, 0), rotation=(-90, 0, 0), scale=(0.5, 0.5, 1))
         s.add_point_light((0.7, 0.1, -0.6), s.add_emitter((0.8, 0.8, 0.6)))
         return s, scenes.VOLUME_CAMERA
+    if which == "mixed_mesh":  # more BVH nodes than are tested inside the tracking stage, but for small pools
+        s = scenes.small_surface(subdiv=2)
+        s.set_volume(configs.fbm_grid(16, 0), 12.0, (0.95,) * 3, (0.05,) * 3, 0.7, maj_res=4)
+        return s, scenes.BOX_CAMERA
     s = Scene()
     s.add_point_light((0.3, 0.35, -0.2), s.add_emitter((3.0, 2.5, 2.0)))
     return s, scenes.VOLUME_CAMERA
@@ -41,9 +46,10 @@ SIZES = [(1, 1, 1, 0), (63, 1, 1, 0), (64, 1, 1, 0), (65, 1, 1, 256), (255, 1, 1
 # (with nothing to hit, the wavefront has no stage that counts extension rays)
 EVENTS = {"surface": ("paths", "ext_rays", "shadow_rays"), "neither": ("paths", "shadow_rays"),
           "mixed": ("paths", "ext_rays", "shadow_rays", "density_lookups", "majorant_cells")}
+EVENTS["mixed_mesh"] = EVENTS["mixed"]
 
 
-@pytest.mark.parametrize("which", ["surface", "mixed", "neither"])
+@pytest.mark.parametrize("which", ["surface", "mixed", "mixed_mesh", "neither"])
 @pytest.mark.parametrize("order", ["plain", "sort", "spatial"])
 def test_units_trace_the_megakernels_paths(ctx, which, order):
     print_case(f"units {which} {order}")
