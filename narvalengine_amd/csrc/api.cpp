@@ -1172,7 +1172,7 @@ static ne_status render_locked(ne_ctx* c, const ne_scene* s, const ne_camera_des
   int block = p->block_size ? p->block_size : 128;
   if (timed) NE_HIP(c, hipEventRecord(c->ev0, c->stream));
   if (tm) NE_HIP(c, tm->mark(kStageMegakernel));
-  NE_HIP(c, launch_render(s->dev, dc, a, p->precision, count, block, p->occupancy, c->stream));
+  NE_HIP(c, launch_render(s->dev, dc, a, p->precision, count, block, p->occupancy, c->cus, c->stream));
   if (timed) {
     NE_HIP(c, hipEventRecord(c->ev1, c->stream));
     c->timed = true;
@@ -1221,7 +1221,7 @@ ne_status ne_render_noalloc(ne_ctx* c, const ne_scene* s, const ne_camera_desc* 
   const bool timed = (p->flags & NE_FLAG_TIME) != 0;
   if (timed) NE_HIP(c, hipEventRecord(c->ev0, c->stream));
   NE_HIP(c, launch_render(s->dev, make_camera(cam), a, p->precision, false, p->block_size ? p->block_size : 128,
-                          p->occupancy, c->stream));
+                          p->occupancy, c->cus, c->stream));
   if (timed) {
     NE_HIP(c, hipEventRecord(c->ev1, c->stream));
     c->timed = true;
@@ -1340,7 +1340,7 @@ ne_status ne_li(ne_ctx* c, const ne_scene* s, int32_t n, const float* rays, int3
     char* d = c->stage_dev + (p - c->stage);
     std::memcpy(p, rays, rb);
     NE_HIP(c, launch_li(s->dev, n, reinterpret_cast<const float*>(d), max_bounces, seed, sample_index,
-                        reinterpret_cast<float*>(d + rb), c->stream));
+                        reinterpret_cast<float*>(d + rb), c->cus, c->stream));
     NE_HIP(c, hipStreamSynchronize(c->stream));
     c->stage_in = 0;
     std::memcpy(radiance, p + rb, ob);
@@ -1351,7 +1351,7 @@ ne_status ne_li(ne_ctx* c, const ne_scene* s, int32_t n, const float* rays, int3
   if ((st = tmp_in(c, br, rays, size_t(n) * 6)) != NE_OK) return st;
   if ((st = tmp_out<float>(c, bo, size_t(n) * 3)) != NE_OK) return st;
   NE_HIP(c, launch_li(s->dev, n, static_cast<const float*>(br.p), max_bounces, seed, sample_index,
-                      static_cast<float*>(bo.p), c->stream));
+                      static_cast<float*>(bo.p), c->cus, c->stream));
   return tmp_back(c, radiance, bo, size_t(n) * 3);
 }
 

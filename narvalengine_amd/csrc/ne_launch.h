@@ -52,7 +52,7 @@ inline bool scene_has_surfaces(const DevScene& s) {
 }
 
 hipError_t launch_render(const DevScene& s, const DevCamera& cam, const RenderArgs& a, int precision, bool count,
-                         int block, int occupancy, hipStream_t st);
+                         int block, int occupancy, int cus, hipStream_t st);
 
 // ---- wavefront pipeline ---------------------------------------------------
 // The path pool is split into chunks of kChunk slots; stage kernels run one
@@ -332,7 +332,7 @@ hipError_t launch_test_bsdf(int kind, int n, const float* in0, const float* in1,
 hipError_t launch_test_rng(uint64_t seed, uint32_t pixel, uint32_t sample, uint32_t job, int n, float* out,
                            hipStream_t st);
 hipError_t launch_li(const DevScene& s, int n, const float* rays, int max_bounces, uint64_t seed, uint32_t sample,
-                     float* out, hipStream_t st);
+                     float* out, int cus, hipStream_t st);
 // row-major density -> bricked layout (grid_offset), zero padding
 hipError_t launch_brick_grid(const float* lin, float* out, const int res[3], hipStream_t st);
 // the bricked grid s.grid -> quad layout (quad_pad sizes)

@@ -154,8 +154,23 @@ static hipError_t launch_render_t(const DevScene& s, const DevCamera& cam, const
   return hipGetLastError();
 }
 
+// FP64: unbounded, the kernel takes 256 VGPRs and as many accumulation
+// registers: one wave per SIMD.  Launches of several rounds of that are held to
+// 2 waves per SIMD, large ones without surfaces to 3 (registers spill, the same
+// arithmetic).  ms at 1 / 2 / 3 waves per SIMD (1024 SIMDs): cloud, 1463 waves
+// 0.54 / 0.70, 2070 waves 1.26 / 1.31, 4800 waves 1.03 / 0.99 / 1.19, 32,000
+// waves 4.2 / 3.4 / 3.0; fBm volume, 2088 waves 0.22 / 0.25, 4800 waves 0.90 /
+// 0.83 / 0.82, 32,000 waves 4.2 / 3.4 / 2.8; mesh, 64 waves 1.09 / 1.11 / 1.15,
+// 3025 waves 2.0 / 1.4, 4800 waves 4.1 / 2.8 / 3.0, 32,000 waves 23.3 / 13.8 /
+// 14.1.
 hipError_t launch_render(const DevScene& s, const DevCamera& cam, const RenderArgs& a, int precision, bool count,
-                         int block, int occupancy, hipStream_t st) {
+                         int block, int occupancy, int cus, hipStream_t st) {
+  const int64_t simds = 4 * int64_t(cus), waves = int64_t(a.ntx) * a.nty * a.nchunks;
+  if (precision == 1 && !count && block == 128) {
+    const bool surf = scene_has_surfaces(s);
+    if (!surf && waves >= 16 * simds) return launch_render_t<double, false, 128, 3>(s, cam, a, st);
+    if (waves >= (surf ? 2 : 4) * simds) return launch_render_t<double, false, 128, 2>(s, cam, a, st);
+  }
   if (precision == 0 && !count && occupancy == 4) return launch_render_t<float, false, 128, 4>(s, cam, a, st);
   if (precision == 0 && !count && occupancy == 6) return launch_render_t<float, false, 128, 6>(s, cam, a, st);
 #define NE_DISPATCH(BLK)                                                                       \
@@ -409,17 +424,27 @@ __global__ void k_test_rng(uint64_t seed, uint32_t pixel, uint32_t sample, uint3
   for (int i = 0; i < n; ++i) out[i] = r.next();
 }
 
-template <int BLOCK>
-__global__ __launch_bounds__(BLOCK) void k_li(DevScene s, int n, const float* rays, int max_bounces, uint64_t seed,
-                                               uint32_t sample, float* out) {
+// One path per ray; a wave takes `lanes` rays.  A call is as long as its longest
+// wave, and a wave as its lanes' branches one after the other: calls that would
+// not fill the SIMDs spread their rays over more waves of fewer lanes, up to two
+// waves per SIMD (launch_li).  Volume-only scenes take the kernel without
+// surface code (131 VGPRs instead of 156).  us, 64 lanes / spread: a cloud, 64
+// rays 580 / 298, 1000 rays 705 / 320, 20,000 rays 751 / 481, 65,536 rays 937 /
+// 633, 250,000 rays 1687 / 1568; a mesh of 20 k triangles, 1000 rays 900 / 380,
+// 65,536 rays 1209 / 927.  Up to three waves gained at 20,000 rays (444) and
+// lost from 65,536 on (733, 100,000 rays 1055 against 950).
+template <int BLOCK, bool SURF>
+__global__ __launch_bounds__(BLOCK) void k_li(DevScene s, int n, int lanes, const float* rays, int max_bounces,
+                                               uint64_t seed, uint32_t sample, float* out) {
   __shared__ uint32_t lds_stack[kShortStack * BLOCK];
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+  const int lane = int(threadIdx.x & 63u), wave = int(blockIdx.x) * (BLOCK / 64) + int(threadIdx.x >> 6);
+  const int64_t i = int64_t(wave) * lanes + lane;
+  if (lane >= lanes || i >= n) return;
   Count<false> cnt;
   PathRng rng;
   rng.init(seed, uint32_t(i), sample, 0);
-  Vec3<float> L = trace_path<float, false>(s, v3f<float>(rays + 6 * i), v3f<float>(rays + 6 * i + 3), max_bounces,
-                                           rng, lds_stack + threadIdx.x, BLOCK, cnt);
+  Vec3<float> L = trace_path<float, false, SURF>(s, v3f<float>(rays + 6 * i), v3f<float>(rays + 6 * i + 3),
+                                                 max_bounces, rng, lds_stack + threadIdx.x, BLOCK, cnt);
   out[3 * i] = L.x; out[3 * i + 1] = L.y; out[3 * i + 2] = L.z;
 }
 
@@ -468,8 +493,16 @@ hipError_t launch_test_rng(uint64_t seed, uint32_t pixel, uint32_t sample, uint3
   return hipGetLastError();
 }
 hipError_t launch_li(const DevScene& s, int n, const float* rays, int max_bounces, uint64_t seed, uint32_t sample,
-                     float* out, hipStream_t st) {
-  hipLaunchKernelGGL(k_li<128>, grid1(n, 128), dim3(128), 0, st, s, n, rays, max_bounces, seed, sample, out);
+                     float* out, int cus, hipStream_t st) {
+  constexpr int kBlock = 128;
+  const int spread = std::max(1, cus * 4 * 2);
+  const int lanes = std::min(64, std::max(1, n / spread));
+  const int waves = (n - 1) / lanes + 1;
+  const dim3 grid(uint32_t((waves + kBlock / 64 - 1) / (kBlock / 64))), blk(kBlock);
+  if (scene_has_surfaces(s))
+    hipLaunchKernelGGL((k_li<kBlock, true>), grid, blk, 0, st, s, n, lanes, rays, max_bounces, seed, sample, out);
+  else
+    hipLaunchKernelGGL((k_li<kBlock, false>), grid, blk, 0, st, s, n, lanes, rays, max_bounces, seed, sample, out);
   return hipGetLastError();
 }
 
