@@ -144,6 +144,8 @@ struct WfArgs {
   int32_t shadow_full;  // every shadow record carries its origin and RNG key (surface-only scenes)
   int32_t wide_offsets;  // density lookups by 64-bit offsets whatever the grid's size
   uint32_t plan_stall;   // test hook: the plan's look-back waits for an epoch that never comes
+  int32_t shadows;      // the BVH stage takes the last iteration's shadow rays too
+  int32_t regen_done;   // the buffer that the shadow rays' paths go on in holds regen_m new paths besides
   int32_t regen_fused;  // this iteration's medium stage makes the new paths and leaves the live
                         // counts as they were: later stages add regen_m
 };

@@ -200,6 +200,7 @@ struct TravState {
   uint32_t cur, leaf, bkey, bslot;  // leaf: parked leaf item (trav_step_wave), or kItemNone
   int sp, btype;
   bool found;
+  bool any;  // the ray's kind where one kernel takes both (ANY == 2)
 };
 
 template <typename R>
@@ -245,9 +246,9 @@ NE_DEV bool trav_pop(TravState<R>& st, const uint32_t* lds, int lane_stride, con
 }
 
 // Test of the first primitive of leaf item `it`: updates the closest hit and
-// returns true on a hit for ANY.  next: the leaf's next primitive item, or
+// returns true on a hit for ANY (0 closest hit, 1 any hit, 2 as st.any says).  next: the leaf's next primitive item, or
 // kItemNone after its last.
-template <typename R, bool ANY, bool C>
+template <typename R, int ANY, bool C>
 NE_DEV bool trav_prim(const DevScene& s, TravState<R>& st, uint32_t it, uint32_t& next, Count<C>& cnt) {
   const uint32_t ty = (it >> 29) & 3u, k = it & kItemFirstMask;
   R t;
@@ -267,7 +268,7 @@ NE_DEV bool trav_prim(const DevScene& s, TravState<R>& st, uint32_t it, uint32_t
     if (ok) key = __float_as_uint(rc[2].w);
   }
   if (ok) {
-    if (ANY) {
+    if (ANY == 1 || (ANY == 2 && st.any)) {
       st.found = true;
       return true;
     }
@@ -290,7 +291,7 @@ NE_DEV bool trav_prim(const DevScene& s, TravState<R>& st, uint32_t it, uint32_t
 // (surface1m at 64 spp: 101.3 -> 87.6 ms).  The seven loads go out together,
 // which takes 68 VGPRs in k_wf_trace: held to 64 for an eighth wave the
 // compiler splits them and the frame takes 97 ms.
-template <typename R, bool ANY, bool C>
+template <typename R, int ANY, bool C>
 NE_DEV bool trav_node(const DevScene& s, TravState<R>& st, uint32_t* lds, int lane_stride, uint32_t* spill,
                       Count<C>& cnt) {
   // 4-wide inner node (128 B): test the four child boxes, continue with the
@@ -318,7 +319,7 @@ NE_DEV bool trav_node(const DevScene& s, TravState<R>& st, uint32_t* lds, int la
     const uint32_t il = swap ? ib : ia, ih = swap ? ia : ib;
     ta = lo; tb = hi; ia = il; ib = ih;
   };
-  if constexpr (ANY) {
+  if constexpr (ANY == 1) {
     order(t2, i2, t3, i3);
     order(t1, i1, t2, i2);
     order(t0, i0, t1, i1);
@@ -353,7 +354,7 @@ NE_DEV bool trav_node(const DevScene& s, TravState<R>& st, uint32_t* lds, int la
 // One node visit or one primitive test.  Returns true when the query is
 // complete: the stack is empty, or (ANY) a hit was found.  lds: this lane's
 // short stack (entries lane_stride apart); spill: its private overflow array.
-template <typename R, bool ANY, bool C>
+template <typename R, int ANY, bool C>
 NE_DEV bool trav_step(const DevScene& s, TravState<R>& st, uint32_t* lds, int lane_stride, uint32_t* spill,
                       Count<C>& cnt) {
   const uint32_t it = st.cur;
@@ -379,7 +380,7 @@ NE_DEV bool trav_step(const DevScene& s, TravState<R>& st, uint32_t* lds, int la
 // change the closest hit (ties break on type and original index); parked
 // leaves only delay the shrinking of the search interval.  Every lane with a
 // live query calls it; returns true when this lane's query is complete.
-template <typename R, bool ANY, bool C>
+template <typename R, int ANY, bool C>
 NE_DEV bool trav_step_wave(const DevScene& s, TravState<R>& st, uint32_t* lds, int lane_stride, uint32_t* spill,
                            Count<C>& cnt) {
   const bool at_node = !(st.cur & kItemLeaf);
@@ -400,7 +401,7 @@ NE_DEV bool trav_step_wave(const DevScene& s, TravState<R>& st, uint32_t* lds, i
   return st.cur == kItemNone && st.leaf == kItemNone;
 }
 
-template <typename R, bool ANY, bool C>
+template <typename R, int ANY, bool C>
 NE_DEV bool traverse(const DevScene& s, Vec3<R> o, Vec3<R> d, R tmin, R tmax, uint32_t* lds, int lane_stride,
                      SurfHit<R>& hit, Count<C>& cnt) {
   if (s.n_nodes == 0) return false;

@@ -304,27 +304,33 @@ __global__ __launch_bounds__(kChunk) void k_wf_regen(WfState w, WfArgs a, DevCam
 struct UnitQueue {
   uint32_t* next;     // the block's next unit (LDS)
   uint32_t nchunks;
+  uint32_t nshadow;   // its units of shadow rays, taken before those of paths
   uint32_t cur, end;  // slots left of the current unit
+  bool shadow;        // what the current unit holds
 };
 constexpr uint32_t kUnits = kChunk / 64;  // per chunk
 __device__ __forceinline__ uint32_t uniform(uint32_t v) { return uint32_t(__builtin_amdgcn_readfirstlane(int(v))); }
-__device__ __forceinline__ void units_init(UnitQueue& q, uint32_t* next, uint32_t nchunks) {
+__device__ __forceinline__ void units_init(UnitQueue& q, uint32_t* next, uint32_t nchunks, bool shadows) {
   if (threadIdx.x == 0) *next = 0u;
   q.next = next;
   q.nchunks = nchunks;
+  q.nshadow = shadows ? (nchunks - blockIdx.x + gridDim.x - 1) / gridDim.x * kUnits : 0u;  // gridDim.x <= nchunks
   q.cur = q.end = 0;
+  q.shadow = false;
   __syncthreads();
 }
-// Next unit that holds rays (cnt: rays per chunk) into q.cur, q.end; false when
-// the block has none left.  The whole wave calls it.
-__device__ __forceinline__ bool units_next(UnitQueue& q, const uint32_t* cnt) {
+// Next unit that holds rays (paths, shadows: rays per chunk) into q.cur, q.end;
+// false when the block has none left.  The whole wave calls it.
+__device__ __forceinline__ bool units_next(UnitQueue& q, const uint32_t* paths, const uint32_t* shadows) {
   while (true) {
     uint32_t u = 0;
     if (__lane_id() == 0) u = atomicAdd(q.next, 1u);
     u = uniform(u);
+    q.shadow = u < q.nshadow;
+    if (!q.shadow) u -= q.nshadow;
     const uint32_t c = blockIdx.x + u / kUnits * gridDim.x, lo = u % kUnits * 64;
     if (c >= q.nchunks) return false;
-    const uint32_t n = uniform(cnt[c]);
+    const uint32_t n = uniform((q.shadow ? shadows : paths)[c]);
     if (n > lo) {
       q.cur = c * kChunk + lo;
       q.end = c * kChunk + (n < lo + 64 ? n : lo + 64);
@@ -334,8 +340,9 @@ __device__ __forceinline__ bool units_next(UnitQueue& q, const uint32_t* cnt) {
 }
 // Slots for the lanes with need == true from the current unit (or the next);
 // kNoHit for the lanes that it does not reach.  none: nothing is left.
-__device__ __forceinline__ uint32_t units_fetch(UnitQueue& q, const uint32_t* cnt, bool need, bool& none) {
-  if (q.cur == q.end && !units_next(q, cnt)) {
+__device__ __forceinline__ uint32_t units_fetch(UnitQueue& q, const uint32_t* paths, const uint32_t* shadows, bool need,
+                                                bool& none) {
+  if (q.cur == q.end && !units_next(q, paths, shadows)) {
     none = true;
     return kNoHit;
   }
@@ -352,46 +359,154 @@ __device__ __forceinline__ uint32_t units_fetch(UnitQueue& q, const uint32_t* cn
 // fewer steps, and so do the finished rays' stores, which are made there.
 __device__ __forceinline__ bool refill_due(bool have, int min_idle) { return __popcll(__ballot(!have)) >= min_idle; }
 
-// Closest surface hit of every live ray: pure BVH traversal (no random
-// numbers), lane refill.
+// Shadow-queue layouts.  Full (WfArgs::shadow_full): the chunk's rays packed,
+// each record whole.  Otherwise (scenes with a volume): slot k < ncont of the
+// chunk is the ray of the continuing path at the same index of the next
+// buffer (a hole, light pdf 0, if that path has none), whose record there
+// holds the ray's origin (the vertex), pixel, sample and vertex (its depth
+// minus one); the rays of paths that end follow, each record whole.
+// own: slot k is a continuing path's.
+// (Branch-free: each array chosen per lane, so the six loads go out together.)
+__device__ __forceinline__ void shadow_source(const WfShadow& S, const WfPaths& B, uint32_t k, bool own,
+                                              Vec3<float>& x, uint32_t& pix, uint32_t& smp, uint32_t& vert) {
+  const SlotF ax = own ? B.ox : S.ox, ay = own ? B.oy : S.oy, az = own ? B.oz : S.oz;
+  const SlotU ap = own ? B.pix : S.pix, as = own ? B.smp : S.smp, av = own ? B.depth : S.vert;
+  x = v3(ax[k], ay[k], az[k]);
+  pix = ap[k];
+  smp = as[k];
+  vert = av[k] - (own ? 1u : 0u);
+}
+
+// NEE contribution of an unoccluded shadow ray k (transmittance tr): to the
+// continuing path in the next buffer (same chunk) or straight to the film.
+__device__ __forceinline__ void shadow_deliver(const WfShadow& S, const WfPaths& B, const WfArgs& a,
+                                               const DevScene& s, uint32_t k, float tr, bool own = false) {
+  const float q = tr * S.wt[k] * float(s.n_lights) / S.pl[k];
+  const float cx = S.cx[k] * q, cy = S.cy[k] * q, cz = S.cz[k] * q;
+  if (own) {
+    B.Lx[k] += cx; B.Ly[k] += cy; B.Lz[k] += cz;
+    return;
+  }
+  const uint32_t tg = S.target[k];
+  if (tg & kToFilm) {
+    // the final vertex's light sample: a fire-and-forget atomic on the
+    // fixed-point film (a read-modify-write of the sample slot would wait)
+    film_add(a.film_fixed, tg & ~kToFilm, cx, cy, cz);
+  } else {
+    const uint32_t b = (k / kChunk) * kChunk + tg;
+    B.Lx[b] += cx; B.Ly[b] += cy; B.Lz[b] += cz;
+  }
+}
+
+// Continuing paths whose shadow rays sit at their own slots of chunk c (none in
+// the full layout): b is the buffer that they go on in, which may hold
+// a.regen_done new paths besides.
+__device__ __forceinline__ uint32_t shadow_own(const WfState& w, const WfArgs& a, int b, uint32_t c) {
+  if (a.shadow_full) return 0u;
+  return w.cnt_paths[b][c] - (a.regen_done ? w.regen_m[c] : 0u);
+}
+
+// The BVH stage: the closest surface hit of every live ray and, for the shadow
+// rays that the last iteration queued (a.shadows), whether a surface occludes
+// them: pure traversal (no random numbers), lane refill, both kinds in one
+// launch.  Each launch ends with the long rays of a few waves; the two kinds,
+// which do not depend on each other, share one such end (two launches / one, ms:
+// 640 x 360 preview at 4 spp 2.45 / 2.03, room with a volume 22.9 / 22.1,
+// surface1m at 64 spp 81.1 / 80.4).
+// Occluded rays are marked (tmax = -1) for the stage that delivers the others:
+// out of the refill loop, where a finishing lane would hold its whole wave.
+struct TraceArgs {
+  WfState w;
+  WfArgs a;
+  DevScene s;
+};
+// The arguments' address, opaque to the optimiser: what the refill path reads
+// through it is loaded there, by scalar loads.  Hoisted out of the loop, the
+// record arrays' addresses took 106 SGPRs, and only 6 of 7 blocks fit on a CU:
+// the grid's last blocks ran alone (surface1m 101 ms).
+__device__ __forceinline__ const TraceArgs& refill_args() {
+  typedef const __attribute__((address_space(4))) TraceArgs* Ptr;
+  Ptr p = (Ptr)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *(const TraceArgs*)p;
+}
 template <bool C>
-__global__ __launch_bounds__(kChunk) void k_wf_trace(WfState w, WfArgs a, DevScene s) {
+__global__ __launch_bounds__(kChunk) void k_wf_trace(TraceArgs g) {
   __shared__ uint32_t lds_stack[kShortStack * kChunk];
   __shared__ uint32_t red[kChunk / 64];
-  const WfPaths A = w.paths[a.cur];
   __shared__ uint32_t next;
+  const DevScene& s = g.s;
+  const int refill_min = g.a.refill_min;
   UnitQueue q;
-  units_init(q, &next, a.nchunks);
+  units_init(q, &next, g.a.nchunks, g.a.shadows != 0);
   uint32_t* stk = lds_stack + threadIdx.x;
   uint32_t spill[kSpillStack];
-  Count<C> cnt;
+  Count<C> cnt, scnt;
   TravState<float> st;
+  st.any = false;
   uint32_t slot = kNoHit;
   bool have = false, none = false;
   while (true) {
-    if (refill_due(have, none ? 64 : a.refill_min)) {
+    if (refill_due(have, none ? 64 : refill_min)) {
+      const TraceArgs& ra = refill_args();
+      const WfState& w = ra.w;
+      const WfArgs& a = ra.a;
+      const WfPaths& A = w.paths[a.cur];
+      const WfShadow& S = w.shadow;
       if (!have && slot != kNoHit) {
-        A.hit_t[slot] = st.found ? st.best : xinf<float>();
-        A.hit_ref[slot] = st.found ? ((uint32_t(st.btype) << 30) | st.bslot) : kNoHit;
-        A.kind[slot] = st.found ? uint32_t(WF_KIND_SURFACE) : uint32_t(WF_KIND_MISS);
+        if (!st.any) {
+          A.hit_t[slot] = st.found ? st.best : xinf<float>();
+          A.hit_ref[slot] = st.found ? ((uint32_t(st.btype) << 30) | st.bslot) : kNoHit;
+          A.kind[slot] = st.found ? uint32_t(WF_KIND_SURFACE) : uint32_t(WF_KIND_MISS);
+        } else if (st.found) {
+          S.tmax[slot] = -1.0f;
+        }
         slot = kNoHit;
       }
       if (none) break;
-      const uint32_t got = units_fetch(q, w.cnt_paths[a.cur], !have, none);
+      const uint32_t got = units_fetch(q, w.cnt_paths[a.cur], w.cnt_shadow, !have, none);
       if (got != kNoHit) {
-        slot = got;
-        have = true;
-        cnt.ext();
-        trav_init(st, v3(A.ox[slot], A.oy[slot], A.oz[slot]), v3(A.dx[slot], A.dy[slot], A.dz[slot]), 1e-4f,
-                  xinf<float>());
+        Vec3<float> o, d;
+        float tmax = xinf<float>();
+        bool hole = false;
+        if (!q.shadow) {
+          o = v3(A.ox[got], A.oy[got], A.oz[got]);
+          d = v3(A.dx[got], A.dy[got], A.dz[got]);
+          cnt.ext();
+        } else {
+          const bool own = got % kChunk < shadow_own(w, a, a.cur, got / kChunk);
+          uint32_t pix, smp, vert;
+          shadow_source(S, A, got, own, o, pix, smp, vert);
+          d = v3(S.dx[got], S.dy[got], S.dz[got]);
+          tmax = S.tmax[got];
+          hole = own && !(S.pl[got] > 0.0f);
+          if (!hole) scnt.shadow();
+        }
+        if (!hole) {
+          slot = got;
+          have = true;
+          st.any = q.shadow;
+          trav_init(st, o, d, 1e-4f, tmax);
+        }
       }
     }
-    if (have && trav_step_wave<float, false, C>(s, st, stk, kChunk, spill, cnt)) have = false;
+    if (have) {
+      Count<C> one;
+      if (trav_step_wave<float, 2, C>(s, st, stk, kChunk, spill, one)) have = false;
+      if constexpr (C) {
+        Count<C>& to = st.any ? scnt : cnt;
+        to.n_node += one.n_node;
+        to.n_prim += one.n_prim;
+      }
+    }
   }
   if constexpr (C) {
-    block_count<C>(&a.counters->ext_rays, cnt.n_ext, red);
-    block_count<C>(&a.counters->bvh_nodes, cnt.n_node, red);
-    block_count<C>(&a.counters->prim_tests, cnt.n_prim, red);
+    block_count<C>(&g.a.counters->ext_rays, cnt.n_ext, red);
+    block_count<C>(&g.a.counters->bvh_nodes, cnt.n_node, red);
+    block_count<C>(&g.a.counters->prim_tests, cnt.n_prim, red);
+    block_count<C>(&g.a.counters->shadow_rays, scnt.n_shadow, red);
+    block_count<C>(&g.a.counters->sh_nodes, scnt.n_node, red);
+    block_count<C>(&g.a.counters->sh_prims, scnt.n_prim, red);
   }
 }
 
@@ -887,101 +1002,7 @@ __global__ __launch_bounds__(kChunk, (GUIDED && !TRAIN) ? 7 : 1) void k_wf_shade
   }
 }
 
-// Shadow-queue layouts.  Full (WfArgs::shadow_full): the chunk's rays packed,
-// each record whole.  Otherwise (scenes with a volume): slot k < ncont of the
-// chunk is the ray of the continuing path at the same index of the next
-// buffer (a hole, light pdf 0, if that path has none), whose record there
-// holds the ray's origin (the vertex), pixel, sample and vertex (its depth
-// minus one); the rays of paths that end follow, each record whole.
-// own: slot k is a continuing path's.
-// (Branch-free: each array chosen per lane, so the six loads go out together.)
-__device__ __forceinline__ void shadow_source(const WfShadow& S, const WfPaths& B, uint32_t k, bool own,
-                                              Vec3<float>& x, uint32_t& pix, uint32_t& smp, uint32_t& vert) {
-  const SlotF ax = own ? B.ox : S.ox, ay = own ? B.oy : S.oy, az = own ? B.oz : S.oz;
-  const SlotU ap = own ? B.pix : S.pix, as = own ? B.smp : S.smp, av = own ? B.depth : S.vert;
-  x = v3(ax[k], ay[k], az[k]);
-  pix = ap[k];
-  smp = as[k];
-  vert = av[k] - (own ? 1u : 0u);
-}
-
-// NEE contribution of an unoccluded shadow ray k (transmittance tr): to the
-// continuing path in the next buffer (same chunk) or straight to the film.
-__device__ __forceinline__ void shadow_deliver(const WfShadow& S, const WfPaths& B, const WfArgs& a,
-                                               const DevScene& s, uint32_t k, float tr, bool own = false) {
-  const float q = tr * S.wt[k] * float(s.n_lights) / S.pl[k];
-  const float cx = S.cx[k] * q, cy = S.cy[k] * q, cz = S.cz[k] * q;
-  if (own) {
-    B.Lx[k] += cx; B.Ly[k] += cy; B.Lz[k] += cz;
-    return;
-  }
-  const uint32_t tg = S.target[k];
-  if (tg & kToFilm) {
-    // the final vertex's light sample: a fire-and-forget atomic on the
-    // fixed-point film (a read-modify-write of the sample slot would wait)
-    film_add(a.film_fixed, tg & ~kToFilm, cx, cy, cz);
-  } else {
-    const uint32_t b = (k / kChunk) * kChunk + tg;
-    B.Lx[b] += cx; B.Ly[b] += cy; B.Lz[b] += cz;
-  }
-}
-
-// Shadow rays against the surfaces: any-hit BVH occlusion with lane refill.
-// Occluded rays are marked (tmax = -1) for the stage that delivers the others:
-// out of the refill loop, where a finishing lane would hold its whole wave.
-// FULL: the queue's layout (WfArgs::shadow_full).
-template <bool C, bool FULL>
-__global__ __launch_bounds__(kChunk) void k_wf_occlude(WfState w, WfArgs a, DevScene s) {
-  __shared__ uint32_t lds_stack[kShortStack * kChunk];
-  __shared__ uint32_t red[kChunk / 64];
-  const WfShadow S = w.shadow;
-  const WfPaths B = w.paths[a.cur ^ 1];
-  __shared__ uint32_t next;
-  UnitQueue q;
-  units_init(q, &next, a.nchunks);
-  uint32_t* stk = lds_stack + threadIdx.x;
-  uint32_t spill[kSpillStack];
-  Count<C> cnt;
-  TravState<float> st;
-  uint32_t k = kNoHit;
-  bool have = false, none = false;
-  while (true) {
-    if (refill_due(have, none ? 64 : a.refill_min)) {
-      if (!have && k != kNoHit) {
-        if (st.found) S.tmax[k] = -1.0f;
-        k = kNoHit;
-      }
-      if (none) break;
-      const uint32_t got = units_fetch(q, w.cnt_shadow, !have, none);
-      if (got != kNoHit) {
-        Vec3<float> x;
-        bool hole = false;
-        if constexpr (FULL) {
-          x = v3(S.ox[got], S.oy[got], S.oz[got]);
-        } else {
-          const bool own = got % kChunk < w.cnt_paths[a.cur ^ 1][got / kChunk];
-          uint32_t pix, smp, vert;
-          shadow_source(S, B, got, own, x, pix, smp, vert);
-          hole = own && !(S.pl[got] > 0.0f);
-        }
-        if (!hole) {
-          k = got;
-          have = true;
-          cnt.shadow();
-          trav_init(st, x, v3(S.dx[k], S.dy[k], S.dz[k]), 1e-4f, S.tmax[k]);
-        }
-      }
-    }
-    if (have && trav_step_wave<float, true, C>(s, st, stk, kChunk, spill, cnt)) have = false;
-  }
-  if constexpr (C) {
-    block_count<C>(&a.counters->shadow_rays, cnt.n_shadow, red);
-    block_count<C>(&a.counters->sh_nodes, cnt.n_node, red);
-    block_count<C>(&a.counters->sh_prims, cnt.n_prim, red);
-  }
-}
-
-// Scenes without a volume: the contributions of the rays that k_wf_occlude left
+// Scenes without a volume: the contributions of the rays that k_wf_trace left
 // unoccluded, one queue entry per thread in order (coalesced).
 // C: count the rays (scenes without surfaces, where no other stage does).
 template <bool C>
@@ -993,32 +1014,26 @@ __global__ __launch_bounds__(kChunk) void k_wf_deliver(WfState w, WfArgs a, DevS
 
 // Shadow rays through the volume: ratio tracking, the megakernel's
 // transmittance() after its occlusion test.
-// SURF: with surfaces, the rays that are left unoccluded and cross the volume
-// are packed first, so that waves track whole: both tests in one go in one
-// thread per ray ran 11% of the lanes (a room with a volume, 857 x 481 at 32
-// spp: 13.2 ms a frame; 8.0 ms with a stage for the occlusion and this one, the
-// frame 28.1 -> 23.0 ms).
-// kSurfInline keeps the occlusion test here, before the packing, and saves a
-// launch: for a BVH of a few nodes, whose traversals hardly differ in length,
-// and for small pools, which are launch bound.  Frames of 12 to 24 bounces, us,
-// inline / two stages: 1 node, 130k paths 1122 / 1172, 960k 2301 / 2396; 5936
-// nodes, 120k paths 2754 / 2858, 960k 8299 / 7596, 13M 29800 / 23060.
+// HAS_SURF: k_wf_trace has marked the occluded rays.  The rays that are left
+// and cross the volume are packed first, so that waves track whole: both tests
+// in one go in one thread per ray ran 11% of the lanes (a room with a volume,
+// 857 x 481 at 32 spp: 13.2 ms a frame; 8.0 ms in two stages, the frame 28.1 ->
+// 23.0 ms).  With the occlusion test in the BVH stage that is launched anyway,
+// two stages are no slower in small frames either (us, tested here / there: 90 x
+// 90 at 16 spp, 5936 nodes 2861 / 2212, one node 1155 / 1139).
 // SPATIAL: the chunk's shadow rays are taken in Morton order of their origins
 // (each keeps its own stream: same transmittances).
 // GRID: how density lookups read the grid (kGrid*).
-constexpr uint32_t kInlineNodes = 8, kInlineChunks = 512;
-enum { kSurfNone, kSurfMarked, kSurfInline };  // no surfaces; k_wf_occlude has marked the occluded rays; tested here
-template <bool C, int SURF, bool SPATIAL, int GRID>
+template <bool C, bool HAS_SURF, bool SPATIAL, int GRID>
 __global__ __launch_bounds__(kChunk) void k_wf_shadow(WfState w, WfArgs a, DevScene s) {
-  __shared__ uint32_t lds_stack[SURF == kSurfInline ? kShortStack * kChunk : 1];
   __shared__ uint32_t red[kChunk / 64];
   __shared__ uint32_t skey[SPATIAL ? kChunk : 1];
-  __shared__ uint32_t list[SURF != kSurfNone ? kChunk : 1];
+  __shared__ uint32_t list[HAS_SURF ? kChunk : 1];
   const WfShadow S = w.shadow;
   const WfPaths B = w.paths[a.cur ^ 1];
   const uint32_t c = blockIdx.x, t = threadIdx.x;
   const uint32_t n = w.cnt_shadow[c];
-  const uint32_t nc = a.shadow_full ? 0u : w.cnt_paths[a.cur ^ 1][c];  // slots of continuing paths' rays
+  const uint32_t nc = shadow_own(w, a, a.cur ^ 1, c);  // slots of continuing paths' rays
   Count<C> cnt;
   uint32_t slot = t;
   if constexpr (SPATIAL) {
@@ -1029,28 +1044,20 @@ __global__ __launch_bounds__(kChunk) void k_wf_shadow(WfState w, WfArgs a, DevSc
                               skey);
   }
   uint32_t nt = n;  // threads that take a ray
-  if constexpr (SURF != kSurfNone) {
+  if constexpr (HAS_SURF) {
     const uint32_t k = c * kChunk + slot;
     const bool own = slot < nc;
     bool track = false;
-    if (t < n && (!own || S.pl[k] > 0.0f)) {  // holes skipped
-      const float tmax = S.tmax[k];
+    const float tmax = t < n && (!own || S.pl[k] > 0.0f) ? S.tmax[k] : -1.0f;
+    if (!(tmax < 0.0f)) {  // holes and occluded rays skipped
       Vec3<float> x;
       uint32_t spix, ssmp, svert;
       shadow_source(S, B, k, own, x, spix, ssmp, svert);
       const Vec3<float> wi = v3(S.dx[k], S.dy[k], S.dz[k]);
-      bool clear = !(tmax < 0.0f);
-      if constexpr (SURF == kSurfInline) {
-        cnt.shadow();
-        SurfHit<float> h;
-        clear = !traverse<float, true, C>(s, x, wi, 1e-4f, tmax, lds_stack + t, kChunk, h, cnt);
-      }
-      if (clear) {
-        float ta, tb;
-        track = box_interval<float>(s, xf_point<float>(s.inv, x), xf_vec<float>(s.inv, wi), ta, tb) &&
-                xmax(ta, 0.0f) < xmin(tb, tmax);
-        if (!track) shadow_deliver(S, B, a, s, k, 1.0f, own);
-      }
+      float ta, tb;
+      track = box_interval<float>(s, xf_point<float>(s.inv, x), xf_vec<float>(s.inv, wi), ta, tb) &&
+              xmax(ta, 0.0f) < xmin(tb, tmax);
+      if (!track) shadow_deliver(S, B, a, s, k, 1.0f, own);
     }
     const uint32_t at = block_compact(track, red, nt);
     if (track) list[at] = slot;
@@ -1078,7 +1085,7 @@ __global__ __launch_bounds__(kChunk) void k_wf_shadow(WfState w, WfArgs a, DevSc
     PathRng rng;
     rng.init(a.seed, spix, ssmp, a.job);
     PathRng srng = rng.shadow_stream(int(svert));
-    if (SURF == kSurfNone) cnt.shadow();
+    if (!HAS_SURF) cnt.shadow();
     float tr = 1.0f;
     const Vec3<float> oo = xf_point<float>(s.inv, x), dd = xf_vec<float>(s.inv, wi);
     float ta, tb;
@@ -1090,11 +1097,7 @@ __global__ __launch_bounds__(kChunk) void k_wf_shadow(WfState w, WfArgs a, DevSc
     if (tr > 0.0f) shadow_deliver(S, B, a, s, k, tr, own);
   }
   if constexpr (C) {
-    if (SURF != kSurfMarked) block_count<C>(&a.counters->shadow_rays, cnt.n_shadow, red);
-    if (SURF == kSurfInline) {
-      block_count<C>(&a.counters->sh_nodes, cnt.n_node, red);
-      block_count<C>(&a.counters->sh_prims, cnt.n_prim, red);
-    }
+    if (!HAS_SURF) block_count<C>(&a.counters->shadow_rays, cnt.n_shadow, red);
     block_count<C>(&a.counters->sh_lookups, cnt.n_lookup, red);
     block_count<C>(&a.counters->sh_cells, cnt.n_cell, red);
   }
@@ -1266,6 +1269,27 @@ hipError_t launch_wavefront(const DevScene& s, const DevCamera& cam, WfState& w,
   // Drain: once every path of the render has been issued, the plan would
   // only count the paths in flight, so it is no longer launched (nor regen);
   // the loop ends on the live flag the shading stage keeps instead.
+#define NE_SHADOW_SP(CNT, S_, SM, ARGS)                                                             \
+  do {                                                                                              \
+    if (spatial) hipLaunchKernelGGL((k_wf_shadow<CNT, S_, true, SM>), grid, blk, 0, st, w, ARGS, s);  \
+    else hipLaunchKernelGGL((k_wf_shadow<CNT, S_, false, SM>), grid, blk, 0, st, w, ARGS, s);       \
+  } while (0)
+#define NE_SHADOW(CNT, S_, ARGS)                                      \
+  do {                                                                \
+    if (form == kGridQuad) NE_SHADOW_SP(CNT, S_, kGridQuad, ARGS);        \
+    else if (form == kGridBrick) NE_SHADOW_SP(CNT, S_, kGridBrick, ARGS); \
+    else NE_SHADOW_SP(CNT, S_, kGridWide, ARGS);                      \
+  } while (0)
+  // the rest of the last iteration's shadow rays, after the BVH stage that took
+  // them; planned: new paths have joined theirs since
+  auto deliver_last = [&](bool planned) {
+    WfArgs d = a;
+    d.cur ^= 1;
+    d.regen_done = planned ? 1 : 0;
+    if (!hv) hipLaunchKernelGGL(k_wf_deliver<false>, grid, blk, 0, st, w, d, s);
+    else if (count) NE_SHADOW(true, true, d);
+    else NE_SHADOW(false, true, d);
+  };
   bool drain = false;
   for (uint32_t it = 0;; ++it) {
     a.cur = int(it & 1u);
@@ -1296,7 +1320,18 @@ hipError_t launch_wavefront(const DevScene& s, const DevCamera& cam, WfState& w,
         return e;
       if ((e = hipStreamSynchronize(st)) != hipSuccess) return e;
       if (h_status[4] != 0) return hipErrorLaunchTimeOut;  // a plan block's look-back gave up
-      if (h_status[0] == 0) break;
+      if (h_status[0] == 0) {
+        if (hs && it > 0) {  // no paths are left, but the last vertices' shadow rays
+          NE_MARK(kStageOther);
+          a.shadows = 1;
+          a.regen_done = 0;
+          if (count) hipLaunchKernelGGL(k_wf_trace<true>, pgrid, blk, 0, st, TraceArgs{w, a, s});
+          else hipLaunchKernelGGL(k_wf_trace<false>, pgrid, blk, 0, st, TraceArgs{w, a, s});
+          NE_MARK(kStageShadow);
+          deliver_last(false);
+        }
+        break;
+      }
       if (planned) {
         unsigned long long issued;
         std::memcpy(&issued, h_status + 2, sizeof(issued));
@@ -1323,8 +1358,15 @@ hipError_t launch_wavefront(const DevScene& s, const DevCamera& cam, WfState& w,
     }
     if (hs) {
       NE_MARK(kStageTrace);
-      if (count) hipLaunchKernelGGL(k_wf_trace<true>, pgrid, blk, 0, st, w, a, s);
-      else hipLaunchKernelGGL(k_wf_trace<false>, pgrid, blk, 0, st, w, a, s);
+      a.shadows = it > 0 ? 1 : 0;
+      a.regen_done = planned ? 1 : 0;
+      if (count) hipLaunchKernelGGL(k_wf_trace<true>, pgrid, blk, 0, st, TraceArgs{w, a, s});
+      else hipLaunchKernelGGL(k_wf_trace<false>, pgrid, blk, 0, st, TraceArgs{w, a, s});
+      if (a.shadows) {
+        NE_MARK(kStageShadow);
+        deliver_last(planned);
+      }
+      a.regen_done = 0;
     }
     if (hv) {
       NE_MARK(kStageMedium);
@@ -1382,48 +1424,23 @@ hipError_t launch_wavefront(const DevScene& s, const DevCamera& cam, WfState& w,
     else if (gh) hipLaunchKernelGGL((k_wf_shade<true, false, false>), grid, blk, 0, st, w, a, s, gh->g);
     else if (sort) hipLaunchKernelGGL((k_wf_shade<false, true, false>), grid, blk, 0, st, w, a, s, WfGuide{});
     else hipLaunchKernelGGL((k_wf_shade<false, false, false>), grid, blk, 0, st, w, a, s, WfGuide{});
-    if (!fuse) NE_MARK(kStageShadow);
-#define NE_SHADOW_SP(CNT, S_, SM)                                                                   \
-  do {                                                                                              \
-    if (spatial) hipLaunchKernelGGL((k_wf_shadow<CNT, S_, true, SM>), grid, blk, 0, st, w, a, s);     \
-    else hipLaunchKernelGGL((k_wf_shadow<CNT, S_, false, SM>), grid, blk, 0, st, w, a, s);          \
-  } while (0)
-#define NE_SHADOW(CNT, S_)                                      \
-  do {                                                          \
-    if (form == kGridQuad) NE_SHADOW_SP(CNT, S_, kGridQuad);        \
-    else if (form == kGridBrick) NE_SHADOW_SP(CNT, S_, kGridBrick); \
-    else NE_SHADOW_SP(CNT, S_, kGridWide);                      \
-  } while (0)
-#define NE_OCCLUDE(FULL)                                                                          \
-  do {                                                                                            \
-    if (count) hipLaunchKernelGGL((k_wf_occlude<true, FULL>), pgrid, blk, 0, st, w, a, s);         \
-    else hipLaunchKernelGGL((k_wf_occlude<false, FULL>), pgrid, blk, 0, st, w, a, s);              \
-  } while (0)
+    if (!fuse && !hs) NE_MARK(kStageShadow);
     if (fuse) {
       // done in the shading stage
-    } else if (hs && hv && (s.n_nodes <= kInlineNodes || NC <= kInlineChunks)) {
-      if (count) NE_SHADOW(true, kSurfInline);
-      else NE_SHADOW(false, kSurfInline);
-    } else if (hs && hv) {
-      NE_OCCLUDE(false);
-      if (count) NE_SHADOW(true, kSurfMarked);
-      else NE_SHADOW(false, kSurfMarked);
     } else if (hs) {
-      NE_OCCLUDE(true);
-      hipLaunchKernelGGL(k_wf_deliver<false>, grid, blk, 0, st, w, a, s);
+      // with the next iteration's paths
     } else if (hv) {
-      if (count) NE_SHADOW(true, kSurfNone);
-      else NE_SHADOW(false, kSurfNone);
+      if (count) NE_SHADOW(true, false, a);
+      else NE_SHADOW(false, false, a);
     } else if (count) {  // neither: nothing is in the way
       hipLaunchKernelGGL(k_wf_deliver<true>, grid, blk, 0, st, w, a, s);
     } else {
       hipLaunchKernelGGL(k_wf_deliver<false>, grid, blk, 0, st, w, a, s);
     }
-#undef NE_SHADOW
-#undef NE_SHADOW_SP
-#undef NE_OCCLUDE
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
+#undef NE_SHADOW
+#undef NE_SHADOW_SP
   NE_MARK(kStageOther);
   if ((e = wf_flush(a, st)) != hipSuccess) return e;
   NE_MARK(kStageEnd);

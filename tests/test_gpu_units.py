@@ -29,7 +29,7 @@ def _scene(which):
         s.add_rectangle(s.add_emitter((4.0, 4.0, 4.0)), position=(0, 0.9, 0), rotation=(-90, 0, 0), scale=(0.5, 0.5, 1))
         s.add_point_light((0.7, 0.1, -0.6), s.add_emitter((0.8, 0.8, 0.6)))
         return s, scenes.VOLUME_CAMERA
-    if which == "mixed_mesh":  # more BVH nodes than are tested inside the tracking stage, but for small pools
+    if which == "mixed_mesh":  # a BVH of many nodes
         s = scenes.small_surface(subdiv=2)
         s.set_volume(configs.fbm_grid(16, 0), 12.0, (0.95,) * 3, (0.05,) * 3, 0.7, maj_res=4)
         return s, scenes.BOX_CAMERA
