@@ -36,18 +36,18 @@ HBM_PEAK_GBS = 8000.0
 PROFILES = ROOT / "profiles"
 
 # Algorithmic bytes per counted event: a trilinear density lookup reads 8 FP32
-# corners, a majorant cell 4 B, a BVH node record 64 B (four quantized child
-# boxes, child references and leaf counts), a primitive record 48 B
-# (triangle: 3 x float4).  Ray-state traffic of the
+# corners, a majorant cell 4 B, a BVH node record 112 B (four child boxes and
+# their work items), a primitive record 48 B (triangle: 3 x float4).  Ray-state traffic of the
 # wavefront stages per ray (structure-of-arrays records):
-#   trace  reads origin + direction (24 B), writes hit t / ref / kind (12 B)
+#   trace  reads origin + direction (24 B), writes hit t / ref / kind (12 B);
+#          it also traverses the last bounce's shadow rays
 #   medium reads origin, direction, hit t, pixel, sample, RNG count (40 B),
 #          writes hit t, kind, RNG count (12 B)
 #   shadow reads the 64 B queue record, read-modify-writes the 12 B radiance
 #   shade  reads the 84 B path record, writes 64 B per continuation and per
 #          shadow ray
 # The film costs 24 B read + 24 B write per pixel (FP64 RGB), once per frame.
-EV = {"density_lookups": 32, "majorant_cells": 4, "bvh_nodes": 64, "prim_tests": 48}
+EV = {"density_lookups": 32, "majorant_cells": 4, "bvh_nodes": 112, "prim_tests": 48}
 RAY_BYTES = {"trace": 36, "medium": 52, "shadow": 88}
 SHADE_IN, SHADE_OUT = 84, 64
 
@@ -69,16 +69,17 @@ def stage_bytes(stage: str, c: dict, film_bytes: int, regen_in_medium: bool = Fa
     if stage == "megakernel":
         return sum(c[k] * b for k, b in EV.items()) + film_bytes
     if stage == "trace":
-        return ext["bvh_nodes"] * EV["bvh_nodes"] + ext["prim_tests"] * 48 + c["ext_rays"] * RAY_BYTES["trace"]
+        return c["bvh_nodes"] * EV["bvh_nodes"] + c["prim_tests"] * 48 + c["ext_rays"] * RAY_BYTES["trace"]
     if stage == "medium":
         return (ext["density_lookups"] * 32 + ext["majorant_cells"] * 4 + c["ext_rays"] * RAY_BYTES["medium"] +
                 (c["paths"] * REGEN_BYTES if regen_in_medium else 0))
+    tracked = sh["density_lookups"] * EV["density_lookups"] + sh["majorant_cells"] * EV["majorant_cells"]
     if stage == "shadow":
-        return sum(sh[k] * b for k, b in EV.items()) + c["shadow_rays"] * RAY_BYTES["shadow"]
+        return tracked + c["shadow_rays"] * RAY_BYTES["shadow"]
     if stage == "shade":
         cont = max(c["ext_rays"] - c["paths"], 0)
         if shadow_in_shade:
-            return c["ext_rays"] * SHADE_IN + cont * SHADE_OUT + sum(sh[k] * b for k, b in EV.items())
+            return c["ext_rays"] * SHADE_IN + cont * SHADE_OUT + tracked
         return c["ext_rays"] * SHADE_IN + (cont + c["shadow_rays"]) * SHADE_OUT
     return 0
 
@@ -971,7 +972,10 @@ def main():
                             "algorithmic_bytes_per_launch": int(b),
                             "achieved_GBs": round(b / (per_launch_ms * 1e-3) / 1e9, 2) if b else None}
         d = stages[dom]
-        kernel = {"megakernel": "k_render", "trace": "k_wf_trace", "medium": "k_wf_medium", "shade": "k_wf_shade",
+        # one launch of whole paths: k_paths where mode AUTO meets a volume without surfaces
+        volume_only = g.info()["bvh_nodes"] == 0 and wl.scene.volume is not None
+        whole = "k_paths" if args.mode == "auto" and volume_only else "k_render"
+        kernel = {"megakernel": whole, "trace": "k_wf_trace", "medium": "k_wf_medium", "shade": "k_wf_shade",
                   "shadow": "k_wf_shadow", "plan": "k_wf_plan", "regen": "k_wf_regen"}.get(dom, dom)
         achieved = d["achieved_GBs"] or 0.0
         roofline = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
