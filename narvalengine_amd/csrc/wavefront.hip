@@ -294,6 +294,9 @@ __global__ __launch_bounds__(kChunk) void k_wf_regen(WfState w, WfArgs a, DevCam
 // A unit is 64 slots of a chunk; its chunk's four units go to the four waves of
 // a block, the chunks blockIdx.x + round * gridDim.x to one block (chunks map to
 // image regions, so interleaving spreads expensive regions over all blocks).
+// With shadow rays the chunks of their queue come first in one numbering, then
+// the paths': in a small pool they go to blocks of their own (frames of one
+// sample, us: 90 x 90 mesh 1000 -> 952, room with a volume 1780 -> 1708).
 // The block's waves take its units in turn from an LDS counter, so a wave holds
 // one unit at a time, in registers, and a refill is a rank in a ballot: against
 // a block-wide queue of single rays, and finished rays stored one by one as they
@@ -304,7 +307,7 @@ __global__ __launch_bounds__(kChunk) void k_wf_regen(WfState w, WfArgs a, DevCam
 struct UnitQueue {
   uint32_t* next;     // the block's next unit (LDS)
   uint32_t nchunks;
-  uint32_t nshadow;   // its units of shadow rays, taken before those of paths
+  uint32_t nshadow;   // chunks of shadow rays, numbered before those of paths
   uint32_t cur, end;  // slots left of the current unit
   bool shadow;        // what the current unit holds
 };
@@ -314,7 +317,7 @@ __device__ __forceinline__ void units_init(UnitQueue& q, uint32_t* next, uint32_
   if (threadIdx.x == 0) *next = 0u;
   q.next = next;
   q.nchunks = nchunks;
-  q.nshadow = shadows ? (nchunks - blockIdx.x + gridDim.x - 1) / gridDim.x * kUnits : 0u;  // gridDim.x <= nchunks
+  q.nshadow = shadows ? nchunks : 0u;
   q.cur = q.end = 0;
   q.shadow = false;
   __syncthreads();
@@ -326,9 +329,9 @@ __device__ __forceinline__ bool units_next(UnitQueue& q, const uint32_t* paths, 
     uint32_t u = 0;
     if (__lane_id() == 0) u = atomicAdd(q.next, 1u);
     u = uniform(u);
-    q.shadow = u < q.nshadow;
-    if (!q.shadow) u -= q.nshadow;
-    const uint32_t c = blockIdx.x + u / kUnits * gridDim.x, lo = u % kUnits * 64;
+    const uint32_t item = blockIdx.x + u / kUnits * gridDim.x, lo = u % kUnits * 64;
+    q.shadow = item < q.nshadow;
+    const uint32_t c = q.shadow ? item : item - q.nshadow;
     if (c >= q.nchunks) return false;
     const uint32_t n = uniform((q.shadow ? shadows : paths)[c]);
     if (n > lo) {
@@ -1256,7 +1259,8 @@ hipError_t launch_wavefront(const DevScene& s, const DevCamera& cam, WfState& w,
   NE_MARK(kStageOther);
   hipLaunchKernelGGL(k_wf_init, dim3((NC + 255) / 256), dim3(256), 0, st, w, NC);
   const dim3 grid = dim3(NC);
-  const dim3 pgrid = dim3(std::min(NC, a.refill_blocks));  // lane-refill kernels: one round of resident blocks
+  // BVH stage: a block per chunk of rays, at most one round of resident blocks
+  auto trace_grid = [&](bool shadows) { return dim3(std::min(shadows ? 2 * NC : NC, a.refill_blocks)); };
   const dim3 blk = dim3(unsigned(kChunk));
   if (!count) a.counters = nullptr;
   const bool hs = s.n_nodes > 0, hv = s.has_volume != 0;
@@ -1325,8 +1329,8 @@ hipError_t launch_wavefront(const DevScene& s, const DevCamera& cam, WfState& w,
           NE_MARK(kStageOther);
           a.shadows = 1;
           a.regen_done = 0;
-          if (count) hipLaunchKernelGGL(k_wf_trace<true>, pgrid, blk, 0, st, TraceArgs{w, a, s});
-          else hipLaunchKernelGGL(k_wf_trace<false>, pgrid, blk, 0, st, TraceArgs{w, a, s});
+          if (count) hipLaunchKernelGGL(k_wf_trace<true>, trace_grid(a.shadows), blk, 0, st, TraceArgs{w, a, s});
+          else hipLaunchKernelGGL(k_wf_trace<false>, trace_grid(a.shadows), blk, 0, st, TraceArgs{w, a, s});
           NE_MARK(kStageShadow);
           deliver_last(false);
         }
@@ -1360,8 +1364,8 @@ hipError_t launch_wavefront(const DevScene& s, const DevCamera& cam, WfState& w,
       NE_MARK(kStageTrace);
       a.shadows = it > 0 ? 1 : 0;
       a.regen_done = planned ? 1 : 0;
-      if (count) hipLaunchKernelGGL(k_wf_trace<true>, pgrid, blk, 0, st, TraceArgs{w, a, s});
-      else hipLaunchKernelGGL(k_wf_trace<false>, pgrid, blk, 0, st, TraceArgs{w, a, s});
+      if (count) hipLaunchKernelGGL(k_wf_trace<true>, trace_grid(a.shadows), blk, 0, st, TraceArgs{w, a, s});
+      else hipLaunchKernelGGL(k_wf_trace<false>, trace_grid(a.shadows), blk, 0, st, TraceArgs{w, a, s});
       if (a.shadows) {
         NE_MARK(kStageShadow);
         deliver_last(planned);
