@@ -150,11 +150,11 @@ enum {
                               FP32, volume-only scenes) the persistent volume path kernel */
   NE_STAGE_PLAN = 1,       /* wavefront: hand out new path ids per chunk (until every path is issued) */
   NE_STAGE_REGEN = 2,      /* wavefront: camera rays into free slots (volume-only scenes: inside MEDIUM) */
-  NE_STAGE_TRACE = 3,      /* wavefront: BVH closest hit */
+  NE_STAGE_TRACE = 3,      /* wavefront: BVH closest hit, and occlusion of the last bounce's shadow rays */
   NE_STAGE_MEDIUM = 4,     /* wavefront: delta tracking */
   NE_STAGE_SHADE = 5,      /* wavefront: emission, NEE sample, scattering, compaction (volume-only
                               scenes without training or counting: also the shadow rays' ratio tracking) */
-  NE_STAGE_SHADOW = 6,     /* wavefront: occlusion + ratio tracking (when not in SHADE) */
+  NE_STAGE_SHADOW = 6,     /* wavefront: ratio tracking and delivery of shadow rays (when not in SHADE) */
   NE_STAGE_OTHER = 7,      /* initialisation, film reduction / flush */
   NE_STAGE_GUIDE = 8,      /* guided wavefront: learned proposal evaluation (MFMA) */
   NE_STAGE_TRAIN = 9,      /* guided wavefront: online training steps */
@@ -181,8 +181,8 @@ typedef struct ne_render_params {
                                  without surfaces, where no flag or pool_size asks for the staged
                                  wavefront, else the staged wavefront; FP64: megakernel) */
   int32_t pool_size;          /* staged wavefront path slots (rounded up to 256); 0 = library default
-                                 (2^23 for surface-only scenes and for renders of 2^28 paths
-                                 or more, else 2^22) */
+                                 (surface-only scenes 2^23, 2^24 for renders of 2^25 paths or
+                                 more; with a volume 2^22, 2^23 for 2^28 paths or more) */
 } ne_render_params;
 
 enum { NE_MODE_AUTO = 0, NE_MODE_MEGAKERNEL = 1, NE_MODE_WAVEFRONT = 2 };
