@@ -759,12 +759,13 @@ struct Walk {
     dd = xf_vec<float>(s.inv, d);
     inv = v3(dd.x != 0.0f ? 1.0f / dd.x : 0.0f, dd.y != 0.0f ? 1.0f / dd.y : 0.0f, dd.z != 0.0f ? 1.0f / dd.z : 0.0f);
   }
-  // box_interval of the ray with the reciprocals above (an infinite one, of
-  // either sign, bounds an axis the same way)
+  // box_interval of the ray with the reciprocals above (that of a direction of
+  // 0 or -0 is infinite with its sign: a ray in a face's plane enters the box or
+  // not by that sign)
   NE_DEV bool box(float& ta, float& te) const {
     float t0 = -xinf<float>(), t1 = xinf<float>();
     auto axis = [&](float o, float d, float i) {
-      const float id = d != 0.0f ? i : xinf<float>();
+      const float id = d != 0.0f ? i : __builtin_copysignf(xinf<float>(), d);
       float tn_ = (-0.5f - o) * id, tf = (0.5f - o) * id;
       if (tn_ > tf) { const float x = tn_; tn_ = tf; tf = x; }
       t0 = tn_ > t0 ? tn_ : t0;

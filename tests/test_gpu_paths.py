@@ -68,3 +68,31 @@ def test_persistent_paths_equal_the_staged_wavefront(ctx, which, form):
         np.testing.assert_array_equal(films[0], films[1], err_msg=f"{w}x{h}x{spp}, {bounces} bounces")
         lit = lit or films[0].any()
     assert lit
+
+
+@pytest.mark.parametrize("axis", [0, 1, 2])
+@pytest.mark.parametrize("side", [-0.5, 0.5])
+@pytest.mark.parametrize("toward", [-1.0, 1.0])
+def test_rays_in_a_face_of_the_volume(ctx, axis, side, toward):
+    """Camera rays that run in a face's plane, parallel to another axis: a
+    direction component of 0 or -0 there has an infinite reciprocal of that
+    sign, and with the origin on the face that sign decides the box test.  A
+    field of view of 1e-9 degrees makes every ray the axis itself."""
+    print_case(f"rays in a face: axis {axis}, side {side}, toward {toward}")
+    from narvalengine_amd import configs
+    from narvalengine_amd.abi import NE_MODE_AUTO, NE_MODE_MEGAKERNEL, NE_MODE_WAVEFRONT
+    from narvalengine_amd.scene import Camera
+    along = (axis + 1) % 3
+    pos, target, up = [0.1, 0.1, 0.1], [0.1, 0.1, 0.1], [0.0, 0.0, 0.0]
+    pos[axis] = target[axis] = side
+    pos[along], target[along] = -2.0 * toward, 0.0
+    up[axis] = 1.0
+    cam = Camera(position=tuple(pos), look_at=tuple(target), up=tuple(up), vfov=1e-9, aspect=1.0)
+    g = ctx.upload(configs.volume_scene(np.ones((8, 8, 8), np.float32), maj_res=2))
+    films = []
+    for mode in (NE_MODE_MEGAKERNEL, NE_MODE_WAVEFRONT, NE_MODE_AUTO):
+        f = ctx.film(16, 16)
+        ctx.render(g, cam, f, spp=16, max_bounces=8, seed=5, mode=mode)
+        films.append(f.read())
+    np.testing.assert_array_equal(films[1], films[2])
+    np.testing.assert_allclose(films[2], films[0], rtol=1e-6, atol=16 * 2.0 ** -30)
