@@ -357,16 +357,18 @@ __global__ __launch_bounds__(kBwdBlock) void k_guide_train_bwd(GuideNet g, Guide
     }
     __syncthreads();
   }
+  // normalised by sum r here: a sum of all samples' unscaled terms leaves FP32's
+  // range where their weights' sum is still in it
+  const float scale = t.loss[1] > 0.0f ? 1.0f / t.loss[1] : 0.0f;
   float* part = t.partial + size_t(blockIdx.x) * kGuideParams;
-  for (int e = int(threadIdx.x); e < KIN * NOUT; e += kBwdBlock) part[guide_w_off(L) + e] = sw[e];
-  if (threadIdx.x < NOUT) part[guide_b_off(L) + threadIdx.x] = sw[KIN * NOUT + threadIdx.x];
+  for (int e = int(threadIdx.x); e < KIN * NOUT; e += kBwdBlock) part[guide_w_off(L) + e] = sw[e] * scale;
+  if (threadIdx.x < NOUT) part[guide_b_off(L) + threadIdx.x] = sw[KIN * NOUT + threadIdx.x] * scale;
 }
 
 // mlp_grad[p] = sum over the backward blocks of the partials, in a fixed order
-// (deterministic), over sum r: a block takes 64 parameters, its 16 thread groups
-// sum the partials w = j mod 16 each, and the group sums are added in order.
+// (deterministic): a block takes 64 parameters, its 16 thread groups sum the
+// partials w = j mod 16 each, and the group sums are added in order.
 __global__ __launch_bounds__(1024) void k_guide_reduce(GuideNet g, GuideTrain t, int parts) {
-  const float scale = t.loss[1] > 0.0f ? 1.0f / t.loss[1] : 0.0f;  // loss normalised by sum r
   __shared__ float part[16][64];
   const int j = int(threadIdx.x >> 6), col = int(threadIdx.x & 63);
   const int p = int(blockIdx.x) * 64 + col;
@@ -379,7 +381,7 @@ __global__ __launch_bounds__(1024) void k_guide_reduce(GuideNet g, GuideTrain t,
   if (j == 0 && p < kGuideParams) {
     float v = part[0][col];
     for (int k = 1; k < 16; ++k) v += part[k][col];
-    g.mlp_grad[p] = v * scale;
+    g.mlp_grad[p] = v;
   }
 }
 

@@ -419,3 +419,37 @@ def test_tabulated_guided_render_is_unbiased(ctx):
     assert abs(z) < 5.0, (z, a.mean(), b.mean())
     assert abs(b.mean() - a.mean()) < 0.03 * a.mean()
     g.close()
+
+
+@pytest.mark.parametrize("n", [4096, 65536])
+def test_guide_gradients_do_not_depend_on_the_weights_scale(ctx, n):
+    """The loss is normalised by the weights' sum: weights times 2^k give the
+    same gradients, bit for bit as long as nothing leaves FP32's range.  k is
+    taken so that the weights' sum is just below 2^124 while the gradients are
+    above 16, so a sum over all samples before the normalisation would
+    overflow."""
+    print_case(f"guide gradients: {n} samples of large weights")
+    g = Guide(ctx, log2_table=LOG2T, batch=n, seed=1)
+    table, mlp = _random_params(g, 5)
+    rng = np.random.default_rng(n)
+    # short mean vectors, so that the loss is steep in them: d/d(mean) ~ kappa / |mean|
+    last = mlp[G.W_OFF[4]:G.W_OFF[5]]
+    last *= 1e-4
+    b = mlp[G.B_OFF[4]:G.B_OFF[4] + 40].reshape(8, 5)
+    b[:, 0] = 0.0
+    b[:, 1:4] = rng.normal(size=(8, 3)) * 0.005
+    b[:, 4] = 0.5
+    g.set_params(table, mlp)
+    w = np.array([0.3, 0.8, 0.5]) + 0.2 * rng.normal(size=(n, 3))
+    w /= np.linalg.norm(w, axis=1, keepdims=True)
+    s = np.concatenate([_queries(n, n + 1), w, rng.uniform(0.5, 1.0, (n, 1))], 1).astype(np.float32)
+    loss = g.train_step(s, update=False)
+    gt, gm = g.grads()
+    assert np.isfinite(gm).all() and np.abs(gm).max() > 16.0, np.abs(gm).max()
+    assert gt.any()
+    s[:, 9] *= np.float32(2.0) ** (124 - int(np.log2(n)))
+    assert g.train_step(s, update=False) == loss
+    ht, hm = g.grads()
+    np.testing.assert_array_equal(hm, gm)
+    np.testing.assert_array_equal(ht, gt)
+    g.close()
