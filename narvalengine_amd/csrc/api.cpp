@@ -2054,7 +2054,7 @@ ne_status ne_guide_create(ne_ctx* c, const ne_guide_config* cfg_in, ne_guide** o
             guide_alloc(g, t.dy, cap * kGuideWidth) && guide_alloc(g, t.dy2, cap * kGuideWidth) &&
             guide_alloc(g, t.denc, cap * kGuideEnc) && guide_alloc(g, t.partial, size_t(t.parts) * kGuideParams) &&
             guide_alloc(g, t.loss, 2) && guide_alloc(g, t.loss_part, 2 * size_t(kGuideFwdBlocks)) && guide_alloc(g, t.aos, 10 * cap);
-  if (ok && guide_table_chunks(n) > 1) ok = guide_alloc(g, t.table_part, size_t(guide_table_chunks(n)) * g->table_n);
+  if (const size_t floats = ok ? guide_table_part(n) : 0) ok = guide_alloc(g, t.table_part, floats);
   if (ok && cfg.cache_res > 0) {
     const size_t entries = size_t(cfg.cache_res) * cfg.cache_res * cfg.cache_res * size_t(cfg.cache_dirs) * cfg.cache_dirs;
     ok = guide_alloc(g, g->cache_mix, entries * 40);

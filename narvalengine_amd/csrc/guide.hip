@@ -395,8 +395,9 @@ __global__ __launch_bounds__(1024) void k_guide_reduce(GuideNet g, GuideTrain t,
 // a wave: ds_add_f64 21 cycles, ds_add_f32 194).  A sample is read by every
 // block of its level, but only the blocks that own one of its corners work on
 // it: tables of more ranges than the chip has CUs take all samples in every
-// block; smaller ones split the samples into `chunks` and sum the chunks'
-// copies after (k_guide_table_sum).  The whole training pass with its copies,
+// block; smaller ones split the samples into `chunks`, each with a copy of the
+// ranges (t.table_part, 64 KiB per range and chunk: at most 16 MiB, as chunks x
+// ranges fill the chip once), and sum the copies after (k_guide_table_sum).  The whole training pass with its copies,
 // 65,536 samples, this kernel against atomics at every level, us:
 // log2_table 15: 488 / 1306, 17: 648 / 1292, 19: 658 / 1301, 21: 971 / 1360;
 // 8192 samples: 15: 316 / 454, 21: 279 / 333.  Atomics for the large levels
@@ -409,12 +410,9 @@ __host__ __device__ inline uint32_t guide_level_entries(const GuideNet& g, int l
   const uint64_t dense = uint64_t(r1) * r1 * r1;
   return dense <= T ? uint32_t(dense) : T;
 }
-__global__ __launch_bounds__(kTableBlock) void k_guide_table_grad(GuideNet g, GuideBatch b, GuideTrain t, int chunks,
-                                                                  float* out, size_t stride) {
-  __shared__ double acc[2 * kTableRange];
-  // blockIdx -> level, range of the level, chunk of the samples
-  uint32_t unit = blockIdx.x / uint32_t(chunks), chunk = blockIdx.x % uint32_t(chunks);
-  int l = 0;
+// Range `unit` of the ranges of all levels: its level, first entry and length.
+__device__ inline void guide_table_range(const GuideNet& g, uint32_t unit, int& l, uint32_t& base, uint32_t& len) {
+  l = 0;
   uint32_t ent = guide_level_entries(g, 0), nr = (ent + kTableRange - 1) / kTableRange;
   while (unit >= nr) {
     unit -= nr;
@@ -422,7 +420,15 @@ __global__ __launch_bounds__(kTableBlock) void k_guide_table_grad(GuideNet g, Gu
     ent = guide_level_entries(g, l);
     nr = (ent + kTableRange - 1) / kTableRange;
   }
-  const uint32_t base = unit * kTableRange, len = ent - base < kTableRange ? ent - base : kTableRange;
+  base = unit * kTableRange;
+  len = ent - base < kTableRange ? ent - base : kTableRange;
+}
+__global__ __launch_bounds__(kTableBlock) void k_guide_table_grad(GuideNet g, GuideBatch b, GuideTrain t, int chunks) {
+  __shared__ double acc[2 * kTableRange];
+  const uint32_t unit = blockIdx.x / uint32_t(chunks), chunk = blockIdx.x % uint32_t(chunks);
+  int l;
+  uint32_t base, len;
+  guide_table_range(g, unit, l, base, len);
   for (uint32_t k = threadIdx.x; k < 2 * len; k += kTableBlock) acc[k] = 0.0;
   __syncthreads();
   const float scale = t.loss[1] > 0.0f ? 1.0f / t.loss[1] : 0.0f;
@@ -460,21 +466,26 @@ __global__ __launch_bounds__(kTableBlock) void k_guide_table_grad(GuideNet g, Gu
     }
   }
   __syncthreads();
-  float2* o = reinterpret_cast<float2*>(out + size_t(chunk) * stride) + size_t(l) * T + base;
+  float2* o = chunks == 1 ? reinterpret_cast<float2*>(g.table_grad) + size_t(l) * T + base
+                          : reinterpret_cast<float2*>(t.table_part) + size_t(blockIdx.x) * kTableRange;
   for (uint32_t k = threadIdx.x; k < len; k += kTableBlock) o[k] = make_float2(float(acc[2 * k]), float(acc[2 * k + 1]));
 }
-// table_grad = the chunks' copies summed in order, over the entries the levels address
-__global__ __launch_bounds__(256) void k_guide_table_sum(GuideNet g, const float* part, size_t stride, int chunks) {
-  const uint32_t T = 1u << g.log2T;
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x, l = i >> g.log2T, k = i & (T - 1u);
-  if (l >= uint32_t(kGuideLevels) || k >= guide_level_entries(g, int(l))) return;
-  float2 s = reinterpret_cast<const float2*>(part)[i];
+// table_grad = the chunks' copies of each range summed in order.
+__global__ __launch_bounds__(256) void k_guide_table_sum(GuideNet g, const float* part, int chunks) {
+  int l;
+  uint32_t base, len;
+  constexpr uint32_t kBlocks = kTableRange / 256;  // per range
+  const uint32_t unit = blockIdx.x / kBlocks, k = blockIdx.x % kBlocks * 256u + threadIdx.x;
+  guide_table_range(g, unit, l, base, len);
+  if (k >= len) return;
+  const float2* p = reinterpret_cast<const float2*>(part) + size_t(unit) * uint32_t(chunks) * kTableRange + k;
+  float2 s = p[0];
   for (int c = 1; c < chunks; ++c) {
-    const float2 v = reinterpret_cast<const float2*>(part + size_t(c) * stride)[i];
+    const float2 v = p[size_t(c) * kTableRange];
     s.x += v.x;
     s.y += v.y;
   }
-  reinterpret_cast<float2*>(g.table_grad)[i] = s;
+  reinterpret_cast<float2*>(g.table_grad)[(size_t(l) << g.log2T) + base + k] = s;
 }
 
 // BF16 copy of the hash features that the encoder reads (after every change
@@ -600,9 +611,11 @@ static int table_units(const GuideNet& g) {
   return units;
 }
 // Chunks of the samples in the table gradient: as many as fill the chip once
-// (256 CUs, one block each), at most kGuideTableChunks.
-int guide_table_chunks(const GuideNet& g) {
-  return std::min(kGuideTableChunks, std::max(1, 256 / table_units(g)));
+// (256 CUs, one block each), at most 16.
+static int table_chunks(const GuideNet& g) { return std::min(16, std::max(1, 256 / table_units(g))); }
+size_t guide_table_part(const GuideNet& g) {
+  const int chunks = table_chunks(g);
+  return chunks == 1 ? 0 : size_t(table_units(g)) * chunks * kTableRange * kGuideFeat;
 }
 
 // Gradients of the weight-normalised loss -sum r log q / sum r (1 / sum r is
@@ -620,13 +633,11 @@ hipError_t launch_guide_grad(const GuideNet& g, const GuideBatch& b, const Guide
   hipLaunchKernelGGL((k_guide_train_bwd<1>), dim3(blocks), blk, 0, st, g, b, t, t.dy2, t.dy);
   hipLaunchKernelGGL((k_guide_train_bwd<0>), dim3(blocks), blk, 0, st, g, b, t, t.dy, t.dy2);
   hipLaunchKernelGGL(k_guide_reduce, dim3((kGuideParams + 63) / 64), dim3(1024), 0, st, g, t, int(blocks));
-  const int chunks = guide_table_chunks(g);
-  const size_t words = table_words(g);
-  float* out = chunks == 1 ? g.table_grad : t.table_part;
-  hipLaunchKernelGGL(k_guide_table_grad, dim3(uint32_t(table_units(g) * chunks)), dim3(kTableBlock), 0, st, g, b, t,
-                     chunks, out, words);
+  const uint32_t units = uint32_t(table_units(g));
+  const int chunks = table_chunks(g);
+  hipLaunchKernelGGL(k_guide_table_grad, dim3(units * uint32_t(chunks)), dim3(kTableBlock), 0, st, g, b, t, chunks);
   if (chunks > 1)
-    hipLaunchKernelGGL(k_guide_table_sum, dim3(uint32_t((words / 2 + 255) / 256)), dim3(256), 0, st, g, out, words, chunks);
+    hipLaunchKernelGGL(k_guide_table_sum, dim3(units * (kTableRange / 256)), dim3(256), 0, st, g, t.table_part, chunks);
   return hipGetLastError();
 }
 

@@ -254,12 +254,11 @@ struct GuideTrain {
   float* loss;         // [0] summed loss, [1] summed weight
   float* loss_part;    // the same per forward block
   float* aos;          // samples as the caller gave them (10 floats each)
-  float* table_part;   // table gradient per chunk of the samples (guide_table_chunks > 1)
+  float* table_part;   // table gradient per chunk of the samples (guide_table_part floats)
   int32_t parts;       // backward blocks at most
 };
 constexpr uint32_t kGuideFwdBlocks = 8192;
-constexpr int kGuideTableChunks = 16;
-int guide_table_chunks(const GuideNet& g);  // copies of the table gradient that a step keeps
+size_t guide_table_part(const GuideNet& g);  // floats of table_part; 0: the samples are not split
 
 // Guided wavefront: per-path training record (one per slot and path buffer).
 // state 0: none; 1: a guided vertex was sampled, the radiance baseline is

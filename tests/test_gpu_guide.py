@@ -453,3 +453,36 @@ def test_guide_gradients_do_not_depend_on_the_weights_scale(ctx, n):
     np.testing.assert_array_equal(hm, gm)
     np.testing.assert_array_equal(ht, gt)
     g.close()
+
+
+@pytest.mark.parametrize("log2_table,max_res", [(20, 16), (22, 8), (14, 512)])
+def test_guide_gradients_of_levels_that_use_little_of_their_table(ctx, log2_table, max_res):
+    """Dense levels smaller than the table: the copies of the table's gradient
+    that a step keeps hold the entries in use alone (at most 16 MiB), and the
+    sums are the reference network's."""
+    from hipmem import free_bytes
+    print_case(f"guide gradients: log2_table {log2_table}, levels up to {max_res}")
+    n = 1000
+    ctx.synchronize()
+    before = free_bytes()
+    g = Guide(ctx, log2_table=log2_table, base_res=4, max_res=max_res, batch=1024, seed=1)
+    used = before - free_bytes()
+    # the table, its gradient and Adam's two moments in FP32, the BF16 copy; the
+    # network's partial sums are 512 x 19.7 k floats
+    assert used < 4.5 * 4 * g.table_floats + 512 * 4 * g.mlp_floats + (32 << 20), used
+    table, mlp = _random_params(g, 5)
+    g.set_params(table, mlp)
+    rng = np.random.default_rng(n)
+    w = rng.normal(size=(n, 3))
+    w /= np.linalg.norm(w, axis=1, keepdims=True)
+    s = np.concatenate([_queries(n, n + 1), w, rng.uniform(0.1, 2.0, (n, 1))], 1).astype(np.float32)
+    loss = g.train_step(s, update=False)
+    gt, gm = g.grads()
+    rl, rt, rm = G.loss_and_grad(s, table, mlp, g.level_res, log2_table, quantize=True)
+    assert abs(loss - rl) < 1e-3 * abs(rl) + 1e-4, (loss, rl)
+    for got, ref in ((gm, rm), (gt, rt)):
+        cos = got @ ref / (np.linalg.norm(got) * np.linalg.norm(ref))
+        rel = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+        assert cos > 0.995 and rel < 0.08, (cos, rel)
+    assert not gt[rt == 0.0].any()
+    g.close()
