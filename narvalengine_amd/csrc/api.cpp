@@ -945,16 +945,17 @@ ne_status ne_film_tonemap(ne_film* f, int32_t spp, float* pixels) {
 constexpr size_t kMaxSampleBuffer = size_t(16) << 30;
 
 // Default wavefront pool (slots) for a render of `total` paths, measured on
-// MI355X.  Surface-only scenes: fewer, larger BVH launches amortise each
-// launch's tail, 2^24 slots for renders of 2^25 paths and more, else 2^23
-// (surface1m, ms at 2^23 / 2^24 slots: 16 spp 25.0 / 25.8, 32 spp 45.3 / 44.3,
-// 64 spp 84.5 / 81.0).  With a volume 2^22, where a larger pool adds
-// cache pressure, except for long renders (2^28 paths and more, e.g. the
+// MI355X: 2^23 for surface-only scenes, where fewer, larger BVH launches
+// amortise each launch's tail (2^24 slots take twice the memory and more time on
+// most renders, ms at 2^23 / 2^24: 1024x1024 x 32 spp of an icosphere of 5 k
+// triangles 35.2 / 37.5, 82 k 38.5 / 40.6, 1.3 M 42.9 / 44.8; x 128 spp 133.4 /
+// 134.5, 144.8 / 144.5, 160.2 / 157.0).  With a volume 2^22, where a larger pool
+// adds cache pressure, except for long renders (2^28 paths and more, e.g. the
 // 1920x1080 cloud at 256 spp), whose iterations' fixed costs (launches, the
 // plan scan) halve with 2^23 slots: 236.4 -> 231.5 ms per cloud frame, while
 // a 512^2 x 64-spp volume frame took 12.0 ms at 2^22 and 13.4 ms at 2^23.
 static uint64_t default_pool(const DevScene& ds, uint64_t total) {
-  if (ds.n_nodes > 0 && !ds.has_volume) return uint64_t(1) << (total >= (uint64_t(1) << 25) ? 24 : 23);
+  if (ds.n_nodes > 0 && !ds.has_volume) return uint64_t(1) << 23;
   return total >= (uint64_t(1) << 28) ? (uint64_t(1) << 23) : (uint64_t(1) << 22);
 }
 
