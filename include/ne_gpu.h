@@ -209,7 +209,8 @@ typedef struct ne_scene_info {
   uint32_t bvh_depth;
   uint32_t bvh_leaf_prims_max;
   uint32_t maj_res;
-  uint64_t device_bytes;
+  uint64_t device_bytes;   /* held now: a density grid's quad copy is given back where another
+                              allocation of the context needs its room */
   float grid_max_density;
   float pad;
 } ne_scene_info;

@@ -58,6 +58,7 @@ struct ne_ctx {
   char* stage_dev = nullptr;    // its device address
   hipEvent_t stage_ev[2] = {nullptr, nullptr};
   size_t stage_in = 0;          // bytes of the inputs' part that copies in flight may read
+  std::vector<ne_scene*> quad_scenes;  // scenes that hold quads (under mu)
 };
 
 struct ne_scene {
@@ -65,6 +66,8 @@ struct ne_scene {
   DevScene dev{};
   std::vector<void*> allocs;
   uint64_t bytes = 0;
+  void* quads = nullptr;  // the density's quad copy (dev.quad), or null
+  size_t quad_bytes = 0;
   ne_scene_info info{};
 };
 
@@ -139,13 +142,47 @@ ne_status fail(ne_ctx* c, ne_status st, const std::string& msg) {
                   std::string(#call) + ": " + hipGetErrorString(e_));                             \
   } while (0)
 
+// Gives back the quads of the context's scenes, whose lookups then read the
+// bricks; false if there were none.  Called under mu, where no kernel but those
+// of c->stream reads a scene.
+bool release_quads(ne_ctx* c) {
+  if (c->quad_scenes.empty()) return false;
+  (void)hipStreamSynchronize(c->stream);
+  for (ne_scene* s : c->quad_scenes) {
+    (void)hipFree(s->quads);
+    s->quads = nullptr;
+    s->dev.quad = nullptr;
+    s->dev.grid_form = kGridBrick;
+    s->bytes -= s->quad_bytes;
+    s->info.device_bytes = s->bytes;
+  }
+  c->quad_scenes.clear();
+  return true;
+}
+
+// Device memory for everything but the quads: those are copies (four times the
+// bricks) that a lookup can do without, so they make room for what finds none.
+// A scene's DevScene is read after the allocations of the call that uses it.
+template <class T>
+hipError_t dev_alloc(ne_ctx* c, T** p, size_t bytes) {
+  void* q = nullptr;
+  hipError_t e = hipMalloc(&q, bytes);
+  if (e != hipSuccess) (void)hipGetLastError();  // (the next launch would report it again)
+  if (e == hipErrorOutOfMemory && release_quads(c)) {
+    e = hipMalloc(&q, bytes);
+    if (e != hipSuccess) (void)hipGetLastError();
+  }
+  if (e == hipSuccess) *p = static_cast<T*>(q);
+  return e;
+}
+
 template <class T>
 ne_status dev_upload(ne_ctx* c, ne_scene* s, const T* src, size_t count, const T** dst) {
   *dst = nullptr;
   if (count == 0) return NE_OK;
   void* p = nullptr;
   size_t bytes = count * sizeof(T);
-  NE_HIP(c, hipMalloc(&p, bytes));
+  NE_HIP(c, dev_alloc(c, &p, bytes));
   s->allocs.push_back(p);
   s->bytes += bytes;
   NE_HIP(c, hipMemcpyAsync(p, src, bytes, hipMemcpyHostToDevice, c->stream));
@@ -218,7 +255,7 @@ struct DevBuf {
 template <class T>
 ne_status tmp_in(ne_ctx* c, DevBuf& b, const T* src, size_t count) {
   if (count == 0 || src == nullptr) return NE_OK;
-  NE_HIP(c, hipMalloc(&b.p, count * sizeof(T)));
+  NE_HIP(c, dev_alloc(c, &b.p, count * sizeof(T)));
   const void* from = src;
   if (char* p = stage_input(c, count * sizeof(T))) from = std::memcpy(p, src, count * sizeof(T));
   NE_HIP(c, hipMemcpyAsync(b.p, from, count * sizeof(T), hipMemcpyHostToDevice, c->stream));
@@ -226,7 +263,7 @@ ne_status tmp_in(ne_ctx* c, DevBuf& b, const T* src, size_t count) {
 }
 template <class T>
 ne_status tmp_out(ne_ctx* c, DevBuf& b, size_t count) {
-  NE_HIP(c, hipMalloc(&b.p, std::max<size_t>(count, 1) * sizeof(T)));
+  NE_HIP(c, dev_alloc(c, &b.p, std::max<size_t>(count, 1) * sizeof(T)));
   return NE_OK;
 }
 template <class T>
@@ -579,18 +616,16 @@ ne_status ne_synchronize(ne_ctx* c) {
   return NE_OK;
 }
 
-ne_status ne_scene_upload(ne_ctx* c, const ne_scene_desc* d, ne_scene** out) {
-  if (!c || !out) return fail(c, NE_ERR_INVALID_ARG, "ctx/out is NULL");
-  *out = nullptr;
-  std::lock_guard<std::mutex> lk(c->mu);
-  ne_status st = validate_desc(c, d);
-  if (st != NE_OK) return st;
-  NE_HIP(c, hipSetDevice(c->device));
+// The scene of a valid description on the device; quads: whether the density may
+// have its quad copy.
+static ne_status upload_scene(ne_ctx* c, const ne_scene_desc* d, bool quads, ne_scene** out) {
+  ne_status st = NE_OK;
   ne_scene* s = new ne_scene();
   s->ctx = c;
   auto bail = [&](ne_status e) {
     (void)hipStreamSynchronize(c->stream);
     for (void* p : s->allocs) (void)hipFree(p);
+    if (s->quads) (void)hipFree(s->quads);
     delete s;
     return e;
   };
@@ -743,11 +778,11 @@ ne_status ne_scene_upload(ne_ctx* c, const ne_scene_desc* d, ne_scene** out) {
       const uint32_t px = grid_pad_x(ds.res[0]), py = grid_pad_y(ds.res[1]), pz = grid_pad_z(ds.res[2]);
       const size_t nb = (size_t(px) * py * pz + kBrickFloats) * sizeof(float);
       DevBuf lin;
-      NE_HIP_BAIL(hipMalloc(&lin.p, nvox * sizeof(float)));
+      NE_HIP_BAIL(dev_alloc(c, &lin.p, nvox * sizeof(float)));
       NE_HIP_BAIL(hipMemcpyAsync(lin.p, homog ? &kOne : d->grid, nvox * sizeof(float), hipMemcpyHostToDevice,
                                  c->stream));
       void* pg = nullptr;
-      NE_HIP_BAIL(hipMalloc(&pg, nb));
+      NE_HIP_BAIL(dev_alloc(c, &pg, nb));
       s->allocs.push_back(pg);
       s->bytes += nb;
       NE_HIP_BAIL(hipMemsetAsync(pg, 0, nb, c->stream));
@@ -760,24 +795,24 @@ ne_status ne_scene_upload(ne_ctx* c, const ne_scene_desc* d, ne_scene** out) {
       // the quads: four times the memory; without room for them the bricks serve
       const uint32_t qx = quad_pad(ds.res[0]), qy = quad_pad(ds.res[1]), qz = quad_pad_z(ds.res[2]);
       const uint64_t qstep = uint64_t(qx / 2u) * (qy / 2u) * 8u, qbytes = qstep * (qz / 2u) * sizeof(float4);
-      void* pq = nullptr;
-      if (ds.grid_form == kGridBrick && qbytes < (uint64_t(1) << 32) && qstep < (1u << 24)) {
-        if (hipMalloc(&pq, qbytes) == hipSuccess) {
-          s->allocs.push_back(pq);
+      if (quads && ds.grid_form == kGridBrick && qbytes < (uint64_t(1) << 32) && qstep < (1u << 24)) {
+        if (hipMalloc(&s->quads, qbytes) == hipSuccess) {
+          s->quad_bytes = qbytes;
           s->bytes += qbytes;
-          NE_HIP_BAIL(launch_quad_grid(ds, static_cast<float4*>(pq), c->stream));
-          ds.quad = static_cast<const float4*>(pq);
+          NE_HIP_BAIL(launch_quad_grid(ds, static_cast<float4*>(s->quads), c->stream));
+          ds.quad = static_cast<const float4*>(s->quads);
           ds.quad_step_y = (qx / 2u) * 8u;
           ds.quad_step_z = uint32_t(qstep);
           ds.grid_form = kGridQuad;
         } else {
+          s->quads = nullptr;
           (void)hipGetLastError();
         }
       }
     }
     size_t ncell = size_t(ds.mres) * ds.mres * ds.mres;
     void* pm = nullptr;
-    NE_HIP_BAIL(hipMalloc(&pm, ncell * sizeof(float)));
+    NE_HIP_BAIL(dev_alloc(c, &pm, ncell * sizeof(float)));
     s->allocs.push_back(pm);
     s->bytes += ncell * sizeof(float);
     NE_HIP_BAIL(launch_majorants(ds, static_cast<float*>(pm), c->stream));
@@ -822,7 +857,7 @@ ne_status ne_scene_upload(ne_ctx* c, const ne_scene_desc* d, ne_scene** out) {
         mp[i] = make_float2(v, v > 0.0f && std::isfinite(v) ? 1.0f / v : 0.0f);
       }
       void* pp = nullptr;
-      NE_HIP_BAIL(hipMalloc(&pp, ncell * sizeof(float2)));
+      NE_HIP_BAIL(dev_alloc(c, &pp, ncell * sizeof(float2)));
       s->allocs.push_back(pp);
       s->bytes += ncell * sizeof(float2);
       NE_HIP_BAIL(hipMemcpyAsync(pp, mp.data(), ncell * sizeof(float2), hipMemcpyHostToDevice, c->stream));
@@ -854,11 +889,25 @@ ne_status ne_scene_upload(ne_ctx* c, const ne_scene_desc* d, ne_scene** out) {
   s->info.maj_res = uint32_t(d->has_volume ? ds.mres : 0);
   s->info.device_bytes = s->bytes;
   s->info.grid_max_density = gmax;
+  if (s->quads) c->quad_scenes.push_back(s);
   c->refs.fetch_add(1);
   *out = s;
   return NE_OK;
 }
 #undef NE_HIP_BAIL
+
+ne_status ne_scene_upload(ne_ctx* c, const ne_scene_desc* d, ne_scene** out) {
+  if (!c || !out) return fail(c, NE_ERR_INVALID_ARG, "ctx/out is NULL");
+  *out = nullptr;
+  std::lock_guard<std::mutex> lk(c->mu);
+  ne_status st = validate_desc(c, d);
+  if (st != NE_OK) return st;
+  NE_HIP(c, hipSetDevice(c->device));
+  st = upload_scene(c, d, true, out);
+  // its own quads may have taken what the rest of it needed
+  if (st == NE_ERR_OUT_OF_MEMORY && d->has_volume) st = upload_scene(c, d, false, out);
+  return st;
+}
 
 void ne_scene_release(ne_scene* s) {
   if (!s) return;
@@ -868,6 +917,10 @@ void ne_scene_release(ne_scene* s) {
     (void)hipSetDevice(c->device);
     (void)hipStreamSynchronize(c->stream);
     for (void* p : s->allocs) (void)hipFree(p);
+    if (s->quads) {
+      (void)hipFree(s->quads);
+      c->quad_scenes.erase(std::find(c->quad_scenes.begin(), c->quad_scenes.end(), s));
+    }
     delete s;
   }
   ctx_unref(c);
@@ -875,6 +928,7 @@ void ne_scene_release(ne_scene* s) {
 
 ne_status ne_scene_get_info(const ne_scene* s, ne_scene_info* out) {
   if (!s || !out) return fail(nullptr, NE_ERR_INVALID_ARG, "scene/out is NULL");
+  std::lock_guard<std::mutex> lk(s->ctx->mu);  // (its device bytes change where its quads make room)
   *out = s->info;
   return NE_OK;
 }
@@ -888,7 +942,7 @@ ne_status ne_film_create(ne_ctx* c, int32_t w, int32_t h, ne_film** out) {
   ne_film* f = new ne_film();
   f->ctx = c; f->W = w; f->H = h;
   size_t bytes = size_t(w) * h * 3 * sizeof(double);
-  hipError_t e = hipMalloc(&f->d_sum, bytes);
+  hipError_t e = dev_alloc(c, &f->d_sum, bytes);
   if (e != hipSuccess) { delete f; return fail(c, NE_ERR_OUT_OF_MEMORY, "film allocation failed"); }
   e = hipMemsetAsync(f->d_sum, 0, bytes, c->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
@@ -993,13 +1047,13 @@ static ne_status render_wavefront(ne_ctx* c, const ne_scene* s, const DevCamera&
       NE_HIP(c, hipFree(old));
     }
     void* nb = nullptr;
-    NE_HIP(c, hipMalloc(&nb, wf_bytes(uint32_t(P))));
+    NE_HIP(c, dev_alloc(c, &nb, wf_bytes(uint32_t(P))));
     c->wf_buf = nb;
     c->wf_P = uint32_t(P);
   }
   if (!f->d_fixed) {
     const size_t bytes = size_t(f->W) * f->H * 3 * sizeof(long long);
-    NE_HIP(c, hipMalloc(&f->d_fixed, bytes));
+    NE_HIP(c, dev_alloc(c, &f->d_fixed, bytes));
     NE_HIP(c, hipMemsetAsync(f->d_fixed, 0, bytes, c->stream));
   }
   WfArgs a{};
@@ -1034,7 +1088,7 @@ static ne_status render_wavefront(ne_ctx* c, const ne_scene* s, const DevCamera&
       c->sbuf_bytes = 0;
       if (old) NE_HIP(c, hipFree(old));
       void* nb = nullptr;
-      if (hipMalloc(&nb, sbytes) == hipSuccess) {
+      if (dev_alloc(c, &nb, sbytes) == hipSuccess) {
         c->sbuf = nb;
         c->sbuf_bytes = sbytes;
       } else {
@@ -1051,7 +1105,7 @@ static ne_status render_wavefront(ne_ctx* c, const ne_scene* s, const DevCamera&
       gu.max_depth = gh->g.max_depth;
       gu.prob = gh->g.prob;
     }
-    if (!c->paths_scratch) NE_HIP(c, hipMalloc(&c->paths_scratch, paths_scratch_bytes(c->cus)));
+    if (!c->paths_scratch) NE_HIP(c, dev_alloc(c, &c->paths_scratch, paths_scratch_bytes(c->cus)));
     if (timed) NE_HIP(c, hipEventRecord(c->ev0, c->stream));
     NE_HIP(c, launch_paths(s->dev, dc, a, gu, c->paths_scratch, c->cus, c->stream, tm));
     if (timed) {
@@ -1072,7 +1126,7 @@ static ne_status render_wavefront(ne_ctx* c, const ne_scene* s, const DevCamera&
         NE_HIP(c, hipFree(old));
       }
       void* nb = nullptr;
-      NE_HIP(c, hipMalloc(&nb, wf_guide_bytes(uint32_t(P))));
+      NE_HIP(c, dev_alloc(c, &nb, wf_guide_bytes(uint32_t(P))));
       c->wfg_buf = nb;
       c->wfg_P = uint32_t(P);
     }
@@ -1164,7 +1218,7 @@ static ne_status render_locked(ne_ctx* c, const ne_scene* s, const ne_camera_des
         NE_HIP(c, hipFree(old));
       }
       void* nb = nullptr;
-      NE_HIP(c, hipMalloc(&nb, need));
+      NE_HIP(c, dev_alloc(c, &nb, need));
       c->d_partial = static_cast<decltype(c->d_partial)>(nb);
       c->partial_bytes = need;
     }
@@ -1565,7 +1619,6 @@ ne_status batch_prepare(ne_batch* b, const ne_batch_config& cfg, int div) {
   for (size_t j = 0; j < b->jobs.size(); ++j) {
     const ne_job& J = b->jobs[j];
     BatchJob& T = table[j];
-    T.scene = J.scene->dev;
     T.cam = make_camera(&J.camera);
     T.W = J.width; T.H = J.height;
     T.spp = (J.spp + div - 1) / div;
@@ -1592,10 +1645,11 @@ ne_status batch_prepare(ne_batch* b, const ne_batch_config& cfg, int div) {
     if (old_times) NE_HIP(c, hipFree(old_times));
     if (old_exec) NE_HIP(c, hipGraphExecDestroy(old_exec));
     void* p = nullptr;
-    NE_HIP(c, hipMalloc(&p, items * sizeof(unsigned long long)));
+    NE_HIP(c, dev_alloc(c, &p, items * sizeof(unsigned long long)));
     b->d_item_time = static_cast<unsigned long long*>(p);
     b->item_cap = items;
   }
+  for (size_t j = 0; j < b->jobs.size(); ++j) table[j].scene = b->jobs[j].scene->dev;
   NE_HIP(c, hipMemcpyAsync(b->d_jobs, table.data(), table.size() * sizeof(BatchJob), hipMemcpyHostToDevice,
                            c->stream));
   const bool same = b->exec && b->exec_div == div && b->exec_cfg.tile_w == cfg.tile_w &&
@@ -1769,14 +1823,14 @@ ne_status batch_run_lanes(ne_batch* b, int div, float* ms) {
   }
   for (int i = 0; i < nl; ++i) {
     BatchLane& L = b->lanes[i];
-    if (paths && !L.paths_scratch) NE_HIP(c, hipMalloc(&L.paths_scratch, paths_scratch_bytes(c->cus)));
+    if (paths && !L.paths_scratch) NE_HIP(c, dev_alloc(c, &L.paths_scratch, paths_scratch_bytes(c->cus)));
     if (Pmax > L.pool_P) {
       void* old = L.pool;
       L.pool = nullptr;
       L.pool_P = 0;
       if (old) NE_HIP(c, hipFree(old));
       void* nb = nullptr;
-      NE_HIP(c, hipMalloc(&nb, wf_bytes(uint32_t(Pmax))));
+      NE_HIP(c, dev_alloc(c, &nb, wf_bytes(uint32_t(Pmax))));
       L.pool = nb;
       L.pool_P = uint32_t(Pmax);
     }
@@ -1786,7 +1840,7 @@ ne_status batch_run_lanes(ne_batch* b, int div, float* ms) {
       L.sbuf_bytes = 0;
       if (old) NE_HIP(c, hipFree(old));
       void* nb = nullptr;
-      NE_HIP(c, hipMalloc(&nb, sbytes));
+      NE_HIP(c, dev_alloc(c, &nb, sbytes));
       L.sbuf = nb;
       L.sbuf_bytes = sbytes;
     }
@@ -1885,10 +1939,10 @@ ne_status ne_batch_create(ne_ctx* c, const ne_job* jobs, int32_t n, ne_batch** o
     return bail(fail(c, NE_ERR_HIP, "device attribute query failed"));
   b->grid_blocks = uint32_t(std::max(1, cus * std::max(1, per_cu)));
   b->ticks_per_ms = double(khz);
-  if (hipMalloc(&b->d_films, b->film_words * sizeof(long long)) != hipSuccess ||
-      hipMalloc(&b->d_jobs, size_t(n) * sizeof(BatchJob)) != hipSuccess ||
-      hipMalloc(&b->d_misc, 2 * sizeof(unsigned long long)) != hipSuccess ||
-      hipMalloc(&b->d_job_ms, size_t(n) * sizeof(float)) != hipSuccess)
+  if (dev_alloc(c, &b->d_films, b->film_words * sizeof(long long)) != hipSuccess ||
+      dev_alloc(c, &b->d_jobs, size_t(n) * sizeof(BatchJob)) != hipSuccess ||
+      dev_alloc(c, &b->d_misc, 2 * sizeof(unsigned long long)) != hipSuccess ||
+      dev_alloc(c, &b->d_job_ms, size_t(n) * sizeof(float)) != hipSuccess)
     return bail(fail(c, NE_ERR_OUT_OF_MEMORY, "batch allocation failed"));
   if (hipEventCreate(&b->ev0) != hipSuccess || hipEventCreate(&b->ev1) != hipSuccess)
     return bail(fail(c, NE_ERR_HIP, "event creation failed"));
@@ -2002,7 +2056,7 @@ void guide_free(ne_guide* g) {
 template <class T>
 bool guide_alloc(ne_guide* g, T*& p, size_t count) {
   void* q = nullptr;
-  if (hipMalloc(&q, std::max<size_t>(count, 1) * sizeof(T)) != hipSuccess) return false;
+  if (dev_alloc(g->ctx, &q, std::max<size_t>(count, 1) * sizeof(T)) != hipSuccess) return false;
   g->allocs.push_back(q);
   p = static_cast<T*>(q);
   return true;

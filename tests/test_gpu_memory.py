@@ -1,10 +1,11 @@
 """Device memory: what the library holds beyond a call's needs, and what it gives
 back when an allocation would fail."""
+import numpy as np
 import pytest
 
 import scenes
 from conftest import print_case
-from hipmem import free_bytes
+from hipmem import Block, free_bytes
 
 pytestmark = pytest.mark.gpu
 GIB = 1 << 30
@@ -25,3 +26,53 @@ def test_surface_renders_keep_a_pool_of_2_23_slots():
     assert f.read().any()
     assert used < (1 << 23) * 260 + (1 << 25) * 12 + (64 << 20), used / GIB
     ctx.close()
+
+
+def test_quads_make_room_for_other_allocations(ctx):
+    """The quad copies of the grids (four times the bricks) are a convenience: an
+    allocation that they leave no room for gets it, and the scenes then read the
+    bricks, with the same films."""
+    print_case("quads and a full card")
+    from narvalengine_amd import Batch
+    from narvalengine_amd.abi import NE_BATCH_PERSISTENT, NE_BATCH_WAVEFRONT
+    rng = np.random.default_rng(4)
+    s = scenes.small_volume(res=8, maj_res=4)
+    s.set_volume(rng.random((192, 192, 192), np.float32), 12.0, (0.95,) * 3, (0.05,) * 3, 0.7, maj_res=4)
+    g = [ctx.upload(s) for _ in range(24)]
+    size = g[0].info()["device_bytes"]
+    small = ctx.film(40, 30)
+
+    def frame():
+        small.clear()
+        ctx.render(g[5], scenes.VOLUME_CAMERA, small, spp=4, max_bounces=8, seed=3)
+        return small.read()
+
+    job = dict(scene=g[7], camera=scenes.VOLUME_CAMERA, width=40, height=30, spp=4, max_bounces=8, seed=3, job=0)
+    batch = Batch(ctx, [job])
+
+    def batches():
+        out = []
+        for executor in (NE_BATCH_PERSISTENT, NE_BATCH_WAVEFRONT):
+            batch.run((8, 8, 4, executor))
+            out.append(batch.read(0))
+        return out
+
+    want, want_batches = frame(), batches()
+    assert want.any()
+    # all but 1 GiB taken by others, then a film of 2 GiB: 2.7 GiB are in quads
+    fill = Block(free_bytes() - GIB)
+    try:
+        big = ctx.film(32768, 2731)
+    finally:
+        fill.free()
+    assert g[5].info()["device_bytes"] < size // 3
+    np.testing.assert_array_equal(frame(), want)
+    np.testing.assert_array_equal(batches(), want_batches)
+    big.close()
+    batch.close()
+    # an upload after that has its quads again
+    h = ctx.upload(s)
+    assert h.info()["device_bytes"] == size
+    for x in g:
+        x.close()
+    h.close()
