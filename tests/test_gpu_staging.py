@@ -65,3 +65,21 @@ def test_films_and_tiles_come_back_whole(ctx, w, h):
     np.testing.assert_array_equal(eng.pixels[y:y + th, x:x + tw], frame[y:y + th, x:x + tw])
     eng.pixels[y:y + th, x:x + tw] = 0
     assert not eng.pixels.any()
+
+
+@pytest.mark.parametrize("value", [np.nan, np.inf, -np.inf, -1e-38])
+def test_a_bad_voxel_is_refused_wherever_it_lies(ctx, value):
+    """17 x 17 x 15 voxels: a block of 4096 that are looked over together and a
+    remainder; first and last of each."""
+    from narvalengine_amd import NarvalError
+    print_case(f"voxel {value}")
+    for at in (0, 4095, 4096, 17 * 17 * 15 - 1):
+        grid = np.full((15, 17, 17), -0.0, np.float32)
+        grid.reshape(-1)[::3] = np.finfo(np.float32).max
+        s = scenes.small_volume(res=8, maj_res=2)
+        s.set_volume(grid, 1e-6, (0.95,) * 3, (0.05,) * 3, 0.7, maj_res=2)
+        ctx.upload(s).close()
+        grid.reshape(-1)[at] = value
+        s.set_volume(grid, 1e-6, (0.95,) * 3, (0.05,) * 3, 0.7, maj_res=2)
+        with pytest.raises(NarvalError, match="finite"):
+            ctx.upload(s)
