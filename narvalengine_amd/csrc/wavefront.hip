@@ -1,26 +1,37 @@
 // wavefront.hip -- wavefront path tracer for gfx950 (FP32 product path).
 //
 // Path state lives in HBM as two structure-of-arrays buffers A and B of P
-// slots, split into chunks of 256 slots.  Every stage kernel runs one
-// 256-thread block per chunk, thread t owning slot t of its chunk, and the
-// live paths of a chunk are kept packed at its front, so all state accesses
-// are coalesced.  One iteration:
+// slots, split into chunks of 256 slots, and the live paths of a chunk are kept
+// packed at its front, so all state accesses are coalesced.  Regen, medium,
+// shade, deliver and shadow run one 256-thread block per chunk, thread t owning
+// slot t of its chunk; plan runs one block per 1024 chunks, trace one round of
+// resident blocks that take units of 64 rays from the chunks.  One iteration:
 //
-//   plan      one block scans the chunks' free slots and hands each chunk a
-//             contiguous range of new path ids (no atomics: the assignment is
-//             a deterministic prefix sum)
+//   plan      scans the chunks' free slots and hands each chunk a contiguous
+//             range of new path ids (a prefix sum over the blocks with a
+//             look-back: the assignment is deterministic); not launched any more
+//             once every path is issued
 //   regen     fills the free tail of each chunk with camera rays for its ids
 //             (ids -> pixels in 8x8 tiles: neighbouring slots trace
-//             neighbouring pixels)
-//   trace     BVH closest hit, LDS short stack            (scenes with surfaces)
+//             neighbouring pixels); in volume-only scenes inside medium
+//   trace     (scenes with surfaces) BVH closest hit of the live paths, and any
+//             hit of the shadow rays that the last iteration queued
+//   deliver   (scenes with surfaces) those shadow rays' contributions, through
+//             ratio tracking where there is a volume (the kernel of `shadow`), to
+//             the continuing paths or to the film: until here the paths' radiance
+//             lacks the light samples of their last vertices
 //   medium    delta tracking through the majorant grid    (scenes with a volume)
 //   shade     emission / escape / depth limit, then the phase-function or
 //             glossy vertex: NEE light sample -> shadow queue of the chunk,
 //             continuation -> chunk of B (block-local compaction in LDS),
 //             ended paths -> film
-//   shadow    any-hit occlusion and/or ratio tracking; the NEE contribution
-//             goes to the continuing path in B or to the film
+//   shadow    (scenes without surfaces) ratio tracking of the rays just queued;
+//             the NEE contribution goes to the continuing path in B or to the
+//             film.  Plain and frozen-guide renders do this inside shade
 //   swap A/B
+//
+// With surfaces the loop is followed by one more trace and deliver, for the
+// shadow rays of the last iteration.
 //
 // Same-address global atomics serialise across the XCDs (about 11 ns each on
 // MI355X), so nothing here appends to a shared queue: compaction is a
@@ -1021,9 +1032,13 @@ __global__ __launch_bounds__(kChunk) void k_wf_deliver(WfState w, WfArgs a, DevS
 // and cross the volume are packed first, so that waves track whole: both tests
 // in one go in one thread per ray ran 11% of the lanes (a room with a volume,
 // 857 x 481 at 32 spp: 13.2 ms a frame; 8.0 ms in two stages, the frame 28.1 ->
-// 23.0 ms).  With the occlusion test in the BVH stage that is launched anyway,
-// two stages are no slower in small frames either (us, tested here / there: 90 x
-// 90 at 16 spp, 5936 nodes 2861 / 2212, one node 1155 / 1139).
+// 23.0 ms).  The occlusion test is in the BVH stage, which is launched anyway,
+// also for a BVH of one node: frames of one rectangle under a volume at 12
+// bounces, us, one thread per ray for both tests / tested here before the packing
+// / in the BVH stage: 1200 paths 679 / 700 / 657, 15,000 836 / 842 / 797, 60,000
+// 871 / 926 / 881, 120,000 913 / 961 / 925, 480,000 1181 / 1224 / 1182, 1.9 M
+// 2169 / 2205 / 2111, 14.7 M 8816 / 9056 / 8867: it loses about 1% from 60,000 to
+// 120,000 paths (two launches after the loop) and at 14.7 M.
 // SPATIAL: the chunk's shadow rays are taken in Morton order of their origins
 // (each keeps its own stream: same transmittances).
 // GRID: how density lookups read the grid (kGrid*).
