@@ -1425,18 +1425,21 @@ hipError_t launch_wavefront(const DevScene& s, const DevCamera& cam, WfState& w,
     // 4 GiB: the other guided variant would spill): shade tracks the shadow
     // rays itself
     const bool fuse = hv && !hs && !count && !spatial && !training && (!gh || form != kGridWide);
-#define NE_SHADE_FUSED(G, SO, GD)                                                                           \
-  do {                                                                                                      \
-    if (form == kGridQuad) hipLaunchKernelGGL((k_wf_shade<G, SO, false, 1 + kGridQuad>), grid, blk, 0, st, w, a, s, GD); \
-    else if (form == kGridBrick)                                                                             \
-      hipLaunchKernelGGL((k_wf_shade<G, SO, false, 1 + kGridBrick>), grid, blk, 0, st, w, a, s, GD);        \
-    else hipLaunchKernelGGL((k_wf_shade<G, SO, false, 1 + kGridWide>), grid, blk, 0, st, w, a, s, GD);     \
+#define NE_SHADE_FORM(G, SO, FORM, GD) \
+  hipLaunchKernelGGL((k_wf_shade<G, SO, false, 1 + FORM>), grid, blk, 0, st, w, a, s, GD)
+#define NE_SHADE_FUSED(G, SO, GD)                                    \
+  do {                                                               \
+    if (form == kGridQuad) NE_SHADE_FORM(G, SO, kGridQuad, GD);      \
+    else NE_SHADE_FORM(G, SO, kGridBrick, GD);                       \
   } while (0)
     if (fuse && gh && sort) NE_SHADE_FUSED(true, true, gh->g);
     else if (fuse && gh) NE_SHADE_FUSED(true, false, gh->g);
+    else if (fuse && form == kGridWide && sort) NE_SHADE_FORM(false, true, kGridWide, WfGuide{});
+    else if (fuse && form == kGridWide) NE_SHADE_FORM(false, false, kGridWide, WfGuide{});
     else if (fuse && sort) NE_SHADE_FUSED(false, true, WfGuide{});
     else if (fuse) NE_SHADE_FUSED(false, false, WfGuide{});
 #undef NE_SHADE_FUSED
+#undef NE_SHADE_FORM
     else if (gh && training && sort) hipLaunchKernelGGL((k_wf_shade<true, true, true>), grid, blk, 0, st, w, a, s, gh->g);
     else if (gh && training) hipLaunchKernelGGL((k_wf_shade<true, false, true>), grid, blk, 0, st, w, a, s, gh->g);
     else if (gh && sort) hipLaunchKernelGGL((k_wf_shade<true, true, false>), grid, blk, 0, st, w, a, s, gh->g);
