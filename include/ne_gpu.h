@@ -137,6 +137,9 @@ enum {
                               Morton order of their origins (same paths, same image) */
   NE_FLAG_WIDE_OFFSETS = 64, /* wavefront: read the density grid by 64-bit offsets even under 4 GiB, the
                                 kernels a grid of 4 GiB or more takes (same addresses, same image) */
+  NE_FLAG_BRICK_OFFSETS = 256, /* wavefront: read a grid that has quads by 32-bit offsets into its bricks, as
+                                  grids whose quads would exceed 4 GiB or found no room are read (same values,
+                                  same image) */
   NE_FLAG_TEST_PLAN_STALL = 128 /* test hook for the failure path: the wavefront plan's look-back waits for
                                    words that never come, its bounded wait gives up after 1024 spins, and
                                    the render fails with NE_ERR_HIP (a launch time-out) instead of hanging.

@@ -1076,7 +1076,7 @@ static ne_status render_wavefront(ne_ctx* c, const ne_scene* s, const DevCamera&
   a.max_bounces = p->max_bounces; a.sample_offset = p->sample_offset; a.job = p->job; a.nchunks = uint32_t(P / kChunk);
   a.seed = p->seed;
   a.sort = ((p->flags & NE_FLAG_SORT) ? 1 : 0) | ((p->flags & NE_FLAG_SPATIAL) ? 2 : 0);
-  a.wide_offsets = (p->flags & NE_FLAG_WIDE_OFFSETS) ? 1 : 0;
+  a.grid_max = (p->flags & NE_FLAG_WIDE_OFFSETS) ? kGridWide : (p->flags & NE_FLAG_BRICK_OFFSETS) ? kGridBrick : kGridQuad;
   a.plan_stall = (p->flags & NE_FLAG_TEST_PLAN_STALL) ? 1u : 0u;
   a.refill_min = kRefillMinIdle;
   if (c->refill_blocks == 0) {
@@ -1761,6 +1761,7 @@ hipError_t lane_render(ne_batch* b, BatchLane& L, size_t j, int div, uint32_t re
   a.max_bounces = J.max_bounces; a.sample_offset = 0; a.job = J.job; a.nchunks = uint32_t(P / kChunk);
   a.seed = J.seed;
   a.sort = 0;
+  a.grid_max = kGridQuad;
   a.refill_min = kRefillMinIdle;
   a.refill_blocks = refill_blocks;
   a.total_paths = total;

@@ -142,7 +142,7 @@ struct WfArgs {
   int32_t refill_min;   // refill kernels: a wave refills once this many of its lanes are idle
   uint32_t plan_epoch;  // tags this plan launch's look-back words (1, 2, ... within a render)
   int32_t shadow_full;  // every shadow record carries its origin and RNG key (surface-only scenes)
-  int32_t wide_offsets;  // density lookups by 64-bit offsets whatever the grid's size
+  int32_t grid_max;      // density lookups take the scene's grid_form, at most this one (kGrid*)
   uint32_t plan_stall;   // test hook: the plan's look-back waits for an epoch that never comes
   int32_t shadows;      // the BVH stage takes the last iteration's shadow rays too
   int32_t regen_done;   // the buffer that the shadow rays' paths go on in holds regen_m new paths besides

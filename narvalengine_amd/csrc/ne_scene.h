@@ -76,7 +76,8 @@ __host__ __device__ inline uint32_t quad_pad_z(int32_t r) { return (uint32_t(r) 
 
 // How a lookup reads the density: 64-bit offsets into the bricks (any grid),
 // 32-bit byte offsets into the bricks (grids under 4 GiB), or the quads by
-// 32-bit byte offsets (grids whose quads stay under 4 GiB, about 645^3).
+// 32-bit byte offsets (grids whose quads stay under 4 GiB, about 645^3), each
+// narrower than the one before.
 enum { kGridWide = 0, kGridBrick = 1, kGridQuad = 2, kGridAuto = 3 };
 
 struct DevScene {

@@ -507,7 +507,7 @@ hipError_t launch_paths(const DevScene& s, const DevCamera& cam, const WfArgs& a
                         int cus, hipStream_t st, StageTimer* tm) {
   hipError_t e = hipSuccess;
   const bool guided = gu.cache.mix != nullptr;
-  const int form = a.wide_offsets ? int(kGridWide) : s.grid_form;
+  const int form = std::min(s.grid_form, a.grid_max);
   void (*fn)(PathArgs) =
       form == kGridQuad    ? (guided ? &k_paths<true, kGridQuad> : &k_paths<false, kGridQuad>)
       : form == kGridBrick ? (guided ? &k_paths<true, kGridBrick> : &k_paths<false, kGridBrick>)

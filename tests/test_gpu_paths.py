@@ -96,3 +96,35 @@ def test_rays_in_a_face_of_the_volume(ctx, axis, side, toward):
         films.append(f.read())
     np.testing.assert_array_equal(films[1], films[2])
     np.testing.assert_allclose(films[2], films[0], rtol=1e-6, atol=16 * 2.0 ** -30)
+
+
+# how a render is run, and whether a guide is sampled
+RUNS = {"persistent": {}, "fixed_film": {"fixed_film": True}, "staged": {"mode": 2}, "small_pool": {"mode": 2, "pool_size": 1000},
+        "sort": {"mode": 2, "sort": True}, "spatial": {"mode": 2, "spatial": True}, "count": {"count": True},
+        "guided": {"guide": True}, "guided_staged": {"guide": True, "mode": 2},
+        "guided_sort": {"guide": True, "mode": 2, "sort": True}, "training": {"guide": True, "train": True}}
+
+
+@pytest.mark.parametrize("which", ["volume", "cloud", "point_light", "surfaces"])
+@pytest.mark.parametrize("run", list(RUNS))
+def test_the_grids_forms_give_the_same_film(ctx, which, run):
+    """Quads, bricks by 32-bit offsets (what grids of 645^3 to 1024^3 take, and
+    any grid whose quads found no room) and by 64-bit offsets hold the same
+    voxels: equal films and event counts in every kernel that reads them."""
+    print_case(f"grid forms {which} {run}")
+    from narvalengine_amd.runtime import Guide
+    kw = dict(RUNS[run])
+    if kw.get("guide"):  # rates of 0: a training render leaves the guide as it is
+        kw["guide"] = Guide(ctx, log2_table=12, cache_res=8, guided_vertices=3, guide_prob=0.5, batch=4096,
+                            lr_table=0.0, lr_mlp=0.0)
+    g = ctx.upload(scenes.env_map_scene() if which == "surfaces" else _scene(which))
+    for w, h, spp, bounces in [(45, 37, 8, 24), (7, 5, 1, 16)]:
+        out = []
+        for form in ({}, {"brick": True}, {"wide": True}):
+            f = ctx.film(w, h)
+            ctx.render(g, scenes.VOLUME_CAMERA, f, spp=spp, max_bounces=bounces, seed=41, **kw, **form)
+            out.append((f.read(), ctx.counters() if run == "count" else None))
+        assert out[0][0].any()
+        for o in out[1:]:
+            np.testing.assert_array_equal(out[0][0], o[0], err_msg=f"{w}x{h}")
+            assert out[0][1] == o[1]
