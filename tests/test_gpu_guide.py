@@ -7,6 +7,7 @@ from pathlib import Path
 import numpy as np
 import pytest
 
+import scenes
 from conftest import print_case
 from narvalengine_amd import Guide
 
@@ -486,3 +487,65 @@ def test_guide_gradients_of_levels_that_use_little_of_their_table(ctx, log2_tabl
         assert cos > 0.995 and rel < 0.08, (cos, rel)
     assert not gt[rt == 0.0].any()
     g.close()
+
+
+def _surfaces_and_volume(which):
+    s = scenes.env_map_scene() if which == "floor" else scenes.small_surface(subdiv=2)
+    if which == "mesh":  # a BVH of many nodes around the volume
+        from narvalengine_amd import configs
+        s.set_volume(configs.fbm_grid(16, 0), 12.0, (0.95,) * 3, (0.05,) * 3, 0.7, maj_res=4)
+    return s, scenes.VOLUME_CAMERA if which == "floor" else scenes.BOX_CAMERA
+
+
+@pytest.mark.parametrize("which", ["floor", "mesh"])
+@pytest.mark.parametrize("pool", [0, 1000])
+def test_guided_paths_among_surfaces_are_the_megakernels(ctx, which, pool):
+    """Surfaces and a volume, a frozen guide at the volume's vertices: shadow rays
+    are traced with the next iteration's paths and delivered before these are
+    shaded.  The wavefront's film is the guided megakernel's up to the
+    fixed-point rounding of a path's last light sample; a training render whose
+    rates are 0 gives the frozen guide's film bit for bit."""
+    print_case(f"guided among surfaces: {which}, pool {pool}")
+    from narvalengine_amd.abi import NE_MODE_MEGAKERNEL, NE_MODE_WAVEFRONT
+    s, cam = _surfaces_and_volume(which)
+    gs = ctx.upload(s)
+    g = Guide(ctx, log2_table=12, batch=512, seed=4, cache_res=8, guided_vertices=3, guide_prob=0.5, lr_table=0.0,
+              lr_mlp=0.0)
+    films = []
+    for kw in (dict(mode=NE_MODE_MEGAKERNEL), dict(mode=NE_MODE_WAVEFRONT, pool_size=pool),
+               dict(mode=NE_MODE_WAVEFRONT, pool_size=pool, train=True)):
+        f = ctx.film(45, 37)
+        ctx.render(gs, cam, f, spp=8, max_bounces=12, seed=6, guide=g, **kw)
+        films.append(f.read())
+    assert films[0].any() and g.stats()["steps"] >= 1
+    np.testing.assert_allclose(films[1], films[0], rtol=1e-6, atol=8 * 2.0 ** -30)
+    np.testing.assert_array_equal(films[2], films[1])
+    g.close()
+
+
+@pytest.mark.parametrize("cache_res", [0, 8])
+def test_training_samples_do_not_depend_on_a_surface_that_nothing_meets(ctx, cache_res):
+    """A rectangle of a thousandth at a distance of 100 turns a volume's scene into
+    one with surfaces, whose shadow rays are delivered an iteration later, and
+    changes no path.  A training sample's weight is what its path gathers after
+    the guided vertex: with the same samples in every batch, the loss (of a guide
+    that rates of 0 leave as it is) is the same but for the order of its sum."""
+    print_case(f"training samples with and without a surface, cache {cache_res}")
+    stats, films = [], []
+    for surface in (False, True):
+        s = scenes.small_volume(res=32, maj_res=4)
+        if surface:
+            s.add_rectangle(s.add_glossy((0.5, 0.5, 0.5), 0.5), position=(0, 0, -100), scale=(1e-3, 1e-3, 1))
+        gs = ctx.upload(s)
+        g = Guide(ctx, log2_table=12, batch=16384, seed=4, cache_res=cache_res, guided_vertices=3, lr_table=0.0,
+                  lr_mlp=0.0)
+        f = ctx.film(64, 48)
+        ctx.render(gs, scenes.VOLUME_CAMERA, f, spp=32, max_bounces=16, seed=6, guide=g, train=True, pool_size=4096)
+        stats.append(g.stats())
+        films.append(f.read())
+        g.close()
+    np.testing.assert_allclose(films[1], films[0], rtol=1e-6, atol=32 * 2.0 ** -30)
+    assert stats[0]["steps"] >= 2
+    assert (stats[0]["steps"], stats[0]["samples"]) == (stats[1]["steps"], stats[1]["samples"])
+    # sums of n FP32 terms of one sign or mixed, in two orders: n eps relative at worst
+    assert abs(stats[0]["last_loss"] - stats[1]["last_loss"]) <= 16384 * 2.0 ** -24 * abs(stats[0]["last_loss"]), stats
