@@ -232,6 +232,26 @@ ne_status dev_read(ne_ctx* c, void* dst, const void* src, size_t bytes) {
   return NE_OK;
 }
 
+// The same for `rows` rows of `row` bytes (contiguous on the device), `pitch`
+// bytes apart in the caller's memory.
+ne_status dev_read_rows(ne_ctx* c, void* dst, size_t pitch, const void* src, size_t row, size_t rows) {
+  if (!c->stage || row > kStageChunk) {
+    NE_HIP(c, hipMemcpy2DAsync(dst, pitch, src, row, row, rows, hipMemcpyDeviceToHost, c->stream));
+    NE_HIP(c, hipStreamSynchronize(c->stream));
+    return NE_OK;
+  }
+  const size_t step = kStageChunk / row;
+  for (size_t y = 0; y < rows; y += step) {
+    const size_t n = std::min(step, rows - y);
+    NE_HIP(c, hipMemcpyAsync(c->stage, static_cast<const char*>(src) + y * row, n * row, hipMemcpyDeviceToHost,
+                             c->stream));
+    NE_HIP(c, hipStreamSynchronize(c->stream));
+    c->stage_in = 0;
+    for (size_t k = 0; k < n; ++k) std::memcpy(static_cast<char*>(dst) + (y + k) * pitch, c->stage + k * row, row);
+  }
+  return NE_OK;
+}
+
 // Space for an input of at most kStageIn bytes, or null (no staging, or too
 // large); waits if copies in flight still read the part that it needs.
 char* stage_input(ne_ctx* c, size_t bytes) {
@@ -1325,18 +1345,14 @@ ne_status ne_render_tile(ne_ctx* c, const ne_scene* s, const ne_camera_desc* cam
   NE_HIP(c, launch_clear_rect(f->d_sum, f->W, q.x0, q.y0, q.x1, q.y1, c->stream));
   st = render_locked(c, s, cam, &q, f);
   if (st != NE_OK) return st;
-  // post-process the tile only, one contiguous read, then its rows into the
-  // caller's full-frame pixel array
+  // post-process the tile only, then its rows into the caller's full-frame
+  // pixel array
   DevBuf b;
   if ((st = tmp_out<float>(c, b, size_t(tw) * th * 3)) != NE_OK) return st;
   NE_HIP(c, launch_tonemap_rect(f->d_sum, f->W, q.x0, q.y0, tw, th, 1.0f / float(p->spp), static_cast<float*>(b.p),
                                 c->stream));
-  const size_t row = size_t(tw) * 3;
-  std::vector<float> tile(row * size_t(th));
-  if ((st = tmp_back(c, tile.data(), b, tile.size())) != NE_OK) return st;
-  for (int y = 0; y < th; ++y)
-    std::copy_n(&tile[row * size_t(y)], row, pixels + (size_t(q.y0 + y) * f->W + q.x0) * 3);
-  return NE_OK;
+  return dev_read_rows(c, pixels + (size_t(q.y0) * f->W + q.x0) * 3, size_t(f->W) * 3 * sizeof(float), b.p,
+                       size_t(tw) * 3 * sizeof(float), size_t(th));
 }
 
 ne_status ne_get_kernel_time(ne_ctx* c, float* ms) {

@@ -83,3 +83,23 @@ def test_a_bad_voxel_is_refused_wherever_it_lies(ctx, value):
         s.set_volume(grid, 1e-6, (0.95,) * 3, (0.05,) * 3, 0.7, maj_res=2)
         with pytest.raises(NarvalError, match="finite"):
             ctx.upload(s)
+
+
+def test_a_tile_of_more_than_a_chunk_comes_back_whole(ctx):
+    """A tile of 440 x 420 pixels, 2.2 MB in rows of 5,280 bytes: 397 rows in the
+    first chunk, 23 in the second; nothing beside the tile is written."""
+    from narvalengine_amd.engine import OfflineEngine, SceneSettings
+    print_case("large tile")
+    w, h, tw, th = 17600, 4200, 440, 420
+    eng = OfflineEngine(scenes.VOLUME_CAMERA, SceneSettings((w, h), 1, 2), scenes.small_volume(res=16, maj_res=4),
+                        ctx=ctx, seed=9)
+    index = 4 * 40 + 19
+    y, x = (index // 40) * th, (index % 40) * tw
+    eng.renderTile(scenes.VOLUME_CAMERA, index)
+    f = ctx.film(w, h)
+    ctx.render(eng.gscene, scenes.VOLUME_CAMERA, f, spp=1, max_bounces=2, seed=9, rect=(x, y, x + tw, y + th))
+    want = f.tonemap(1)
+    f.close()
+    assert want[y:y + th, x:x + tw].any()
+    np.testing.assert_array_equal(eng.pixels[y - 1:y + th + 1, x - 1:x + tw + 1], want[y - 1:y + th + 1, x - 1:x + tw + 1])
+    assert not eng.pixels[:y].any() and not eng.pixels[y + th:].any()
