@@ -68,8 +68,8 @@ __host__ __device__ inline uint64_t grid_offset(uint32_t x, uint32_t y, uint32_t
 // vector cache's address rate (a wave's load takes one tag lookup per line it
 // touches, whatever its width), so a lookup costs a quarter of it, and fewer
 // address instructions.  Bricks -> quads, ms per frame: 1920x1080 x 256 spp
-// cloud of 512^3 111.4 -> 103.5, 512x512 x 64 spp fBm of 128^3 6.96 -> 6.68,
-// 960x540 x 16 spp guided cloud of 256^3 3.29 -> 3.15.  Zero where a corner's
+// cloud of 512^3 112.2 -> 105.0, 512x512 x 64 spp fBm of 128^3 6.84 -> 6.63,
+// 960x540 x 16 spp guided cloud of 256^3 2.68 -> 2.60.  Zero where a corner's
 // index is >= res; corners at index res on x and y, res + 1 on z.
 __host__ __device__ inline uint32_t quad_pad(int32_t r) { return (uint32_t(r) + 2u) & ~1u; }    // x, y: >= res + 1
 __host__ __device__ inline uint32_t quad_pad_z(int32_t r) { return (uint32_t(r) + 3u) & ~1u; }  // z: >= res + 2

@@ -15,11 +15,12 @@
 // the next iteration packs them with other rays.  A path's shadow ray and its
 // continuation are two entries of the lists, so they also run side by side.
 //
-// Measured against the staged pipeline on one MI355X (frames with the tone
-// map): 1920x1080 x 256 spp cloud (512^3, 128 bounces) 171.0 -> 110.8 ms,
-// 512x512 x 64 spp fBm volume 9.44 -> 6.75 ms, 960x540 x 16 spp guided cloud
-// 6.51 -> 3.27 ms; VALU instructions of the cloud frame 1.0e11 -> 5.6e10, lanes
-// live 28% -> 46%.
+// Measured against the staged pipeline on one MI355X (both with quads / both with
+// bricks): 1920x1080 x 256 spp cloud (512^3, 128 bounces) 177.6 -> 105.0 / 173.3
+// -> 112.2 ms, 512x512 x 64 spp fBm volume 8.16 -> 6.63 / 9.32 -> 6.84 ms,
+// 960x540 x 16 spp guided cloud 5.75 -> 2.60 / 5.85 -> 2.68 ms; VALU
+// instructions of the cloud frame (bricks) 1.0e11 -> 5.6e10, lanes live 28% ->
+// 46%.
 //
 // A 256-thread block owns 256 path slots.  Nothing scans them: every state
 // change appends the slot to the list of what comes next.  One iteration:
@@ -41,8 +42,13 @@ namespace ne {
 constexpr int kPathBlock = 256;
 // A wave hands its rays back once at most kSuspend of them, or a quarter of
 // its group, are left.  Putting a walk away and taking it up again costs about
-// one tracking step's instructions per ray.  Cloud frame / fBm frame, ms: 0
-// (to the end) 115.5 / 7.4, 8: 110.8 / 7.3, 12: 111.4 / 7.4, 20: 114.2 / 7.7.
+// one tracking step's instructions per ray.  1920x1080 x 256 spp cloud / 640x360
+// x 32 spp cloud / 512x512 x 64 spp fBm / 1280x720 x 64 spp fBm / guided cloud
+// frames, ms: 4: 114.0 / 2.68 / 6.66 / 15.9 / 3.17, 6: 111.5 / 2.60 / 6.71 / 16.0
+// / 3.12, 8: 109.2 / 2.58 / 6.80 / 16.2 / 3.12, 10: 107.6 / 2.54 / 6.90 / 16.4 /
+// 3.10, 12: 106.9 / 2.50 / 6.95 / 16.3 / 3.08, 16: 107.1 / 2.54 / 7.10 / 16.6 /
+// 3.08, 20: 107.0 / 2.49 / 7.07 / 16.7 / 3.14.  The fBm volumes, whose walks end
+// sooner, gain up to 4% from 4, the cloud loses 7%: 12.
 constexpr int kSuspend = 12;
 
 // A slot's depth word: vertices so far, and in the upper half what is over.
