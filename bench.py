@@ -411,13 +411,13 @@ def relmse_parts(img, ref, ref_var, eps=1e-2):
 def equal_time_relmse(ctx, g, wl, args, threads: int) -> dict:
     """Equal-time relMSE of guided against plain rendering on the full frame
     of the workload, against an FP64 converged render that the CPU probes
-    accept.  For each budget of K frames: plain is the FP32 wavefront at K x
+    accept.  For each budget of K frames: plain is the default FP32 render at K x
     the workload's spp, and sets the wall time.  Guided: a fresh guide trains
     online while it renders args.train_spp, then the frozen, tabulated guide
     renders the rest of the same wall time (training included; both phases'
-    samples count), through the wavefront (guided) and through the persistent
-    batch kernel (guided+batched).  The batch kernel's plain frame is timed
-    beside them."""
+    samples count), through ne_render_guided (guided) and through the batch
+    (guided+batched, the executor that its autotuner picks).  The batch's plain
+    frame is timed beside them."""
     W, H, spp = wl.width, wl.height, wl.spp
     ref_spp = args.ref_mult * spp
     ref, ref_var, ref_s = converged_reference(ctx, g, wl, ref_spp, args.ref_passes, seed=1000)
@@ -442,10 +442,10 @@ def equal_time_relmse(ctx, g, wl, args, threads: int) -> dict:
 def equal_time_budget(ctx, g, wl, args, ref, ref_var, f, K: int) -> dict:
     from narvalengine_amd import Batch, Guide
     W, H, spp = wl.width, wl.height, wl.spp
-    # every wavefront render of the comparison on the pool the plain frame
-    # gets by default (2^23 slots at this size), so that the pilot's time per
-    # sample holds for the longer renders and no form runs on a smaller pool
-    kw = dict(max_bounces=wl.max_bounces, pool_size=1 << 23)
+    # every render but the training on the pipeline that a caller gets by
+    # default: an explicit pool would take the staged one, and the batched forms
+    # the default
+    kw = dict(max_bounces=wl.max_bounces)
     n_plain = K * spp
     f.clear()
     ctx.synchronize()

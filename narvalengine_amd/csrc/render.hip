@@ -162,8 +162,8 @@ static hipError_t launch_render_t(const DevScene& s, const DevCamera& cam, const
 // waves 4.2 / 3.4 / 3.0; fBm volume, 2088 waves 0.22 / 0.25, 4800 waves 0.90 /
 // 0.83 / 0.82, 32,000 waves 4.2 / 3.4 / 2.8; mesh, 64 waves 1.09 / 1.11 / 1.15,
 // 3025 waves 2.0 / 1.4, 4800 waves 4.1 / 2.8 / 3.0, 32,000 waves 23.3 / 13.8 /
-// 14.1.  Each side of the lines, ms, all at one wave / as ruled (frames of one
-// sample, 16 bounces): fBm volume, 4032 waves 0.98 / 0.98, 4160 waves 1.02 /
+// 14.1.  Each side of the lines, ms, before the rule (and the quads and decoded
+// nodes) / with them, frames of one sample and 16 bounces: fBm volume, 4032 waves 0.98 / 0.98, 4160 waves 1.02 /
 // 0.94, 4356 waves 1.03 / 0.91, 16,256 waves 3.10 / 2.54, 16,512 waves 3.17 /
 // 2.18; cloud, 4032 waves 1.71 / 1.62, 4160 waves 1.66 / 1.60, 16,256 waves 5.00 /
 // 4.14, 16,512 waves 5.00 / 3.60; mesh of 5 k triangles, 2000 waves 2.64 / 2.04,
