@@ -29,9 +29,18 @@ __device__ __forceinline__ uint32_t xcd_logical_block(uint32_t nreal) {
 
 // SURF = false: a volume lit only by the sun and the environment (no surface
 // code); GUIDED: medium vertices sample the guide's tabulated proposal.
+// WAVES 0 leaves the registers to the compiler, but for FP32 with surfaces: the
+// decoded nodes' seven loads take 173 VGPRs, where two waves per SIMD fit; held
+// to the 168 of three waves it spills seven (320 x 240 x 8 spp, us, 64-B nodes /
+// 173 VGPRs / 168: mesh of 20 k triangles 3950 / 3963 / 3096, box 2266 / 2490 /
+// 1961, rectangle under a volume 1102 / 1191 / 1004).
+template <typename R, bool C, int WAVES, bool SURF, bool GUIDED>
+constexpr int render_waves() {
+  return WAVES == 0 && std::is_same<R, float>::value && !C && SURF && !GUIDED ? 3 : WAVES;
+}
 template <typename R, bool C, int BLOCK, int WAVES = 0, bool SURF = true, bool GUIDED = false>
-__global__ __launch_bounds__(BLOCK, WAVES) void k_render(DevScene s, DevCamera cam, RenderArgs a,
-                                                          uint32_t nreal_blocks) {
+__global__ __launch_bounds__(BLOCK, (render_waves<R, C, WAVES, SURF, GUIDED>())) void k_render(
+    DevScene s, DevCamera cam, RenderArgs a, uint32_t nreal_blocks) {
   __shared__ uint32_t lds_stack[kShortStack * BLOCK];
   uint32_t lb = xcd_logical_block(nreal_blocks);
   if (lb >= nreal_blocks) return;
@@ -163,11 +172,12 @@ static hipError_t launch_render_t(const DevScene& s, const DevCamera& cam, const
 // 0.83 / 0.82, 32,000 waves 4.2 / 3.4 / 2.8; mesh, 64 waves 1.09 / 1.11 / 1.15,
 // 3025 waves 2.0 / 1.4, 4800 waves 4.1 / 2.8 / 3.0, 32,000 waves 23.3 / 13.8 /
 // 14.1.  Each side of the lines, ms, before the rule (and the quads and decoded
-// nodes) / with them, frames of one sample and 16 bounces: fBm volume, 4032 waves 0.98 / 0.98, 4160 waves 1.02 /
-// 0.94, 4356 waves 1.03 / 0.91, 16,256 waves 3.10 / 2.54, 16,512 waves 3.17 /
-// 2.18; cloud, 4032 waves 1.71 / 1.62, 4160 waves 1.66 / 1.60, 16,256 waves 5.00 /
-// 4.14, 16,512 waves 5.00 / 3.60; mesh of 5 k triangles, 2000 waves 2.64 / 2.04,
-// 2070 waves 3.13 / 1.85, 4032 waves 4.66 / 2.42, 16,512 waves 16.6 / 7.96.
+// nodes) / with them, frames of one sample and 16 bounces: fBm volume, 4032 waves
+// 0.98 / 0.98, 4160 waves 1.02 / 0.94, 4356 waves 1.03 / 0.91, 16,256 waves 3.10 /
+// 2.54, 16,512 waves 3.17 / 2.18; cloud, 4032 waves 1.71 / 1.62, 4160 waves 1.66 /
+// 1.60, 16,256 waves 5.00 / 4.14, 16,512 waves 5.00 / 3.60; mesh of 5 k triangles,
+// 2000 waves 2.64 / 2.04, 2070 waves 3.13 / 1.85, 4032 waves 4.66 / 2.42, 16,512
+// waves 16.6 / 7.96.
 hipError_t launch_render(const DevScene& s, const DevCamera& cam, const RenderArgs& a, int precision, bool count,
                          int block, int occupancy, int cus, hipStream_t st) {
   const int64_t simds = 4 * int64_t(cus), waves = int64_t(a.ntx) * a.nty * a.nchunks;
