@@ -397,7 +397,7 @@ __global__ __launch_bounds__(1024) void k_guide_reduce(GuideNet g, GuideTrain t,
 // it: tables of more ranges than the chip has CUs take all samples in every
 // block; smaller ones split the samples into `chunks`, each with a copy of the
 // ranges (t.table_part, 64 KiB per range and chunk: at most 16 MiB, as chunks x
-// ranges fill the chip once), and sum the copies after (k_guide_table_sum).  The whole training pass with its copies,
+// ranges fill the chip once: it fits in the weights' partials), and sum the copies after (k_guide_table_sum).  The whole training pass with its copies,
 // 65,536 samples, this kernel against atomics at every level, us:
 // log2_table 15: 488 / 1306, 17: 648 / 1292, 19: 658 / 1301, 21: 971 / 1360;
 // 8192 samples: 15: 316 / 454, 21: 279 / 333.  Atomics for the large levels
@@ -613,17 +613,14 @@ static int table_units(const GuideNet& g) {
 // Chunks of the samples in the table gradient: as many as fill the chip once
 // (256 CUs, one block each), at most 16.
 static int table_chunks(const GuideNet& g) { return std::min(16, std::max(1, 256 / table_units(g))); }
-size_t guide_table_part(const GuideNet& g) {
-  const int chunks = table_chunks(g);
-  return chunks == 1 ? 0 : size_t(table_units(g)) * chunks * kTableRange * kGuideFeat;
-}
+static_assert(256ull * kTableRange * kGuideFeat <= uint64_t(kGuideParts) * kGuideParams, "table_part lies in partial");
 
 // Gradients of the weight-normalised loss -sum r log q / sum r (1 / sum r is
 // read on the device after the forward pass).  n: at least the sample count.
 hipError_t launch_guide_grad(const GuideNet& g, const GuideBatch& b, const GuideTrain& t, uint32_t n, hipStream_t st) {
   const uint32_t tiles = std::max<uint32_t>(1, (std::min(n, b.cap) + 15) / 16);
   const uint32_t fblocks = std::min<uint32_t>(kGuideFwdBlocks, (tiles + kWavesPerBlock - 1) / kWavesPerBlock);
-  const uint32_t blocks = std::min<uint32_t>(uint32_t(t.parts), (tiles + kBwdWaves - 1) / kBwdWaves);
+  const uint32_t blocks = std::min<uint32_t>(kGuideParts, (tiles + kBwdWaves - 1) / kBwdWaves);
   const dim3 blk(kBwdBlock);
   hipLaunchKernelGGL(k_guide_train_fwd, dim3(fblocks), dim3(kGuideBlock), 0, st, g, b, t);
   hipLaunchKernelGGL(k_guide_loss, dim3(1), dim3(256), 0, st, t, int(fblocks));

@@ -250,15 +250,14 @@ struct GuideTrain {
   uint16_t* dy;        // cap x 64 BF16 output gradient of the current layer
   uint16_t* dy2;       // cap x 64 BF16 (ping-pong)
   float* denc;         // 32 x cap encoding gradient
-  float* partial;      // parts x kGuideParams weight/bias gradient partials
+  float* partial;      // kGuideParts x kGuideParams weight/bias gradient partials
   float* loss;         // [0] summed loss, [1] summed weight
-  float* loss_part;    // the same per forward block
-  float* aos;          // samples as the caller gave them (10 floats each)
-  float* table_part;   // table gradient per chunk of the samples (guide_table_part floats)
-  int32_t parts;       // backward blocks at most
+  float* loss_part;    // the same per forward block, kGuideFwdBlocks pairs
+  float* aos;          // samples as the caller gave them (10 floats each); the memory of act, which is written later
+  float* table_part;   // table gradient per chunk of the samples; the memory of partial, which is read before
 };
 constexpr uint32_t kGuideFwdBlocks = 8192;
-size_t guide_table_part(const GuideNet& g);  // floats of table_part; 0: the samples are not split
+constexpr uint32_t kGuideParts = 512;  // backward blocks at most
 
 // Guided wavefront: per-path training record (one per slot and path buffer).
 // state 0: none; 1: a guided vertex was sampled, the radiance baseline is

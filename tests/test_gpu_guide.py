@@ -549,3 +549,20 @@ def test_training_samples_do_not_depend_on_a_surface_that_nothing_meets(ctx, cac
     assert (stats[0]["steps"], stats[0]["samples"]) == (stats[1]["steps"], stats[1]["samples"])
     # sums of n FP32 terms of one sign or mixed, in two orders: n eps relative at worst
     assert abs(stats[0]["last_loss"] - stats[1]["last_loss"]) <= 16384 * 2.0 ** -24 * abs(stats[0]["last_loss"]), stats
+
+
+def test_a_guide_takes_the_memory_of_its_arrays(ctx):
+    """What a step needs for a while lies in arrays that it does not need then:
+    no allocation beyond the tables (FP32 with gradient and two moments, BF16),
+    the network's partial sums and a batch's activations and gradients."""
+    from hipmem import free_bytes
+    print_case("guide memory")
+    batch = 65536
+    Guide(ctx, log2_table=16, batch=batch).close()
+    before = free_bytes()
+    g = Guide(ctx, log2_table=16, batch=batch)
+    used = before - free_bytes()
+    # per sample: 10 floats, 5 layers of 64 and two gradients of 64 in BF16, 32 floats
+    arrays = 4.5 * 4 * g.table_floats + 512 * 4 * g.mlp_floats + batch * (40 + 640 + 256 + 128)
+    assert used < arrays + (8 << 20), (used, arrays)
+    g.close()
