@@ -817,7 +817,8 @@ static ne_status upload_scene(ne_ctx* c, const ne_scene_desc* d, bool quads, ne_
       ds.grid_form = nb < (size_t(1) << 32) && ds.grid_step_z < (1u << 24) ? kGridBrick : kGridWide;
       const uint32_t qx = quad_pad(ds.res[0]), qy = quad_pad(ds.res[1]), qz = quad_pad_z(ds.res[2]);
       const uint64_t qstep = uint64_t(qx / 2u) * (qy / 2u) * 8u, qbytes = qstep * (qz / 2u) * sizeof(float4);
-      if (quads && ds.grid_form == kGridBrick && qbytes < (uint64_t(1) << 32) && qstep < (1u << 24)) {
+      // (a homogeneous medium's density is not read)
+      if (quads && !homog && ds.grid_form == kGridBrick && qbytes < (uint64_t(1) << 32) && qstep < (1u << 24)) {
         if (hipMalloc(&s->quads, qbytes) == hipSuccess) {
           s->quad_bytes = qbytes;
           s->bytes += qbytes;

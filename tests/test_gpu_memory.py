@@ -76,3 +76,16 @@ def test_quads_make_room_for_other_allocations(ctx):
     for x in g:
         x.close()
     h.close()
+
+
+def test_a_homogeneous_medium_has_no_quads(ctx):
+    """Its density is not read: the 1^3 grid's bricks (two of 128 B in z, one of
+    slack), a majorant and its pair."""
+    from narvalengine_amd.scene import Scene
+    print_case("homogeneous medium")
+    s = Scene()
+    s.set_homogeneous_volume(3.0, (0.9,) * 3, (0.1,) * 3, 0.6)
+    s.set_sun((1, -1, 0.3))
+    g = ctx.upload(s)
+    assert g.info()["device_bytes"] == 3 * 128 + 4 + 8
+    g.close()
