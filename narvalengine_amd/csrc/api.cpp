@@ -196,7 +196,10 @@ ne_status dev_upload(ne_ctx* c, ne_scene* s, const T* src, size_t count, const T
 // 499, 256 KiB out 19 / 114, 4 MiB into fresh pages 82 / 247, 32 KiB in 9 / 20,
 // 256 KiB in 14 / 108.  Inputs of 1 MiB cost the same both ways (51 / 53) and
 // larger ones more (3 MiB: 120 / 105), so those go straight.
-constexpr size_t kStageChunk = size_t(2) << 20, kStageIn = size_t(1) << 20;
+// Reads above kStageWhole go in two chunks or more, one crossing the bus while the
+// one before is copied out (us, straight / whole / in two: a film of 1536 KiB 114 / 113 / 92, of 2047 KiB
+// 135 / 144 / 120).
+constexpr size_t kStageWhole = size_t(1) << 20, kStageChunk = size_t(2) << 20, kStageIn = size_t(1) << 20;
 constexpr size_t kLiDirect = size_t(512) << 10;
 
 // Device -> the caller's memory, after what c->stream holds; returns when it is
@@ -207,25 +210,26 @@ ne_status dev_read(ne_ctx* c, void* dst, const void* src, size_t bytes) {
     NE_HIP(c, hipStreamSynchronize(c->stream));
     return NE_OK;
   }
-  if (bytes <= kStageChunk) {
+  if (bytes <= kStageWhole) {
     NE_HIP(c, hipMemcpyAsync(c->stage, src, bytes, hipMemcpyDeviceToHost, c->stream));
     NE_HIP(c, hipStreamSynchronize(c->stream));
     c->stage_in = 0;
     std::memcpy(dst, c->stage, bytes);
     return NE_OK;
   }
+  const size_t chunk = std::min(kStageChunk, (bytes / 2 + 256) & ~size_t(255));  // two at least
   auto issue = [&](size_t off) {
-    const size_t k = off / kStageChunk & 1;
+    const size_t k = off / chunk & 1;
     const hipError_t e = hipMemcpyAsync(c->stage + k * kStageChunk, static_cast<const char*>(src) + off,
-                                        std::min(kStageChunk, bytes - off), hipMemcpyDeviceToHost, c->stream);
+                                        std::min(chunk, bytes - off), hipMemcpyDeviceToHost, c->stream);
     return e == hipSuccess ? hipEventRecord(c->stage_ev[k], c->stream) : e;
   };
   NE_HIP(c, issue(0));
-  for (size_t off = 0; off < bytes; off += kStageChunk) {
-    const size_t k = off / kStageChunk & 1;
-    if (off + kStageChunk < bytes) NE_HIP(c, issue(off + kStageChunk));
+  for (size_t off = 0; off < bytes; off += chunk) {
+    const size_t k = off / chunk & 1;
+    if (off + chunk < bytes) NE_HIP(c, issue(off + chunk));
     NE_HIP(c, hipEventSynchronize(c->stage_ev[k]));
-    std::memcpy(static_cast<char*>(dst) + off, c->stage + k * kStageChunk, std::min(kStageChunk, bytes - off));
+    std::memcpy(static_cast<char*>(dst) + off, c->stage + k * kStageChunk, std::min(chunk, bytes - off));
   }
   NE_HIP(c, hipStreamSynchronize(c->stream));
   c->stage_in = 0;

@@ -103,3 +103,19 @@ def test_a_tile_of_more_than_a_chunk_comes_back_whole(ctx):
     assert want[y:y + th, x:x + tw].any()
     np.testing.assert_array_equal(eng.pixels[y - 1:y + th + 1, x - 1:x + tw + 1], want[y - 1:y + th + 1, x - 1:x + tw + 1])
     assert not eng.pixels[:y].any() and not eng.pixels[y + th:].any()
+
+
+@pytest.mark.parametrize("n", [6553, 6554, 13107, 13108, 26214, 26215, 39322])
+def test_reads_come_back_whole_at_their_chunks_edges(ctx, n):
+    """160 B a query: below and above 1 MiB (one chunk or two halves), 2 MiB,
+    4 MiB (two chunks and a remainder) and 6 MiB; a query's mixture does not
+    depend on its place in the call."""
+    from narvalengine_amd import Guide
+    print_case(f"eval of {n} queries")
+    g = Guide(ctx, log2_table=10, batch=16, seed=3)
+    q = np.random.default_rng(7).uniform(0, 1, (n, 6)).astype(np.float32)
+    whole = g.eval(q)
+    parts = np.concatenate([g.eval(q[k:k + 1600]) for k in range(0, n, 1600)])
+    assert whole.any()
+    np.testing.assert_array_equal(whole, parts)
+    g.close()
