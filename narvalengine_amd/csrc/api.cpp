@@ -197,8 +197,8 @@ ne_status dev_upload(ne_ctx* c, ne_scene* s, const T* src, size_t count, const T
 // 256 KiB in 14 / 108.  Inputs of 1 MiB cost the same both ways (51 / 53) and
 // larger ones more (3 MiB: 120 / 105), so those go straight.
 // Reads above kStageWhole go in two chunks or more, one crossing the bus while the
-// one before is copied out (us, straight / whole / in two: a film of 1536 KiB 114 / 113 / 92, of 2047 KiB
-// 135 / 144 / 120).
+// one before is copied out (us, straight / whole / in two: a film of 1536 KiB 114 /
+// 113 / 92, of 2047 KiB 135 / 144 / 120).
 constexpr size_t kStageWhole = size_t(1) << 20, kStageChunk = size_t(2) << 20, kStageIn = size_t(1) << 20;
 constexpr size_t kLiDirect = size_t(512) << 10;
 

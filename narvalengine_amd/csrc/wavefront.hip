@@ -532,8 +532,15 @@ __global__ __launch_bounds__(kChunk) void k_wf_trace(TraceArgs g) {
 // REGEN (volume-only scenes): the block first makes its chunk's new paths, as
 // k_wf_regen would, which saves that stage's launch every iteration.
 // GRID: how density lookups read the grid (kGrid*).
+// Held to the SGPRs of eight waves per SIMD: left to the compiler, the variant
+// with REGEN takes 106 and the shadow stage 103 to 106, where seven fit (a few
+// spilled addresses cost less; held by __launch_bounds__ they become 78 and 43
+// spilled).  Staged frames, ms, 106 / 96 / 78: 1920x1080 x 256 spp cloud 178.0 /
+// 172.7 / 169.9, 512x512 x 64 spp fBm 8.14 / 8.13 / 8.18, 320x240 x 8 spp fBm in
+// 256 chunks 1.69 / 1.69 / 1.74; room with a volume 22.1 / 21.8 / 21.7.
+#define NE_SGPRS_8_WAVES __attribute__((amdgpu_num_sgpr(96)))
 template <bool C, bool HAS_SURF, bool SPATIAL, bool REGEN, int GRID>
-__global__ __launch_bounds__(kChunk) void k_wf_medium(WfState w, WfArgs a, DevScene s, DevCamera cam) {
+__global__ __launch_bounds__(kChunk) NE_SGPRS_8_WAVES void k_wf_medium(WfState w, WfArgs a, DevScene s, DevCamera cam) {
   __shared__ uint32_t red[kChunk / 64];
   __shared__ uint32_t skey[SPATIAL ? kChunk : 1];
   const WfPaths A = w.paths[a.cur];
@@ -1043,7 +1050,7 @@ __global__ __launch_bounds__(kChunk) void k_wf_deliver(WfState w, WfArgs a, DevS
 // (each keeps its own stream: same transmittances).
 // GRID: how density lookups read the grid (kGrid*).
 template <bool C, bool HAS_SURF, bool SPATIAL, int GRID>
-__global__ __launch_bounds__(kChunk) void k_wf_shadow(WfState w, WfArgs a, DevScene s) {
+__global__ __launch_bounds__(kChunk) NE_SGPRS_8_WAVES void k_wf_shadow(WfState w, WfArgs a, DevScene s) {
   __shared__ uint32_t red[kChunk / 64];
   __shared__ uint32_t skey[SPATIAL ? kChunk : 1];
   __shared__ uint32_t list[HAS_SURF ? kChunk : 1];
