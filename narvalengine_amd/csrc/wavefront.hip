@@ -30,8 +30,8 @@
 //             film.  Plain and frozen-guide renders do this inside shade
 //   swap A/B
 //
-// With surfaces the loop is followed by one more trace and deliver, for the
-// shadow rays of the last iteration.
+// With surfaces the loop is followed by one more trace (where a shadow ray may be
+// left) and deliver, for the shadow rays of the last iteration.
 //
 // Same-address global atomics serialise across the XCDs (about 11 ns each on
 // MI355X), so nothing here appends to a shared queue: compaction is a
@@ -1045,7 +1045,7 @@ __global__ __launch_bounds__(kChunk) void k_wf_deliver(WfState w, WfArgs a, DevS
 // / in the BVH stage: 1200 paths 679 / 700 / 657, 15,000 836 / 842 / 797, 60,000
 // 871 / 926 / 881, 120,000 913 / 961 / 925, 480,000 1181 / 1224 / 1182, 1.9 M
 // 2169 / 2205 / 2111, 14.7 M 8816 / 9056 / 8867: it loses about 1% from 60,000 to
-// 120,000 paths (two launches after the loop) and at 14.7 M.
+// 120,000 paths (the launches after the loop) and at 14.7 M.
 // SPATIAL: the chunk's shadow rays are taken in Morton order of their origins
 // (each keeps its own stream: same transmittances).
 // GRID: how density lookups read the grid (kGrid*).
@@ -1330,6 +1330,7 @@ hipError_t launch_wavefront(const DevScene& s, const DevCamera& cam, WfState& w,
     else if (count) NE_SHADOW(true, true, d);
     else NE_SHADOW(false, true, d);
   };
+  const bool at_once = a.total_paths <= uint64_t(NC) * kChunk;  // the first iteration issues every path
   bool drain = false;
   for (uint32_t it = 0;; ++it) {
     a.cur = int(it & 1u);
@@ -1365,8 +1366,12 @@ hipError_t launch_wavefront(const DevScene& s, const DevCamera& cam, WfState& w,
           NE_MARK(kStageOther);
           a.shadows = 1;
           a.regen_done = 0;
-          if (count) hipLaunchKernelGGL(k_wf_trace<true>, trace_grid(a.shadows), blk, 0, st, TraceArgs{w, a, s});
-          else hipLaunchKernelGGL(k_wf_trace<false>, trace_grid(a.shadows), blk, 0, st, TraceArgs{w, a, s});
+          // (none to trace where every path was issued at once and has had its
+          // max_bounces + 1 segments: the empty BVH launch cost frames that are
+          // bound by their launches about 1%)
+          const bool queued = !(at_once && it > uint32_t(a.max_bounces));
+          if (queued && count) hipLaunchKernelGGL(k_wf_trace<true>, trace_grid(true), blk, 0, st, TraceArgs{w, a, s});
+          else if (queued) hipLaunchKernelGGL(k_wf_trace<false>, trace_grid(true), blk, 0, st, TraceArgs{w, a, s});
           NE_MARK(kStageShadow);
           deliver_last(false);
         }

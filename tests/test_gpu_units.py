@@ -68,3 +68,24 @@ def test_units_trace_the_megakernels_paths(ctx, which, order):
             counts.append({k: ctx.counters()[k] for k in EVENTS[which]})
         np.testing.assert_allclose(films[1], films[0], rtol=1e-6, atol=spp * 2.0 ** -30, err_msg=f"{w}x{h}x{spp}")
         assert counts[0] == counts[1], (w, h, spp, counts)
+
+
+@pytest.mark.parametrize("which", ["surface", "mixed", "mixed_mesh"])
+@pytest.mark.parametrize("bounces", [0, 1, 5, 6, 7, 8, 13, 14, 15, 16])
+@pytest.mark.parametrize("pool", [0, 1024])
+def test_the_last_shadow_rays_are_delivered(ctx, which, bounces, pool):
+    """The loop looks every 8 iterations whether paths are left; the last vertices'
+    shadow rays are traced with the next segments, or after the loop: max_bounces
+    around the iterations where it ends, all paths issued at once (1045 in a pool
+    of their own) and in a pool that is refilled (4180 in 1024 slots)."""
+    print_case(f"last shadow rays {which}, {bounces} bounces, pool {pool}")
+    from narvalengine_amd.abi import NE_MODE_MEGAKERNEL, NE_MODE_WAVEFRONT
+    s, cam = _scene(which)
+    g = ctx.upload(s)
+    spp = 4 if pool else 1
+    films = []
+    for mode, pool_size in ((NE_MODE_MEGAKERNEL, 0), (NE_MODE_WAVEFRONT, pool)):
+        f = ctx.film(55, 19)
+        ctx.render(g, cam, f, spp=spp, max_bounces=bounces, seed=11, mode=mode, pool_size=pool_size)
+        films.append(f.read())
+    np.testing.assert_allclose(films[1], films[0], rtol=1e-6, atol=spp * 2.0 ** -30)
