@@ -65,7 +65,7 @@ struct ne_scene {
   ne_ctx* ctx = nullptr;
   DevScene dev{};
   std::vector<void*> allocs;
-  uint64_t bytes = 0;
+  std::atomic<uint64_t> bytes{0};  // read without mu (ne_scene_get_info), falls where the quads make room
   void* quads = nullptr;  // the density's quad copy (dev.quad), or null
   size_t quad_bytes = 0;
   ne_scene_info info{};
@@ -154,7 +154,6 @@ bool release_quads(ne_ctx* c) {
     s->dev.quad = nullptr;
     s->dev.grid_form = kGridBrick;
     s->bytes -= s->quad_bytes;
-    s->info.device_bytes = s->bytes;
   }
   c->quad_scenes.clear();
   return true;
@@ -927,7 +926,6 @@ static ne_status upload_scene(ne_ctx* c, const ne_scene_desc* d, bool quads, ne_
   s->info.bvh_depth = bvh.max_depth;
   s->info.bvh_leaf_prims_max = bvh.max_leaf;
   s->info.maj_res = uint32_t(d->has_volume ? ds.mres : 0);
-  s->info.device_bytes = s->bytes;
   s->info.grid_max_density = gmax;
   if (s->quads) c->quad_scenes.push_back(s);
   c->refs.fetch_add(1);
@@ -968,8 +966,8 @@ void ne_scene_release(ne_scene* s) {
 
 ne_status ne_scene_get_info(const ne_scene* s, ne_scene_info* out) {
   if (!s || !out) return fail(nullptr, NE_ERR_INVALID_ARG, "scene/out is NULL");
-  std::lock_guard<std::mutex> lk(s->ctx->mu);  // (its device bytes change where its quads make room)
   *out = s->info;
+  out->device_bytes = s->bytes;
   return NE_OK;
 }
 

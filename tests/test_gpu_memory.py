@@ -89,3 +89,33 @@ def test_a_homogeneous_medium_has_no_quads(ctx):
     g = ctx.upload(s)
     assert g.info()["device_bytes"] == 3 * 128 + 4 + 8
     g.close()
+
+
+def test_scene_info_does_not_wait_for_a_render(ctx):
+    """A scene's info is read while another thread holds the context in a batch of
+    a quarter of a second."""
+    import threading
+    import time
+    from narvalengine_amd import Batch
+    from narvalengine_amd.abi import NE_BATCH_WAVEFRONT
+    print_case("info beside a batch")
+    g = ctx.upload(scenes.small_surface(subdiv=3))
+    job = dict(scene=g, camera=scenes.BOX_CAMERA, width=1024, height=1024, spp=64, max_bounces=8, seed=3, job=0)
+    batch = Batch(ctx, [dict(job, job=j) for j in range(4)])
+    batch.run((8, 8, 4, NE_BATCH_WAVEFRONT))
+    took = []
+
+    def run():
+        t = time.perf_counter()
+        batch.run((8, 8, 4, NE_BATCH_WAVEFRONT))
+        took.append(time.perf_counter() - t)
+
+    th = threading.Thread(target=run)
+    th.start()
+    time.sleep(0.02)
+    t = time.perf_counter()
+    assert g.info()["device_bytes"] > 0
+    waited, alive = time.perf_counter() - t, th.is_alive()
+    th.join()
+    assert alive and waited < 0.25 * took[0], (waited, took)
+    batch.close()
