@@ -184,8 +184,9 @@ typedef struct ne_render_params {
                                  without surfaces, where no flag or pool_size asks for the staged
                                  wavefront, else the staged wavefront; FP64: megakernel) */
   int32_t pool_size;          /* staged wavefront path slots (rounded up to 256); 0 = library default
-                                 (2^23 for surface-only scenes and for renders of 2^28 paths
-                                 or more, else 2^22) */
+                                 (surface-only scenes 2^23, 2^24 for renders of 2^27 paths or
+                                 more of BVHs of 2^16 nodes or more; with a volume 2^22, 2^23
+                                 for 2^28 paths or more) */
 } ne_render_params;
 
 enum { NE_MODE_AUTO = 0, NE_MODE_MEGAKERNEL = 1, NE_MODE_WAVEFRONT = 2 };

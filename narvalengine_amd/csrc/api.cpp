@@ -1037,18 +1037,22 @@ ne_status ne_film_tonemap(ne_film* f, int32_t spp, float* pixels) {
 constexpr size_t kMaxSampleBuffer = size_t(16) << 30;
 
 // Default wavefront pool (slots) for a render of `total` paths, measured on
-// MI355X: 2^23 for surface-only scenes, where fewer, larger BVH launches
-// amortise each launch's tail (2^24 slots take twice the memory and more time on
-// most renders, ms at 2^23 / 2^24: 1024x1024 x 32 spp of an icosphere of 5 k
-// triangles 35.2 / 37.5, 82 k 38.5 / 40.6, 1.3 M 42.9 / 44.8; x 128 spp 133.4 /
-// 134.5, 144.8 / 144.5, 160.2 / 157.0).  With a volume 2^22, where a larger pool
-// adds cache pressure, except for long renders (2^28 paths and more, e.g. the
-// 1920x1080 cloud at 256 spp), whose iterations' fixed costs (launches, the
-// plan scan) halve with 2^23 slots: 236.4 -> 231.5 ms per cloud frame, while
-// a 512^2 x 64-spp volume frame took 12.0 ms at 2^22 and 13.4 ms at 2^23.
+// MI355X.  Surface-only scenes: 2^23, where fewer, larger BVH launches amortise
+// each launch's tail; 2^24 only for long renders of large BVHs, whose rays differ
+// most in length (ms at 2^23 / 2^24, meshes of 320 / 5 k / 82 k / 1.3 M triangles:
+// 2^25 paths - / 35.2 / 37.5, 38.5 / 40.6, 42.9 / 44.8; 2^27 125.7 / 127.6, 133.4 /
+// 134.7, 144.9 / 144.9, 160.7 / 157.5; 2^28 249.5 / 251.4, 264.8 / 265.2, 286.6 /
+// 284.3, 317.4 / 308.8), at twice the memory: a render that finds no room for it
+// takes 2^23.  With a volume 2^22, where a larger pool adds cache pressure, except
+// for long renders (2^28 paths and more, e.g. the 1920x1080 cloud at 256 spp),
+// whose iterations' fixed costs (launches, the plan scan) halve with 2^23 slots:
+// 236.4 -> 231.5 ms per cloud frame, while a 512^2 x 64-spp volume frame took 12.0
+// ms at 2^22 and 13.4 ms at 2^23.
+constexpr uint64_t kPool = uint64_t(1) << 23;
 static uint64_t default_pool(const DevScene& ds, uint64_t total) {
-  if (ds.n_nodes > 0 && !ds.has_volume) return uint64_t(1) << 23;
-  return total >= (uint64_t(1) << 28) ? (uint64_t(1) << 23) : (uint64_t(1) << 22);
+  if (ds.n_nodes > 0 && !ds.has_volume)
+    return total >= (uint64_t(1) << 27) && ds.n_nodes >= (1u << 16) ? 2 * kPool : kPool;
+  return total >= (uint64_t(1) << 28) ? kPool : kPool / 2;
 }
 
 // Scenes that the persistent path kernel takes (paths.hip): a volume, and
@@ -1085,7 +1089,12 @@ static ne_status render_wavefront(ne_ctx* c, const ne_scene* s, const DevCamera&
       NE_HIP(c, hipFree(old));
     }
     void* nb = nullptr;
-    NE_HIP(c, dev_alloc(c, &nb, wf_bytes(uint32_t(P))));
+    hipError_t e = dev_alloc(c, &nb, wf_bytes(uint32_t(P)));
+    if (e == hipErrorOutOfMemory && p->pool_size == 0 && P > kPool) {
+      P = kPool;
+      e = dev_alloc(c, &nb, wf_bytes(uint32_t(P)));
+    }
+    NE_HIP(c, e);
     c->wf_buf = nb;
     c->wf_P = uint32_t(P);
   }
@@ -1746,11 +1755,11 @@ ne_status batch_launch(ne_batch* b, const ne_batch_config& cfg, int div, float* 
 }
 
 // Path-pool slots and sample count of job j at ceil(spp / div) samples, as
-// ne_render sizes them.
+// ne_render sizes them (at most 2^23: each lane has a pool).
 static uint64_t lane_job_pool(const ne_job& J, int div, uint64_t* samples) {
   const DevScene& ds = J.scene->dev;
   const uint64_t total = uint64_t(J.width) * uint64_t(J.height) * uint64_t((J.spp + div - 1) / div);
-  const uint64_t P = std::min<uint64_t>(default_pool(ds, total), total);
+  const uint64_t P = std::min<uint64_t>(std::min(default_pool(ds, total), kPool), total);
   if (samples) *samples = total;
   return (P + kChunk - 1) / kChunk * kChunk;
 }

@@ -119,3 +119,33 @@ def test_scene_info_does_not_wait_for_a_render(ctx):
     th.join()
     assert alive and waited < 0.25 * took[0], (waited, took)
     batch.close()
+
+
+def test_long_surface_renders_fit_in_a_smaller_pool(ctx):
+    """2^27 paths of a BVH of 2^16 nodes take a pool of 2^24 slots (3.6 GB), or half
+    of it where the card has no more room: the same film."""
+    from narvalengine_amd import Context
+    print_case("long surface render on a full card")
+    s = scenes.small_surface(subdiv=7)
+    films, used = [], []
+    for room in (0, 3000 << 20):  # (the first render leaves its pool of 2^20 slots beside it)
+        c = Context(0)
+        g = c.upload(s)
+        assert g.info()["bvh_nodes"] >= 1 << 16
+        f = c.film(1024, 1024)
+        c.render(g, scenes.BOX_CAMERA, f, spp=1, max_bounces=1, seed=3, fixed_film=True)
+        f.clear()
+        c.synchronize()
+        before = free_bytes()
+        fill = Block(before - room) if room else None
+        try:
+            c.render(g, scenes.BOX_CAMERA, f, spp=128, max_bounces=1, seed=3, fixed_film=True)
+        finally:
+            if fill:
+                fill.free()
+        used.append(before - free_bytes())
+        films.append(f.read())
+        c.close()
+    assert films[0].any()
+    np.testing.assert_array_equal(films[0], films[1])
+    assert used[0] > 1.5 * used[1], used
