@@ -128,7 +128,7 @@ def test_long_surface_renders_fit_in_a_smaller_pool(ctx):
     print_case("long surface render on a full card")
     s = scenes.small_surface(subdiv=7)
     films, used = [], []
-    for room in (0, 3000 << 20):  # (the first render leaves its pool of 2^20 slots beside it)
+    for room in (0, 2400 << 20):  # (beside the first render's pool of 2^20 slots)
         c = Context(0)
         g = c.upload(s)
         assert g.info()["bvh_nodes"] >= 1 << 16
