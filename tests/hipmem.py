@@ -3,6 +3,8 @@ import ctypes as C
 
 import narvalengine_amd
 
+MIB = 1 << 20
+
 
 def _hip():
     narvalengine_amd.lib()  # loads its runtime
@@ -15,12 +17,29 @@ def free_bytes() -> int:
     return free.value
 
 
-class Block:
-    """`size` bytes of device memory, never touched."""
+class FullCard:
+    """Takes the device's memory, untouched, until `leave` bytes at least, and at
+    most 256 MiB more, can be allocated beside it (what the runtime says is free
+    may be less than that)."""
 
-    def __init__(self, size: int):
-        self.p = C.c_void_p()
-        assert _hip().hipMalloc(C.byref(self.p), C.c_size_t(size)) == 0
+    def __init__(self, leave: int):
+        self.blocks = []
+        big = free_bytes() - leave - (4 << 30)
+        assert big > 0 and self._take(big)
+        while self._take(256 * MIB):
+            pass
+        for _ in range((leave + 256 * MIB - 1) // (256 * MIB)):
+            assert _hip().hipFree(self.blocks.pop()) == 0
+
+    def _take(self, size: int) -> bool:
+        p = C.c_void_p()
+        if _hip().hipMalloc(C.byref(p), C.c_size_t(size)) != 0:
+            _hip().hipGetLastError()  # or the next launch reports it
+            return False
+        self.blocks.append(p)
+        return True
 
     def free(self):
-        assert _hip().hipFree(self.p) == 0
+        for p in self.blocks:
+            assert _hip().hipFree(p) == 0
+        self.blocks = []

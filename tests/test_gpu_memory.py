@@ -5,7 +5,7 @@ import pytest
 
 import scenes
 from conftest import print_case
-from hipmem import Block, free_bytes
+from hipmem import FullCard, free_bytes
 
 pytestmark = pytest.mark.gpu
 GIB = 1 << 30
@@ -60,7 +60,7 @@ def test_quads_make_room_for_other_allocations(ctx):
     want, want_batches = frame(), batches()
     assert want.any()
     # all but 1 GiB taken by others, then a film of 2 GiB: 2.7 GiB are in quads
-    fill = Block(free_bytes() - GIB)
+    fill = FullCard(leave=GIB)
     try:
         big = ctx.film(32768, 2731)
     finally:
@@ -128,7 +128,7 @@ def test_long_surface_renders_fit_in_a_smaller_pool(ctx):
     print_case("long surface render on a full card")
     s = scenes.small_surface(subdiv=7)
     films, used = [], []
-    for room in (0, 2400 << 20):  # (beside the first render's pool of 2^20 slots)
+    for room in (0, 2304 << 20):  # (beside the first render's pool of 2^20 slots)
         c = Context(0)
         g = c.upload(s)
         assert g.info()["bvh_nodes"] >= 1 << 16
@@ -137,7 +137,7 @@ def test_long_surface_renders_fit_in_a_smaller_pool(ctx):
         f.clear()
         c.synchronize()
         before = free_bytes()
-        fill = Block(before - room) if room else None
+        fill = FullCard(leave=room) if room else None
         try:
             c.render(g, scenes.BOX_CAMERA, f, spp=128, max_bounces=1, seed=3, fixed_film=True)
         finally:
