@@ -397,9 +397,11 @@ __global__ __launch_bounds__(1024) void k_guide_reduce(GuideNet g, GuideTrain t,
 // it: tables of more ranges than the chip has CUs take all samples in every
 // block; smaller ones split the samples into `chunks`, each with a copy of the
 // ranges (t.table_part, 64 KiB per range and chunk: at most 16 MiB, as chunks x
-// ranges fill the chip once: it fits in the weights' partials), and sum the copies after (k_guide_table_sum).  The whole training pass with its copies,
+// ranges fill the chip once: it fits in the weights' partials), and sum the
+// copies after (k_guide_table_sum).  The whole training pass with its copies,
 // 65,536 samples, this kernel against atomics at every level, us:
-// log2_table 15: 488 / 1306, 17: 648 / 1292, 19: 658 / 1301, 21: 971 / 1360;
+// log2_table 15: 488 / 1306, 17: 648 / 1292, 19: 658 / 1301, 21: 971 / 1360,
+// 22: 1210 / 1930;
 // 8192 samples: 15: 316 / 454, 21: 279 / 333.  Atomics for the large levels
 // only lost at every size too (19: 1038).
 constexpr uint32_t kTableRange = 8192;   // 128 KiB of LDS: one block per CU
