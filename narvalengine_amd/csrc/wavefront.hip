@@ -1270,20 +1270,6 @@ hipError_t wf_flush(const WfArgs& a, hipStream_t st) {
   return hipGetLastError();
 }
 
-// The narrowest form that a render in NC chunks reads the density by.  Quads take
-// four times the memory: where the bricks fit in an XCD's L2 (4 MiB) and the quads
-// do not, launches that the chip holds at once wait for the quads longer than
-// their fewer loads save.  Bricks / quads, us: rectangle under a volume of 72^3,
-// 225 chunks 1236 / 1295, 469 chunks 1316 / 1376, 1200 chunks 1454 / 1496, 2400
-// chunks 1699 / 1707; volumes alone, 225 / 1200 / 2400 chunks, 56^3 735 / 720, 852 /
-// 839, 981 / 956, 64^3 741 / 752, 852 / 852, 983 / 966, 88^3 746 / 798, 884 / 907,
-// 1014 / 1010, 104^3 802 / 817, 928 / 918, 1066 / 1030; 48^3 and smaller: quads.
-static int staged_form(const DevScene& s, uint32_t NC, uint32_t resident) {
-  const uint64_t quads = uint64_t(s.quad_step_z) * (quad_pad_z(s.res[2]) / 2u) * sizeof(float4);
-  const uint64_t bricks = uint64_t(s.grid_step_z) * (grid_pad_z(s.res[2]) / 2u) * sizeof(float);
-  return NC <= resident && quads > (2816u << 10) && bricks <= (4096u << 10) ? kGridBrick : kGridQuad;
-}
-
 hipError_t launch_wavefront(const DevScene& s, const DevCamera& cam, WfState& w, WfArgs a, bool count,
                             hipStream_t st, uint32_t* h_status, StageTimer* tm, WfGuideHook* gh) {
   hipError_t e = hipSuccess;
@@ -1302,7 +1288,7 @@ hipError_t launch_wavefront(const DevScene& s, const DevCamera& cam, WfState& w,
   const bool hs = s.n_nodes > 0, hv = s.has_volume != 0;
   const bool sort = (a.sort & 1) != 0;
   const bool spatial = (a.sort & 2) != 0;  // tracking stages in Morton order of the ray origins
-  const int form = std::min(std::min(s.grid_form, a.grid_max), staged_form(s, NC, a.refill_blocks));
+  const int form = std::min(s.grid_form, a.grid_max);  // how density lookups read the grid
   // the volume shadow stage reads a continuing path's origin and RNG key
   // from its next record; the surface-only shadow stage reads whole records
   a.shadow_full = hv ? 0 : 1;

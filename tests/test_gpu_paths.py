@@ -128,27 +128,3 @@ def test_the_grids_forms_give_the_same_film(ctx, which, run):
         for o in out[1:]:
             np.testing.assert_array_equal(out[0][0], o[0], err_msg=f"{w}x{h}")
             assert out[0][1] == o[1]
-
-
-@pytest.mark.parametrize("res", [54, 56, 57, 100, 101])
-@pytest.mark.parametrize("run", ["staged", "surfaces"])
-def test_films_do_not_depend_on_the_grid_form_that_a_launch_takes(ctx, res, run):
-    """The staged pipeline reads the bricks of grids that fit in an XCD's L2 where
-    the quads do not (56^3 to 100^3 here), in pools that the chip holds at once:
-    a frame in such a pool (45 x 37 x 8: 53 chunks), one in a larger one (800 x
-    600 x 2: 3750), and both by 64-bit offsets."""
-    print_case(f"grid form by launch {run} {res}")
-    from narvalengine_amd.scene import Camera
-    s = scenes.env_map_scene() if run == "surfaces" else scenes.small_volume(res=8, maj_res=4)
-    s.set_volume(np.random.default_rng(res).random((res, res, res), np.float32), 6.0, (0.95,) * 3, (0.05,) * 3, 0.7,
-                 maj_res=4)
-    g = ctx.upload(s)
-    cam = Camera(position=(0.0, 0.25, -1.8), look_at=(0, 0, 0), vfov=45.0, aspect=1.3)
-    for w, h, spp in [(45, 37, 8), (800, 600, 2)]:
-        films = []
-        for wide in (False, True):
-            f = ctx.film(w, h)
-            ctx.render(g, cam, f, spp=spp, max_bounces=12, seed=5, mode=2, wide=wide)
-            films.append(f.read())
-        assert films[0].any()
-        np.testing.assert_array_equal(films[0], films[1], err_msg=f"{w}x{h}")
